@@ -196,17 +196,17 @@ int plife_get_accelerations(plife_physics *h, int32_t n, float *acc);
 
 /* Launch shape (no counterpart in the reference, which has no device).  Zero
  * fields mean automatic.  block_homes in {0, 64, 128, 256}: home particles
- * (threads) per force workgroup; list_cap in [0, 512]: per-thread LDS
- * candidate-list entries of the force kernel; stage_slack in [0, 16]: LDS
+ * (threads) per force workgroup; list_cap in [0, 512]: LDS mask
+ * words per home (32 candidates each) of a force workgroup that streams its
+ * neighbourhood in several windows; stage_slack in [0, 16]: LDS
  * staging capacity as a multiple of the expected staged particles;
  * direct_launch 1: launch every kernel directly instead of replaying a HIP
  * graph of two steps; sparse_worlds: which worlds the sparse-world force
  * kernel (one thread per particle, stencil read from global memory) steps
  * instead of the staged one -- 0 those whose cells hold too few particles
  * for staging to pay, 1 none, 2 all; windowed_only 1: the staged force
- * kernel always screens homes in windows with per-thread candidate lists,
- * never on its balanced path (one window, homes dealt to lanes by their
- * kept-candidate counts); small_step: whether worlds that fit one
+ * kernel always streams a neighbourhood in windows, also where it would fit
+ * one; small_step: whether worlds that fit one
  * workgroup's LDS (up to about 10,000 particles in 2D, 7,000 in 3D) step in
  * one launch that bins, sorts and steps them in LDS -- 0 when every world of
  * the handle fits and no other launch-shape field is set, 1 never, 2

@@ -70,13 +70,13 @@ constexpr int kMaxTypesLds = 32;      // matrix staged in LDS up to 32x32 (8 KB 
 constexpr long long kMaxCells = 1LL << 28;
 constexpr int kMaxWorlds = 65535;     // the world index of a slot is a u16
 constexpr int kMaxLds = 65536;
-constexpr int kClusteredLds = 17152;  // force-kernel LDS in clustered worlds: 9 workgroups per CU
 constexpr int kTuneSteps = 24;         // an update long enough to time two configurations
 constexpr int kTuneMax = 22;           // steps such a timing takes at most (4 x 4 + 3 switches + 3)
 constexpr size_t kWordLds = 24576;    // most LDS for the balanced path's mask words
 
 struct ForcePlan {
-    int wpool = 0;                    // mask words per workgroup of the balanced path (0: windowed only)
+    int wpool = 0;                    // mask words per workgroup with one window (0: always several)
+    int wpool2 = 0;                   // mask words per workgroup with several windows
     int bs, lcap, max_cells, cap;
     size_t lds;
 };
@@ -471,6 +471,12 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     d.moff = moff;
     d.wrap = s.wrap ? 1 : 0;
     d.r2hi = (float)(R * R * (1.0 + 0x1p-20));
+    // |D| <= rmax (1 + 2^-20) in steps of 2^-16 box, x and z less than one step
+    // off, y less than two: |d| < rmax / step + sqrt(dim + 3).  (Grids of fewer
+    // than 3 cells per axis are not screened on it; the clamp only keeps the
+    // conversion in range.)
+    const double rq = s.rmax * 65536.0 * (1.0 + 0x1p-20) + std::sqrt((double)(s.dim + 3));
+    d.sbias = -(int)std::min(rq * rq + 2.0, 2147483646.0);
     d.cs = s.rmax;
     d.r2u = (s.rmax * s.rmax) * (kFix * kFix);         // Physics.java:432, exact 2^64 scaling
     d.S = 1.0 / R;
@@ -935,30 +941,27 @@ int record(plife_physics *h, PhaseEvents *ev, int k)
 // occupancy (sum over cells of count^2, divided by N: the mean size of the
 // cell a particle sits in) measured by an earlier step:
 //   * uniform worlds: 256 homes per workgroup and a staging buffer that holds
-//     the whole neighbourhood (one window); 24-entry candidate lists where
-//     cells are dense enough for the LDS to limit occupancy, 32 where sparse;
+//     the whole neighbourhood (one window);
 //   * clustered 3D worlds (occupancy far above the mean N / cells): 128 homes
 //     per workgroup and a small staging buffer, so that many workgroups share
 //     a CU while the dense neighbourhoods stream through it in windows.
-// The plan never changes results: every home visits its candidates in the
-// same order whatever the windows and workgroup size.
-ForcePlan plan_force_for(int dim, double avg, double occ, bool clustered, const plife_tuning &t,
-                         bool dbg, int ntypes_max)
+// mixed: worlds of several densities share the launch.  The plan never changes
+// results: every home visits its candidates in the same order whatever the
+// windows and workgroup size.
+ForcePlan plan_force_for(int dim, double avg, bool clustered, bool mixed, const plife_tuning &t, bool dbg,
+                         int ntypes_max)
 {
     const int NR = dim == 3 ? 9 : 3;
     ForcePlan p;
     p.bs = t.block_homes ? t.block_homes : (clustered ? 128 : 256);
-    p.lcap = t.list_cap > 0 ? std::max(8, std::min(t.list_cap, 512))   // >= the screen group (8)
-                            : (clustered || occ < 12.0 ? 32 : 24);
-    p.lcap = std::min(p.lcap, 16384 / p.bs);             // lists stay within 32 KB of LDS
     // a workgroup of bs homes spans ~bs/avg + 1 cells of a row; it stages NR
     // rows of (span + 2) cells.  Clustered worlds keep a short cell table: the
     // few sparse workgroups that span more cells take the global path.
     const double span = p.bs / std::max(avg, 1e-9) + 1.0;
-    // balanced path (uniform worlds): a home's stencil row is a run of three
-    // cells, ~3 avg candidates, ceil(run / 32) mask words; the workgroup's
-    // pool holds 10% more than the expected total (workgroups needing more
-    // take the windowed path)
+    // one window (uniform worlds): a home's stencil row is a run of three cells,
+    // ~3 avg candidates, ceil(run / 32) mask words; the workgroup's pool holds
+    // 10% more than the expected total (workgroups needing more take several
+    // windows)
     if (!clustered && !t.windowed_only) {
         const double run = 3.0 * avg;
         const long long pool = (long long)std::ceil(p.bs * NR * (run / 32.0 + 0.5) * 1.1) + 64;
@@ -966,20 +969,30 @@ ForcePlan plan_force_for(int dim, double avg, double occ, bool clustered, const 
     }
     p.max_cells = (int)std::min<double>(std::max(64.0, std::ceil(NR * (span + 2.0) * 1.5 + 16)),
                                         clustered ? 384.0 : 2048.0);
-    long long want;
-    size_t budget = kMaxLds;
-    if (t.stage_slack > 0.0 || !clustered) {
-        const double slack = t.stage_slack > 0.0 ? t.stage_slack : 1.25;
-        want = (long long)std::ceil(NR * (span + 2.0) * avg * slack) + 64;
-    } else {
-        want = 65535;
-        budget = kClusteredLds;
-    }
+    // several windows: mask words per home (32 candidates each).  Where one
+    // window is the rule (a single uniform world), no more than fit the space of
+    // its pool: LDS per workgroup sets how many share a CU (1M 2D world: 0.218 ms
+    // a step within the pool, 0.231 at 7 words).  Worlds of several densities in
+    // one launch stream windows in the denser half of them: 9 words (512-world
+    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9).  Clustered worlds: 5 (4M
+    // 3D world: 35.1 ms at 5, 35.7 at 7, 36.5 at 9).
+    const int fixed = force_home_bytes(dim, dbg);
+    const int fit = (int)(((long long)p.wpool * 6 / p.bs - fixed) / 6);
+    p.lcap = t.list_cap > 0 ? std::max(t.list_cap, 2)
+             : clustered    ? 5
+                            : std::max(mixed || p.wpool == 0 ? 9 : 4, std::min(fit, 16));
+    p.lcap = std::min(p.lcap, 32768 / (6 * p.bs));                       // words stay within 32 KB of LDS
+    p.wpool2 = p.lcap * p.bs;
+    const size_t budget = kMaxLds;
+    const double slack = t.stage_slack > 0.0 ? t.stage_slack : 1.25;
+    long long want = (long long)std::ceil(NR * (span + 2.0) * avg * slack) + 64;
+    // where every workgroup streams windows, stage no more than its words cover
+    if (p.wpool == 0) want = std::min<long long>(clustered ? 65535 : want, 32ll * (p.lcap - 1));
     want = std::min<long long>((want + 63) / 64 * 64, 65535);
     const bool m_in_lds = ntypes_max <= kMaxTypesLds;
     auto total = [&](long long c) {
-        return force_lds_layout(dim, dbg, ntypes_max, m_in_lds, (int)c, p.lcap, p.bs,
-                                p.max_cells, p.wpool).total;
+        return force_lds_layout(dim, dbg, ntypes_max, m_in_lds, (int)c, p.bs, p.max_cells,
+                                p.wpool, p.wpool2).total;
     };
     // keep room for a useful staging window: shrink the cell table first
     const long long min_cap = std::min<long long>(want, 256);
@@ -1015,8 +1028,7 @@ ForcePlan plan_force(const plife_physics *h)
         sc = h->ncells;
     }
     const double avg = (double)sn / (double)std::max(sc, 1LL);
-    const double occ = h->occupancy > 0.0 ? h->occupancy : avg + 1.0;   // Poisson: avg + 1
-    return plan_force_for(dim, avg, occ, h->clustered, plan_tuning(h), h->debug != 0, h->ntypes_max);
+    return plan_force_for(dim, avg, h->clustered, h->worlds.size() > 1, plan_tuning(h), h->debug != 0, h->ntypes_max);
 }
 
 // The class of a layout for the measured homes per workgroup: dimension,
@@ -1513,9 +1525,9 @@ int do_step(plife_physics *h, PhaseEvents *ev)
     a.ntypes_max = h->ntypes_max;
     a.m_in_lds = h->ntypes_max <= kMaxTypesLds ? 1 : 0;
     a.cap = fp.cap;
-    a.lcap = fp.lcap;
     a.max_cells = fp.max_cells;
     a.wpool = fp.wpool;
+    a.wpool2 = fp.wpool2;
     a.pair_total = h->d_pairs;
     a.pair_world = h->d_pairs + 2;
     a.block_work = h->work_dev;
@@ -2555,7 +2567,7 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
     const WorldDev wd = world_dev(wh, 0u, 0);
     const int nc = (int)gr.ncells;
     const double avg = (double)n / (double)nc;
-    const ForcePlan fp = plan_force_for(s->dim, avg, avg + 1.0, false, plife_tuning{}, false, ntypes);
+    const ForcePlan fp = plan_force_for(s->dim, avg, false, false, plife_tuning{}, false, ntypes);
     const int nblocks = ceil_div(n, fp.bs);
     const RadixPlan plan = radix_plan(nc, n);
 
@@ -2651,9 +2663,9 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
         a.ntypes_max = ntypes;
         a.m_in_lds = ntypes <= kMaxTypesLds ? 1 : 0;
         a.cap = fp.cap;
-        a.lcap = fp.lcap;
         a.max_cells = fp.max_cells;
         a.wpool = fp.wpool;
+        a.wpool2 = fp.wpool2;
         a.pair_total = t.d_pairs;
         a.pair_world = t.d_pairs + 2;
         a.block_work = work;

@@ -12,15 +12,15 @@
 // stencil visits.
 //
 // Each home particle runs two phases over its candidates:
-//   A  FP32 screen: exact int32 minimum-image deltas (positions are 32-bit
-//      fixed point), |D|^2 in FP32, keep 0 < |D|^2 <= rmax^2 (1 + 2^-20).  Kept
-//      candidate indices are appended to a per-thread list in LDS.
+//   A  integer screen on the high 16 bits of the coordinates (screen_hi).  Kept
+//      candidates become bits of mask words in LDS, or indices appended to a
+//      per-thread list.
 //   B  For listed candidates only: the reference's predicate in FP64
 //      (d2 = dx*dx + dy*dy, d2 != 0 && d2 <= rmax*rmax; Physics.java:430-432) and
 //      the force law in FP64 (FP64 FMA issues at the non-packed FP32 rate on
 //      CDNA4), accumulated in FP64.
-// The screen is a strict superset of the FP64 predicate (its FP32 rounding is
-// below 2^-21 relative), so neighbour sets are exactly the reference's.
+// The screen is a strict superset of the FP64 predicate, so neighbour sets are
+// exactly the reference's.
 #pragma once
 
 #include <type_traits>
@@ -46,8 +46,9 @@ struct ForceArgs {
     const uint2 *blocks;             // per workgroup: (world, first home slot)
     int block_base;                  // this launch's first entry of blocks
     int ntypes_max, m_in_lds;
-    int cap, lcap, max_cells;
-    int wpool;                       // mask words per workgroup of the balanced path (0: windowed only)
+    int cap, max_cells;
+    int wpool;                       // mask words of a workgroup with one window (0: always several)
+    int wpool2;                      // and of one that streams several
     unsigned long long *pair_total;  // interacting pairs of the step, all worlds
     unsigned long long *pair_world;  // per world
     uint32_t *block_work;            // pinned host memory: per table entry its pairs (saturated); [nb_total] = tag
@@ -153,11 +154,18 @@ __device__ __forceinline__ void record_block_work(const ForceArgs &a, int blk,
     if (e == 0) a.block_work[a.nb_total] = a.work_tag;
 }
 
+// Largest of the wave's values (each >= 0), the same in every lane: the DPP
+// steps of wave_incl_scan with max in place of add, read from lane 63 into a
+// scalar register, so that loops bounded by it branch on scalars.
 __device__ __forceinline__ int wave_max(int v)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
-    return v;
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));    // row_shr:1
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));    // row_bcast:15
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));    // row_bcast:31
+    return __builtin_amdgcn_readlane(v, kWave - 1);
 }
 
 // Phase A screen on exact fixed-point deltas.  In a clamped world the int32
@@ -179,38 +187,44 @@ __device__ __forceinline__ bool screen(uint32_t hx, uint32_t hy, uint32_t hz, ui
     return d2 <= r2hi;
 }
 
-// Periodic distance in cells between columns (rows, layers) a and b of n.
-__device__ __forceinline__ int periodic_cells(int a, int b, int n)
+// The staged kernel keeps each candidate's x and y as two words, the high
+// halves (x >> 16 | y & 0xFFFF0000) and the low halves (x & 0xFFFF | y << 16):
+// phase A reads the first alone, phase B rebuilds the exact coordinates from
+// both (one v_perm_b32 each).
+__device__ __forceinline__ uint32_t high_halves(uint32_t x, uint32_t y)
 {
-    int d = a - b;
-    d = d < 0 ? -d : d;
-    d %= n;
-    return min(d, n - d);
+    return __builtin_amdgcn_perm(y, x, 0x07060302u);
 }
-
-// 16-bit relative coordinate of fixed-point p against the origin o (floor of
-// the periodic int32 difference over 2^sh), as the low 16 bits of a u32.
-__device__ __forceinline__ uint32_t rel16(uint32_t p, uint32_t o, int sh)
+__device__ __forceinline__ uint32_t low_halves(uint32_t x, uint32_t y)
 {
-    return (uint32_t)((int)(p - o) >> sh) & 0xFFFFu;
+    return __builtin_amdgcn_perm(y, x, 0x05040100u);
 }
+__device__ __forceinline__ uint32_t join_x(uint2 hl) { return __builtin_amdgcn_perm(hl.x, hl.y, 0x05040100u); }
+__device__ __forceinline__ uint32_t join_y(uint2 hl) { return __builtin_amdgcn_perm(hl.x, hl.y, 0x07060302u); }
 
 typedef short short2v __attribute__((ext_vector_type(2)));
 
-// Phase A screen on packed 16-bit relative coordinates (x | y << 16, z apart):
-// packed subtract and a saturating dot product against the quantised bound.
-// Each coordinate is at most one unit off its exact quotient, so the bound
-// (Rq + 2)^2 keeps every pair with |D| <= rmax (1 + 2^-20).
+// Phase A screen on the high 16 bits of each coordinate (65,536 steps per
+// box, so differences modulo 2^16 are minimum-image differences): negative
+// when the candidate is kept.  One 32-bit subtract takes both differences: a
+// borrow out of the low half takes one more step off the high one, so x is
+// less than 1 step off the exact difference, y less than 2, z less than 1, and
+// `bias` = -(bq + 1), bq = (rmax / step + sqrt(DIM + 3))^2 (WorldDev::sbias),
+// keeps every pair with |D| <= rmax (1 + 2^-20).  Issue cycles per wave and
+// candidate, measured: subtract 2, dot product with the bias as accumulator
+// 4, the caller's v_alignbit_b32 4 -- against 26 for exact differences in
+// FP32 (two subtracts, two conversions, mul, fma, compare, select, or).  The
+// clamped dot product is the three-operand form (no copy of the bias).
 template <int DIM>
-__device__ __forceinline__ bool screen16(uint32_t q, uint32_t h, uint32_t qz, uint32_t hz, int bq)
+__device__ __forceinline__ int screen_hi(uint32_t q, uint32_t h, uint32_t qz, uint32_t hz, int bias)
 {
-    const short2v d = __builtin_bit_cast(short2v, q) - __builtin_bit_cast(short2v, h);
-    int zz = 0;
+    const short2v d = __builtin_bit_cast(short2v, q - h);
+    int c = bias;
     if constexpr (DIM == 3) {
-        const int dz = (int)(short)(uint16_t)(qz - hz);
-        zz = dz * dz;
+        const uint32_t dz = qz - hz;      // its high half: z's difference in steps
+        asm("v_mad_i32_i16 %0, %1, %1, %2 op_sel:[1,1,0,0]" : "=v"(c) : "v"(dz), "s"(bias));
     }
-    return __builtin_amdgcn_sdot2(d, d, zz, true) <= bq;
+    return __builtin_amdgcn_sdot2(d, d, c, true);
 }
 
 __device__ __forceinline__ int wrap_cell(int c, int n)
@@ -345,58 +359,237 @@ __device__ void home_global(const ForceArgs &a, const WorldDev &w, const double 
             }
 }
 
-// A workgroup of BS threads (BS/64 waves) owns BS consecutive home particles
-// of the cell-sorted order, so every wave is full.  The homes span a few
-// consecutive cells of one grid row, or (at row ends) of a few rows: each
-// distinct row is a "part" whose 3^(DIM-1) stencil rows x (span + 2) cells are
-// staged in LDS for the whole workgroup, in windows of at most `cap` particles
-// when the neighbourhood is denser than the staging buffer.  Workgroups with
-// more parts or staged cells than the cell table holds take the global path.
+// Staged columns of the parts: part q holds rows x p_w[q] cells from
+// p_base[q] on.  A workgroup's homes span a few consecutive cells of one grid
+// row, or (at row ends) of a few rows; each distinct row is a part.
 constexpr int kMaxParts = 4;
-constexpr int kScreenPad = 8;    // >= the screen's group size U
-constexpr int kDealKeys = 5;     // 4 position groups + the inactive threads of a short block
+constexpr int kScreenPad = 32;   // candidates a screen step reads from one base
 
-// Position group of a home inside its cell: y quartile (2D) or y/z halves (3D).
-template <int DIM>
-__device__ __forceinline__ int deal_key(uint32_t y, uint32_t z, int hrow, int nx, double cs)
+// Starts (gs) of the NC staged cells and their exclusive prefix (off, NC + 1
+// entries) for a workgroup of T threads; returns the staged particle count,
+// the same in every thread.  Ends with a barrier.
+template <int DIM, int T>
+__device__ __forceinline__ uint32_t stage_cells(const ForceArgs &a, const int (&p_base)[kMaxParts + 1],
+                                                const int (&p_w)[kMaxParts], const int (&p_row)[kMaxParts],
+                                                const int (&p_ca)[kMaxParts], int nx, uint32_t cb,
+                                                uint32_t *off, uint32_t *gs, uint32_t *s_cnt)
 {
-    const float inv = (float)(kInvFix / cs);
-    const int cy = hrow % nx;
-    const float fy = (float)y * inv - (float)cy;           // ~[0, 1) within the cell
-    if constexpr (DIM == 2) return min(3, max(0, (int)(fy * 4.0f)));
-    const float fz = (float)z * inv - (float)(hrow / nx);
-    return min(1, max(0, (int)(fz * 2.0f))) * 2 + min(1, max(0, (int)(fy * 2.0f)));
+    constexpr int NW = T / kWave;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    const int NC = p_base[kMaxParts];
+    uint32_t carry = 0;
+    for (int f0 = 0; f0 < NC; f0 += T) {
+        const int f = f0 + tid;
+        uint32_t c = 0;
+        if (f < NC) {
+            int pb = p_base[0], pw = p_w[0], pr = p_row[0], pc = p_ca[0];
+#pragma unroll
+            for (int q = 1; q < kMaxParts; ++q)
+                if (f >= p_base[q] && p_w[q] > 0) { pb = p_base[q]; pw = p_w[q]; pr = p_row[q]; pc = p_ca[q]; }
+            const int r = (f - pb) / pw, j = (f - pb) - r * pw;
+            const int oy = (r % 3) - 1, oz = DIM == 3 ? (r / 3) - 1 : 0;
+            const int cy = pr % nx, cz = DIM == 3 ? pr / nx : 0;
+            const int x = wrap_cell(pc - 1 + j, nx);
+            const int y = wrap_cell(cy + oy, nx);
+            const int z = DIM == 3 ? wrap_cell(cz + oz, nx) : 0;
+            const uint32_t ci = cb + (uint32_t)(x + y * nx + z * nx * nx);
+            const uint32_t s0 = a.cell_start[ci];
+            c = a.cell_end[ci] - s0;
+            gs[f] = s0;
+        }
+        const uint32_t inc = wave_incl_scan(c);
+        if (lane == kWave - 1) s_cnt[wv] = inc;
+        __syncthreads();
+        uint32_t wbase0 = carry, tot = 0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            wbase0 += v < wv ? s_cnt[v] : 0u;
+            tot += s_cnt[v];
+        }
+        if (f < NC) off[f] = wbase0 + inc - c;
+        carry += tot;
+        __syncthreads();
+    }
+    if (tid == 0) off[NC] = carry;
+    __syncthreads();
+    return carry;
 }
 
-struct ForceLds {
-    size_t m, sxy, sq, lists, wbase, sz, sqz, sid, off, gs, st, total;
+// Staged candidates in LDS: high and low halves of x and y, z, type and
+// (debug) id.
+struct Staged {
+    uint2 *xy;
+    uint32_t *z, *id;
+    uint8_t *type;
 };
 
-// The candidate lists (windowed path: lcap u16 entries per thread) and the
-// mask words (balanced path: a pool of wpool u32 masks + wpool u16 first
-// indices, each home its own run of them) share one region; a workgroup takes
-// one path.
+// Stages entries [w0, w0 + wn) of the neighbourhood (NC cells) with T threads.
+template <int DIM, bool DEBUG, int T>
+__device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s, const uint32_t *off,
+                                             const uint32_t *gs, int NC, int w0, int wn)
+{
+    for (int t = threadIdx.x; t < wn; t += T) {
+        const int sg = w0 + t;
+        int lo = 0, hi = NC;           // off[lo] <= sg < off[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (off[mid] <= (uint32_t)sg) lo = mid;
+            else hi = mid;
+        }
+        const uint32_t q = a.perm[gs[lo] + ((uint32_t)sg - off[lo])];
+        const uint32_t qx = a.sx[q], qy = a.sy[q];
+        s.xy[t] = make_uint2(high_halves(qx, qy), low_halves(qx, qy));
+        if constexpr (DIM == 3) s.z[t] = a.sz[q];
+        if constexpr (DEBUG) s.id[t] = (uint32_t)a.id[q];
+        s.type[t] = (uint8_t)a.type[q];
+    }
+}
+
+// U candidates from entry kb against one home: word << U, bit u set when
+// candidate kb + u passes the phase-A screen.  Built from the last candidate
+// down, each result's sign bit shifted in by one v_alignbit_b32.
+template <int DIM, int U>
+__device__ __forceinline__ uint32_t screen_group(const Staged &s, int kb, uint32_t hq, uint32_t hz, int bias,
+                                                 uint32_t word)
+{
+    const uint2 *qp = s.xy + kb;
+    const uint32_t *qzp = s.z + kb;
+    int t[U];
+#pragma unroll
+    for (int u = U - 1; u >= 0; --u) t[u] = screen_hi<DIM>(qp[u].x, hq, DIM == 3 ? qzp[u] : 0u, hz, bias);
+#pragma unroll
+    for (int u = U - 1; u >= 0; --u) word = __builtin_amdgcn_alignbit(word, (uint32_t)t[u], 31);
+    return word;
+}
+
+// The low n bits set (n clamped to [0, 32]).
+__device__ __forceinline__ uint32_t low_bits(int n)
+{
+    return n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
+}
+
+// Phase B of one home at (px, py, pz) with matrix row mrow: its `left` kept
+// candidates, word by word in candidate order, two per iteration (half the
+// loop's bookkeeping; their force laws overlap).  load(m, kb) fetches the
+// next non-zero mask word and its first candidate.
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS, typename Load>
+__device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w, const Staged &s,
+                                          const double *M, Acc &ab, int left, Load &&load, uint32_t px,
+                                          uint32_t py, uint32_t pz, int mrow)
+{
+    // one candidate k: the reference's FP64 predicate and force law
+    auto visit = [&](int k) {
+        const uint2 hl = s.xy[k];
+        const uint32_t qx = join_x(hl), qy = join_y(hl), qz = DIM == 3 ? s.z[k] : 0u;
+        const int dxi = (int)(qx - px), dyi = (int)(qy - py);
+        const int dzi = DIM == 3 ? (int)(qz - pz) : 0;
+        bool ok = true;
+        if constexpr (!WRAP) {
+            // plain difference of the clamped world: |D| >= 1/2 unless the
+            // int32 difference has the sign of the unsigned order
+            ok = ((dxi >= 0) == (qx >= px)) & ((dyi >= 0) == (qy >= py));
+            if (DIM == 3) ok &= ((dzi >= 0) == (qz >= pz));
+        }
+        const int idx = mrow + (int)s.type[k];
+        const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
+        pair64_sel<DIM, DEBUG>(ab, ok, dxi, dyi, dzi, m, DEBUG ? s.id[k] : 0u, w);
+    };
+    uint32_t m = 0;
+    int kb = 0;
+    auto next = [&]() {
+        if (m == 0) load(m, kb);
+        const int k = kb + __builtin_ctz(m);
+        m &= m - 1u;
+        return k;
+    };
+#pragma unroll 1
+    for (; left >= 2; left -= 2) {
+        const int k1 = next();
+        const int k2 = next();
+        visit(k1);
+        visit(k2);
+    }
+    if (left > 0) visit(next());
+}
+
+// Counting sort of the HPT * T homes of a workgroup by their kept-candidate
+// counts (thread tid holds the counts of slots tid, tid + T, ..., in bins of
+// 2^shift; the order inside a bin does not matter): s_deal[rank] = slot.
+// Synchronises before it reads anything the homes' threads wrote, and after.
+template <int T, int HPT>
+__device__ __forceinline__ void deal_homes(const int (&count)[HPT], int shift, uint32_t *s_bin,
+                                           uint16_t *s_deal, uint32_t *s_cnt)
+{
+    constexpr int PER = 256 / T;              // bins per thread
+    const int tid = threadIdx.x;
+    for (int t = tid; t < 256; t += T) s_bin[t] = 0u;
+    __syncthreads();
+    int bin[HPT];
+    uint32_t local[HPT];
+#pragma unroll
+    for (int q = 0; q < HPT; ++q) {
+        bin[q] = min(count[q] >> shift, 255);
+        local[q] = atomicAdd(&s_bin[bin[q]], 1u);
+    }
+    __syncthreads();
+    {
+        uint32_t v[PER], sum = 0, total = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            v[q] = s_bin[tid * PER + q];
+            sum += v[q];
+        }
+        uint32_t ex = block_excl_scan<T>(sum, s_cnt, total);
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            s_bin[tid * PER + q] = ex;
+            ex += v[q];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < HPT; ++q) s_deal[s_bin[bin[q]] + local[q]] = (uint16_t)(tid + q * T);
+    __syncthreads();
+}
+
+// The LDS of a staged workgroup: `cap` staged entries at most; the windowed
+// path streams a denser neighbourhood through it.
+struct ForceLds {
+    size_t m, sxy, words, wbase, ax, ay, az, dhash, hxy, hz, dcnt, words2, wbase2, ht, sz, sid, off, gs, st, total;
+};
+
+// Bytes per home that several windows keep in LDS besides the mask words: the
+// sums, the home's position and type, and (debug) its count and hash.
+constexpr int force_home_bytes(int dim, bool debug) { return dim * 8 + (dim == 3 ? 12 : 8) + 1 + (debug ? 12 : 0); }
+
+// A workgroup whose neighbourhood is one window has a pool of wpool mask words
+// (u32 bits + u16 first staged index); one that streams several windows keeps
+// the per-home data in the same region and a pool of wpool2 words.
 __host__ __device__ inline ForceLds force_lds_layout(int dim, bool debug, int ntypes, bool m_in_lds,
-                                                     int cap, int lcap, int bs, int max_cells,
-                                                     int wpool)
+                                                     int cap, int bs, int max_cells, int wpool, int wpool2)
 {
     ForceLds L;
     size_t o = 0;
     L.m = o;     o += m_in_lds ? (size_t)ntypes * ntypes * 8 : 0;
     // the screened arrays carry kScreenPad spare entries: a screen step reads
-    // a group of U candidates from one base, up to U - 1 past a lane's range
+    // up to 32 candidates from one base, up to 31 past a lane's range
     L.sxy = o;   o += (size_t)(cap + kScreenPad) * 8;
-    L.sq = o;    o += dim == 3 ? (size_t)(cap + kScreenPad) * 4 : 0;     // 16-bit screen (3D only)
-    L.lists = o;
+    L.words = o;
     L.wbase = o + (size_t)wpool * 4;
-    {
-        const size_t lsz = (size_t)lcap * bs * 2, wsz = (size_t)wpool * 6;
-        o += lsz > wsz ? lsz : wsz;
-    }
+    const size_t wend = o + (size_t)wpool * 6;
+    L.ax = o;    o += (size_t)bs * 8;
+    L.ay = o;    o += (size_t)bs * 8;
+    L.az = o;    o += dim == 3 ? (size_t)bs * 8 : 0;
+    L.dhash = o; o += debug ? (size_t)bs * 8 : 0;
+    L.hxy = o;   o += (size_t)bs * 8;
+    L.hz = o;    o += dim == 3 ? (size_t)bs * 4 : 0;
+    L.dcnt = o;  o += debug ? (size_t)bs * 4 : 0;
+    L.words2 = o; o += (size_t)wpool2 * 4;
+    L.wbase2 = o; o += (size_t)wpool2 * 2;
+    L.ht = o;    o += (size_t)bs;
+    o = o > wend ? o : wend;
     o = (o + 3) & ~(size_t)3;
     L.sz = o;    o += dim == 3 ? (size_t)(cap + kScreenPad) * 4 : 0;
-    L.sqz = o;   o += dim == 3 ? (size_t)(cap + kScreenPad) * 2 : 0;
-    o = (o + 3) & ~(size_t)3;
     L.sid = o;   o += debug ? (size_t)cap * 4 : 0;
     L.off = o;   o += (size_t)(max_cells + 1) * 4;
     L.gs = o;    o += (size_t)max_cells * 4;
@@ -408,33 +601,32 @@ __host__ __device__ inline ForceLds force_lds_layout(int dim, bool debug, int nt
 // MLDS: the type matrix is staged in LDS (ntypes <= 32); otherwise it is read
 // from global memory.  A compile-time switch, so the hot loop's matrix load is
 // a plain ds_read and never a generic (flat) load.
+//
+// A workgroup of BS threads (BS/64 waves) owns BS consecutive home particles
+// of the cell-sorted order, so every wave is full.  The parts' 3^(DIM-1)
+// stencil rows x (span + 2) cells are staged in LDS for the whole workgroup.
+// Workgroups with more parts or staged cells than the cell table holds take
+// the global path.
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS, int BS>
 __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
 {
     constexpr int NR = DIM == 3 ? 9 : 3;      // stencil rows per part
     constexpr int RMID = DIM == 3 ? 4 : 1;    // the stencil row of the home's own row (oy = oz = 0)
-    constexpr int U = 8;                      // screen group; lists keep U slots free (lcap >= U)
+    constexpr int U = 8;                      // candidates per screen group
     constexpr int NW = BS / kWave;
-    constexpr int PER = 256 / BS;             // count bins per thread in the balanced deal
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_part[kMaxParts][3];      // row, first column, last column
     __shared__ uint32_t s_cnt[NW + 1];
     __shared__ unsigned long long s_pairs[NW];
-    __shared__ uint32_t s_qc[NW][kDealKeys];
-    __shared__ uint32_t s_deal[BS];
-    // balanced path: per home its staged index, kept candidates and mask words
+    __shared__ uint16_t s_deal[BS];
+    // per home: its staged index, kept candidates and first mask word
     __shared__ uint16_t s_si[BS], s_hc[BS], s_wo[BS];
     __shared__ uint32_t s_bin[256];
 
-    const ForceLds L = force_lds_layout(DIM, DEBUG, a.ntypes_max, MLDS, a.cap, a.lcap, BS, a.max_cells,
-                                        a.wpool);
+    const ForceLds L = force_lds_layout(DIM, DEBUG, a.ntypes_max, MLDS, a.cap, BS, a.max_cells,
+                                        a.wpool, a.wpool2);
     double *M = reinterpret_cast<double *>(smem + L.m);
     uint2 *sxy = reinterpret_cast<uint2 *>(smem + L.sxy);
-    uint32_t *sq = reinterpret_cast<uint32_t *>(smem + L.sq);
-    uint16_t *sqz = reinterpret_cast<uint16_t *>(smem + L.sqz);
-    uint16_t *lists = reinterpret_cast<uint16_t *>(smem + L.lists);
-    uint32_t *wmask = reinterpret_cast<uint32_t *>(smem + L.lists);     // balanced path: same region
-    uint16_t *wbase = reinterpret_cast<uint16_t *>(smem + L.wbase);
     uint32_t *szz = reinterpret_cast<uint32_t *>(smem + L.sz);
     uint32_t *sid = reinterpret_cast<uint32_t *>(smem + L.sid);
     uint32_t *off = reinterpret_cast<uint32_t *>(smem + L.off);
@@ -453,28 +645,26 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     if constexpr (MLDS)
         for (int t = tid; t < w.ntypes * w.ntypes; t += BS) M[t] = a.matrix[w.moff + t] * w.R;
 
-    // Thread tid first stands for home g0 + tid (sorted order), to find the
-    // parts: grid rows (2D: cy; 3D: cy + cz*nx) and columns of the homes.
-    // Its position and type, and the origin's (home g0) position, are read
-    // up front: independent loads whose latency overlaps the setup.
-    const bool active0 = tid < nact;
-    const int gs0 = g0 + (active0 ? tid : nact - 1);
-    const uint32_t ho0 = a.perm[gs0];
-    const uint32_t hx0 = a.sx[ho0], hy0 = a.sy[ho0], hz0 = DIM == 3 ? a.sz[ho0] : 0u;
-    const int htype0 = a.type[ho0];
-    const uint32_t go = a.perm[g0];
-    const uint32_t ox = a.sx[go], oy = a.sy[go], oz = DIM == 3 ? a.sz[go] : 0u;
-    const uint32_t hkey0 = a.skeys[gs0] - cb;
-    const int hrow0 = (int)(hkey0 / (uint32_t)nx);
-    const int hcx0 = (int)(hkey0 - (uint32_t)hrow0 * (uint32_t)nx);
+    // Thread tid stands for home g0 + tid (sorted order).  Parts: grid rows (2D:
+    // cy; 3D: cy + cz*nx) and columns of the homes.
+    // Its position and type are read up front: independent loads whose
+    // latency overlaps the setup.
+    const bool active = tid < nact;
+    const int g = g0 + (active ? tid : nact - 1);
+    const uint32_t ho = a.perm[g];
+    const uint32_t hx = a.sx[ho], hy = a.sy[ho], hz = DIM == 3 ? a.sz[ho] : 0u;
+    const int htype = a.type[ho];
+    const uint32_t hkey = a.skeys[g] - cb;
+    const int hrow = (int)(hkey / (uint32_t)nx);
+    const int hcx = (int)(hkey - (uint32_t)hrow * (uint32_t)nx);
 
     // parts = distinct rows among the homes (rows are non-decreasing with tid);
     // only active threads past the first read the previous home's key, so the
     // read stays inside [g0, g0 + nact)
-    const int prow = (tid > 0 && active0) ? (int)((a.skeys[gs0 - 1] - cb) / (uint32_t)nx) : -1;
-    const bool pstart = active0 && (tid == 0 || prow != hrow0);
-    const int nrow_next = (tid + 1 < nact) ? (int)((a.skeys[gs0 + 1] - cb) / (uint32_t)nx) : -1;
-    const bool pend = active0 && (tid + 1 == nact || nrow_next != hrow0);
+    const int prow = (tid > 0 && active) ? (int)((a.skeys[g - 1] - cb) / (uint32_t)nx) : -1;
+    const bool pstart = active && (tid == 0 || prow != hrow);
+    const int nrow_next = (tid + 1 < nact) ? (int)((a.skeys[g + 1] - cb) / (uint32_t)nx) : -1;
+    const bool pend = active && (tid + 1 == nact || nrow_next != hrow);
     const uint64_t wstarts = __ballot(pstart);
     if (lane == 0) s_cnt[wv] = (uint32_t)__popcll(wstarts);
     __syncthreads();
@@ -485,12 +675,12 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
         nparts += s_cnt[w];
     }
     const uint64_t le = lane == 63 ? ~0ull : ((2ull << lane) - 1);
-    const int mypart0 = (int)(before + __popcll(wstarts & le)) - 1;
-    if (pstart && mypart0 < kMaxParts) {
-        s_part[mypart0][0] = hrow0;
-        s_part[mypart0][1] = hcx0;
+    const int mypart = (int)(before + __popcll(wstarts & le)) - 1;
+    if (pstart && mypart < kMaxParts) {
+        s_part[mypart][0] = hrow;
+        s_part[mypart][1] = hcx;
     }
-    if (pend && mypart0 < kMaxParts) s_part[mypart0][2] = hcx0;
+    if (pend && mypart < kMaxParts) s_part[mypart][2] = hcx;
     __syncthreads();
 
     int p_row[kMaxParts], p_ca[kMaxParts], p_w[kMaxParts], p_base[kMaxParts + 1];
@@ -506,200 +696,24 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     const int NC = p_base[kMaxParts];
     const bool use_lds = !w.all_global && a.cap > 0 && nparts <= (uint32_t)kMaxParts && NC <= a.max_cells;
 
-    // staged cells: start and count, then an exclusive prefix in LDS (carry ends
-    // as the staged particle count, the same in every thread)
     uint32_t carry = 0;
-    if (use_lds) {
-        for (int f0 = 0; f0 < NC; f0 += BS) {
-            const int f = f0 + tid;
-            uint32_t c = 0;
-            if (f < NC) {
-                int pb = p_base[0], pw = p_w[0], pr = p_row[0], pc = p_ca[0];
-#pragma unroll
-                for (int q = 1; q < kMaxParts; ++q)
-                    if (f >= p_base[q] && p_w[q] > 0) { pb = p_base[q]; pw = p_w[q]; pr = p_row[q]; pc = p_ca[q]; }
-                const int r = (f - pb) / pw, j = (f - pb) - r * pw;
-                const int oy = (r % 3) - 1, oz = DIM == 3 ? (r / 3) - 1 : 0;
-                const int cy = pr % nx, cz = DIM == 3 ? pr / nx : 0;
-                const int x = wrap_cell(pc - 1 + j, nx);
-                const int y = wrap_cell(cy + oy, nx);
-                const int z = DIM == 3 ? wrap_cell(cz + oz, nx) : 0;
-                const uint32_t ci = cb + (uint32_t)(x + y * nx + z * nx * nx);
-                const uint32_t s0 = a.cell_start[ci];
-                c = a.cell_end[ci] - s0;
-                gs[f] = s0;
-            }
-            const uint32_t inc = wave_incl_scan(c);
-            if (lane == kWave - 1) s_cnt[wv] = inc;
-            __syncthreads();
-            uint32_t wbase0 = carry, tot = 0;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                wbase0 += w < wv ? s_cnt[w] : 0u;
-                tot += s_cnt[w];
-            }
-            if (f < NC) off[f] = wbase0 + inc - c;
-            carry += tot;
-            __syncthreads();
-        }
-        if (tid == 0) off[NC] = carry;
-    }
-    __syncthreads();
+    if (use_lds) carry = stage_cells<DIM, BS>(a, p_base, p_w, p_row, p_ca, nx, cb, off, gs, s_cnt);
+    else __syncthreads();
 
-    // Balanced path: the whole staged neighbourhood fits one window and the
-    // homes' candidate runs fit the pool of mask words (a run of len
-    // candidates takes ceil(len / 32) words; known here from the staged
-    // offsets, so each home gets its own run of the pool).  Homes are then
-    // screened in their sorted order and stepped, after a deal by their
-    // kept-candidate counts, by lanes of nearly equal work.
-    const int S = (int)carry;
-    bool bal = false;
-    if (use_lds && a.wpool > 0 && S <= a.cap) {
-        int need = 0;
-        if (active0) {
-            int pb = p_base[0], pw = p_w[0], pc = p_ca[0];
-#pragma unroll
-            for (int q = 1; q < kMaxParts; ++q)
-                if (mypart0 == q) { pb = p_base[q]; pw = p_w[q]; pc = p_ca[q]; }
-            const int jh = hcx0 - pc + 1;
-            for (int r = 0; r < NR; ++r) {
-                const int rb = pb + r * pw;
-                need += ((int)(off[rb + jh + 2] - off[rb + jh - 1]) + 31) >> 5;
-            }
-        }
-        uint32_t total = 0;
-        const uint32_t woff = block_excl_scan<BS>((uint32_t)need, s_cnt, total);
-        s_wo[tid] = (uint16_t)woff;
-        bal = total <= (uint32_t)a.wpool;
-    }
-
-    // Windowed path: deal the homes to threads grouped by where they sit in
-    // their cell (y quartile in 2D, y/z halves in 3D; stable within a group).
-    // A home's accepted candidates bunch in the stencil rows nearest to it, so
-    // lanes of one wave then fill their candidate lists at similar rates and
-    // list flushes keep more lanes busy.  Each home's own work is unchanged.
-    // The balanced path screens home tid on thread tid.
-    uint32_t dealt = (uint32_t)tid | ((uint32_t)max(0, min(mypart0, 255)) << 16);
-    if (!bal) {
-        const int dkey = active0 ? deal_key<DIM>(hy0, hz0, hrow0, nx, w.cs) : kDealKeys - 1;
-        const uint64_t lt = (1ull << lane) - 1;
-        uint32_t myrank = 0;
-#pragma unroll
-        for (int q = 0; q < kDealKeys; ++q) {
-            const uint64_t b = __ballot(dkey == q);
-            if (lane == 0) s_qc[wv][q] = (uint32_t)__popcll(b);
-            if (dkey == q) myrank = (uint32_t)__popcll(b & lt);
-        }
-        __syncthreads();
-        for (int q = 0; q < kDealKeys; ++q)
-#pragma unroll
-            for (int v = 0; v < NW; ++v)
-                myrank += (q < dkey || (q == dkey && v < wv)) ? s_qc[v][q] : 0u;
-        s_deal[myrank] = dealt;
-        __syncthreads();
-        dealt = s_deal[tid];
-    }
-
-    // this thread's home (after the deal)
-    const int th = (int)(dealt & 0xFFFFu);
-    const int mypart = (int)(dealt >> 16);
-    const bool active = th < nact;
-    const int g = g0 + (active ? th : nact - 1);
-    // (the balanced path keeps home tid: its data is already here)
-    const uint32_t hkey = bal ? hkey0 : a.skeys[g] - cb;
-    const int hrow = (int)(hkey / (uint32_t)nx);
-    const int hcx = (int)(hkey - (uint32_t)hrow * (uint32_t)nx);
-    const uint32_t ho = bal ? ho0 : a.perm[g];
-    const uint32_t hx = bal ? hx0 : a.sx[ho], hy = bal ? hy0 : a.sy[ho];
-    const uint32_t hz = DIM == 3 ? (bal ? hz0 : a.sz[ho]) : 0u;
-    const int htype = bal ? htype0 : a.type[ho];
     const int mrow = htype * w.ntypes;
-
-    // 3D phase A screens on 16-bit positions relative to the workgroup's first
-    // home: rel = (int32)(p - origin) >> sh, with sh chosen so that every
-    // staged particle and home lies within 2^14 units of the origin (periodic
-    // distance, in cells, bounded from the parts' staged ranges).  Relative
-    // differences equal the minimum-image differences only while everything
-    // lies within a quarter box of the origin (two such points are less than
-    // half a box apart); wider workgroups (coarse grids, sparse parts) screen
-    // on the exact 32-bit differences instead.
-    int sh = 0, bq = 0;
-    bool narrow = false;
-    {
-        const uint32_t okey = a.skeys[g0] - cb;
-        const int orow = (int)(okey / (uint32_t)nx);
-        const int ocx = (int)(okey - (uint32_t)orow * (uint32_t)nx);
-        const int ocy = orow % nx, ocz = DIM == 3 ? orow / nx : 0;
-        int ext = 0;
-#pragma unroll
-        for (int p = 0; p < kMaxParts; ++p) {
-            if (p >= (int)nparts) break;
-            const int cy = p_row[p] % nx, cz = DIM == 3 ? p_row[p] / nx : 0;
-            ext = max(ext, periodic_cells(p_ca[p] - 1, ocx, nx) + p_w[p]);
-            ext = max(ext, periodic_cells(cy, ocy, nx) + 2);
-            if (DIM == 3) ext = max(ext, periodic_cells(cz, ocz, nx) + 2);
-        }
-        // + 3 cells: positions inside the particle's and the origin's cells
-        // (the last cell of a row can be up to twice as wide)
-        const double span_units = (double)(ext + 3) * w.cs * kFix;
-        narrow = span_units < 0.25 * kFix;
-        while (sh < 31 && span_units >= 16384.0 * (double)(1u << sh)) ++sh;
-        // |D|^2 <= rmax^2 implies sum (D_i / 2^sh)^2 in quantised units <= (Rq + 2)^2
-        const double rq = w.cs * kFix * (1.0 + 0x1p-20) / (double)(1u << sh) + 2.0;
-        bq = (int)fmin(2147483647.0, floor(rq * rq) + 1.0);
-    }
 
     // The force law's two additive constants held in VGPRs: each meets
     // another scalar operand in an FMA, which reads one scalar at most.
     WorldDev wf = w;
     asm volatile("" : "+v"(wf.one_plus_beta));
     asm volatile("" : "+v"(wf.inv_beta));
-    // One candidate k of the staged window for a home at (px, py, pz) with
-    // matrix row prow_m: the reference's FP64 predicate and force law.
-    auto visit = [&](Acc &ac, int k, uint32_t px, uint32_t py, uint32_t pz, int prow_m) {
-        const uint2 q = sxy[k];
-        const int dxi = (int)(q.x - px), dyi = (int)(q.y - py);
-        const int dzi = DIM == 3 ? (int)(szz[k] - pz) : 0;
-        bool ok = true;
-        if constexpr (!WRAP) {
-            // plain difference of the clamped world: |D| >= 1/2 unless the
-            // int32 difference has the sign of the unsigned order
-            ok = ((dxi >= 0) == (q.x >= px)) & ((dyi >= 0) == (q.y >= py));
-            if (DIM == 3) ok &= ((dzi >= 0) == (szz[k] >= pz));
-        }
-        const int idx = prow_m + (int)st[k];
-        const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-        pair64_sel<DIM, DEBUG>(ac, ok, dxi, dyi, dzi, m, DEBUG ? sid[k] : 0u, wf);
-    };
-    // Stages window [w0, w0 + wn) of the staged neighbourhood.
-    auto stage = [&](int w0, int wn) {
-        for (int s = tid; s < wn; s += BS) {
-            const int sg = w0 + s;
-            int lo = 0, hi = NC;           // off[lo] <= sg < off[hi]
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (off[mid] <= (uint32_t)sg) lo = mid;
-                else hi = mid;
-            }
-            const uint32_t q = a.perm[gs[lo] + ((uint32_t)sg - off[lo])];
-            const uint32_t qx = a.sx[q], qy = a.sy[q];
-            sxy[s] = make_uint2(qx, qy);
-            if constexpr (DIM == 3) {
-                const uint32_t qz = a.sz[q];
-                szz[s] = qz;
-                sq[s] = rel16(qx, ox, sh) | (rel16(qy, oy, sh) << 16);
-                sqz[s] = (uint16_t)rel16(qz, oz, sh);
-            }
-            if constexpr (DEBUG) sid[s] = (uint32_t)a.id[q];
-            st[s] = (uint8_t)a.type[q];
-        }
-    };
+    const Staged stg{sxy, szz, sid, st};
 
     Acc acc;
     acc.x = acc.y = acc.z = 0.0;
     acc.cnt = 0;
     acc.hash = 0ull;
-    unsigned long long mycnt = 0;      // interacting pairs of the homes this thread finished
+    unsigned long long mycnt = 0;      // interacting pairs this thread stepped
     if (use_lds) {
         int pb = p_base[0], pw = p_w[0], pc = p_ca[0];
 #pragma unroll
@@ -717,216 +731,184 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
         if (cy == nx - 1) q2y = stencil_origin(hy, w.cs) == nx;
         if (DIM == 3 && cz == nx - 1) q2z = stencil_origin(hz, w.cs) == nx;
         const int j_lo = jh - 1 + (q2x ? 1 : 0);
-        const uint32_t hq = rel16(hx, ox, sh) | (rel16(hy, oy, sh) << 16);
-        const uint32_t hqz = DIM == 3 ? rel16(hz, oz, sh) : 0u;
+        const uint32_t hq = high_halves(hx, hy);
 
-        // U candidates from base kb of a row run of len (lane-local offset i):
-        // bit u set when candidate kb + u passes the phase-A screen
-        // NARROW (3D): on the staged 16-bit copies; otherwise FP32 on the
-        // exact differences.  Bits at or past the run's end (i + u >= len)
-        // stay clear.
-        auto screen_group = [&](auto narrow_tag, int kb, int i, int len) -> uint32_t {
-            constexpr bool NARROW = decltype(narrow_tag)::value;
-            uint32_t keep = 0;
-            if constexpr (NARROW && DIM == 3) {
-                const uint32_t *qp = sq + kb;
-                const uint16_t *qzp = sqz + kb;
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    keep |= screen16<DIM>(qp[u], hq, (uint32_t)qzp[u], hqz, bq) ? (1u << u) : 0u;
-            } else {
-                const uint2 *qp = sxy + kb;
-                const uint32_t *qzp = szz + kb;
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    keep |= screen<DIM>(hx, hy, hz, qp[u].x, qp[u].y, DIM == 3 ? qzp[u] : 0u, w.r2hi)
-                                ? (1u << u) : 0u;
-            }
-            const int nv = min(max(len - i, 0), U);
-            return keep & ((1u << nv) - 1u);
+        // The home's run of stencil row r inside the window [w0, w0 + wn),
+        // window-relative: returns its length, its first entry in lo.
+        auto run_of = [&](int r, int w0, int wn, int &lo) -> int {
+            const int oyr = (r % 3) - 1, ozr = DIM == 3 ? (r / 3) - 1 : 0;
+            const bool skip = !active || (q2y && oyr == -1) || (q2z && ozr == -1);
+            const int rb = pb + r * pw;
+            lo = max((int)off[rb + j_lo] - w0, 0);
+            const int hi = min((int)off[rb + jh + 2] - w0, wn);
+            return skip ? 0 : max(0, hi - lo);
         };
-
-        if (bal) {
-            // ---- balanced path: one window -------------------------------
-            stage(0, S);
-            __syncthreads();
-            // Phase A: thread tid screens home tid; each 32 candidates of a row
-            // run give one mask word, stored (with its first candidate's index)
-            // when any candidate passed.
-            int nwd = 0, npass = 0;
-            const int wo = s_wo[tid];          // this home's run of the word pool
-            auto scan_words = [&](auto narrow_tag) {
+        // First mask word of each home in the pool (s_wo) for a window, a run of
+        // len candidates taking ceil(len / 32) words; returns the words needed.
+        auto place_words = [&](int w0, int wn) -> uint32_t {
+            int need = 0;
 #pragma unroll 1
-                for (int r = 0; r < NR; ++r) {
-                    const int oyr = (r % 3) - 1, ozr = DIM == 3 ? (r / 3) - 1 : 0;
-                    const bool skip = !active || (q2y && oyr == -1) || (q2z && ozr == -1);
-                    const int rb = pb + r * pw;
-                    const int klo = (int)off[rb + j_lo];
-                    const int len = skip ? 0 : max(0, (int)off[rb + jh + 2] - klo);
-                    const int K = wave_max(len);
-                    for (int i = 0; i < K; i += 4 * U) {
-                        uint32_t word = 0;
+            for (int r = 0; r < NR; ++r) {
+                int lo;
+                need += (run_of(r, w0, wn, lo) + 31) >> 5;
+            }
+            uint32_t total = 0;
+            s_wo[tid] = (uint16_t)block_excl_scan<BS>((uint32_t)need, s_cnt, total);
+            return total;
+        };
+        // Phase A: thread tid screens home tid; each 32 candidates of a row run
+        // give one mask word, stored (with its first candidate's index) when any
+        // candidate passed.  Returns the kept candidates.
+        auto screen_home = [&](int w0, int wn, uint32_t *wmask, uint16_t *wbase) -> int {
+            int at = s_wo[tid], npass = 0;
+#pragma unroll 1
+            for (int r = 0; r < NR; ++r) {
+                int klo;
+                const int len = run_of(r, w0, wn, klo);
+                const int K = wave_max(len);
+#pragma unroll 1
+                for (int i = 0; i < K; i += 4 * U) {
+                    // a lane past its run reads the window's first entries
+                    // (and keeps none of them)
+                    const int kb = i < len ? klo + i : 0;
+                    uint32_t word = 0;
 #pragma unroll
-                        for (int gq = 0; gq < 4; ++gq) {
-                            const int ig = i + gq * U;
-                            if (ig < K) {
-                                // a lane past its run reads the window's first entries
-                                // (and keeps none of them)
-                                const int kb = ig < len ? klo + ig : 0;
-                                word |= screen_group(narrow_tag, kb, ig, len) << (gq * U);
-                            }
-                        }
-                        if (word) {
-                            wmask[wo + nwd] = word;
-                            wbase[wo + nwd] = (uint16_t)(klo + i);
-                            ++nwd;
-                            npass += __popc(word);
-                        }
+                    for (int gq = 3; gq >= 0; --gq)
+                        if (i + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, hz, w.sbias, word);
+                    word &= low_bits(len - i);
+                    if (word) {
+                        wmask[at] = word;
+                        wbase[at] = (uint16_t)kb;
+                        ++at;
+                        npass += __popc(word);
                     }
                 }
-            };
-            // 2D screens on the 32-bit differences: its FP32 screen is short;
-            // 3D gains 2/3 of its screen on the 16-bit copies
-            if constexpr (DIM == 3) {
-                if (narrow) scan_words(std::true_type{});
-                else scan_words(std::false_type{});
-            } else {
-                scan_words(std::false_type{});
             }
+            return npass;
+        };
+
+        const int S = (int)carry;
+        if (a.wpool > 0 && S <= a.cap && place_words(0, S) <= (uint32_t)a.wpool) {
+            // ---- one window ----------------------------------------------
+            uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words);
+            uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase);
+            stage_window<DIM, DEBUG, BS>(a, stg, off, gs, NC, 0, S);
+            __syncthreads();
+            const int count[1] = {screen_home(0, S, wmask, wbase)};
             int si = 0;
             if (active) {
                 const int f = pb + RMID * pw + jh;
                 si = (int)off[f] + (g - (int)gs[f]);
             }
             s_si[tid] = (uint16_t)si;
-            s_hc[tid] = (uint16_t)(active ? npass : 0);
-            // Deal the homes by their kept-candidate counts (a counting sort;
-            // the order inside a count does not matter): lane tid of the
-            // workgroup steps the home of rank tid, so the lanes of a wave
-            // carry nearly equal work.  Each home is stepped whole by one lane
-            // in its scan order, so its sums are those of the windowed path.
-            for (int t = tid; t < 256; t += BS) s_bin[t] = 0u;
-            __syncthreads();
-            const int cbin = min(active ? npass : 0, 255);
-            const uint32_t local = atomicAdd(&s_bin[cbin], 1u);
-            __syncthreads();
-            {
-                uint32_t v[PER], sum = 0, total = 0;
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    v[q] = s_bin[tid * PER + q];
-                    sum += v[q];
-                }
-                uint32_t ex = block_excl_scan<BS>(sum, s_cnt, total);
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    s_bin[tid * PER + q] = ex;
-                    ex += v[q];
-                }
-            }
-            __syncthreads();
-            s_deal[s_bin[cbin] + local] = (uint32_t)tid;
-            __syncthreads();
-
-            // Phase B: the home of rank tid, its kept candidates word by word
+            s_hc[tid] = (uint16_t)count[0];
+            // Phase B: lane tid steps the home of count rank tid whole, in its
+            // scan order, so its sums do not depend on the windows.
+            deal_homes<BS, 1>(count, 0, s_bin, s_deal, s_cnt);
             const int h = (int)s_deal[tid];
             if (h < nact) {
                 const int hsi = s_si[h];
-                const uint2 hp = sxy[hsi];
+                const uint2 hhl = sxy[hsi];
+                const uint2 hp = make_uint2(join_x(hhl), join_y(hhl));
                 const uint32_t bhz = DIM == 3 ? szz[hsi] : 0u;
                 const int btype = (int)st[hsi];
-                const int bmrow = btype * w.ntypes;
                 Acc ab;
                 ab.x = ab.y = ab.z = 0.0;
                 ab.cnt = 0;
                 ab.hash = 0ull;
-                int left = s_hc[h], j = s_wo[h], kb = 0;
-                uint32_t m = 0;
-                auto next = [&]() {
-                    if (m == 0) {
-                        m = wmask[j];
-                        kb = wbase[j];
-                        ++j;
-                    }
-                    const int k = kb + __builtin_ctz(m);
-                    m &= m - 1u;
-                    return k;
-                };
-                // two candidates per iteration (half the loop's bookkeeping;
-                // their force laws overlap), added in candidate order
-#pragma unroll 1
-                for (; left >= 2; left -= 2) {
-                    const int k1 = next();
-                    const int k2 = next();
-                    visit(ab, k1, hp.x, hp.y, bhz, bmrow);
-                    visit(ab, k2, hp.x, hp.y, bhz, bmrow);
-                }
-                if (left > 0) visit(ab, next(), hp.x, hp.y, bhz, bmrow);
+                int j = s_wo[h];
+                walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, (int)s_hc[h], [&](uint32_t &m, int &kb) {
+                    m = wmask[j];
+                    kb = wbase[j];
+                    ++j;
+                }, hp.x, hp.y, bhz, btype * w.ntypes);
                 const int gh = g0 + h;
                 finish_home<DIM, WRAP, DEBUG>(a, w, ab, hp.x, hp.y, bhz, btype, a.perm[gh], gh);
                 mycnt = (unsigned long long)ab.cnt;
             }
         } else {
-            // ---- windowed path --------------------------------------------
-            // The staged neighbourhood is S particles; it is brought into LDS in
-            // windows of at most cap (one window for ordinary densities, several
-            // for clustered cells) and every lane scans its ranges clipped to it.
-            for (int w0 = 0; w0 < S; w0 += a.cap) {
-                const int wn = min(a.cap, S - w0);
-                stage(w0, wn);
+            // ---- several windows -----------------------------------------
+            // The staged neighbourhood streams through LDS in windows of at most
+            // cap entries and wpool2 mask words.  Each window's homes are dealt to
+            // lanes by their counts of that window; a home's sums travel in LDS
+            // from the lane that stepped it in one window to the lane that steps
+            // it in the next, so its candidates are added in staged order
+            // whatever the windows are.  (Per-thread candidate lists, flushed when
+            // one lane's list filled, kept a third to a half of phase B's lanes
+            // busy.)
+            double *const ax = reinterpret_cast<double *>(smem + L.ax);
+            double *const ay = reinterpret_cast<double *>(smem + L.ay);
+            double *const az = reinterpret_cast<double *>(smem + L.az);
+            unsigned long long *const dhash = reinterpret_cast<unsigned long long *>(smem + L.dhash);
+            int *const dcnt = reinterpret_cast<int *>(smem + L.dcnt);
+            uint2 *const hxy = reinterpret_cast<uint2 *>(smem + L.hxy);
+            uint32_t *const hzz = reinterpret_cast<uint32_t *>(smem + L.hz);
+            uint8_t *const ht = smem + L.ht;
+            uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words2);
+            uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase2);
+            ax[tid] = ay[tid] = 0.0;
+            hxy[tid] = make_uint2(hx, hy);
+            ht[tid] = (uint8_t)htype;
+            if constexpr (DIM == 3) {
+                az[tid] = 0.0;
+                hzz[tid] = hz;
+            }
+            if constexpr (DEBUG) {
+                dhash[tid] = 0ull;
+                dcnt[tid] = 0;
+            }
+            for (int w0 = 0; w0 < S;) {
+                // one entry needs a word per home at most, and wpool2 >= BS
+                int wn = min(a.cap, S - w0);
+                while (place_words(w0, wn) > (uint32_t)a.wpool2) wn = (wn + 1) >> 1;
+                stage_window<DIM, DEBUG, BS>(a, stg, off, gs, NC, w0, wn);
                 __syncthreads();
-
-                // Per-lane candidate list: entries at lists[j * BS + tid]; lp walks
-                // the lane's column of the list in steps of BS entries.
-                uint16_t *const lbase = lists + tid;
-                uint16_t *lp = lbase;
-                uint16_t *const lfull = lbase + (a.lcap - U) * BS;     // flush beyond this
-                auto flush = [&]() {
-                    for (uint16_t *e = lbase; e < lp; e += BS) visit(acc, *e, hx, hy, hz, mrow);
-                    lp = lbase;
-                };
-                // the row scan, instantiated for the 16-bit and the 32-bit screen
-                auto scan_rows = [&](auto narrow_tag) {
-#pragma unroll 1
-                    for (int r = 0; r < NR; ++r) {
-                        const int oyr = (r % 3) - 1, ozr = DIM == 3 ? (r / 3) - 1 : 0;
-                        const bool skip = !active || (q2y && oyr == -1) || (q2z && ozr == -1);
-                        const int rb = pb + r * pw;
-                        const int klo = max((int)off[rb + j_lo], w0) - w0;
-                        const int khi = min((int)off[rb + jh + 2], w0 + wn) - w0;
-                        const int len = skip ? 0 : max(0, khi - klo);
-                        const int K = wave_max(len);
-                        for (int i = 0; i < K; i += U) {
-                            if (__any(lp > lfull)) flush();
-                            // U candidates from one base: a lane past its range reads the
-                            // window's first entries instead (and keeps none of them)
-                            const int kb = i < len ? klo + i : 0;
-                            const uint32_t keep = screen_group(narrow_tag, kb, i, len);
-                            // branch-free append: every candidate is written to the next
-                            // free slot, which only a kept one claims (the flush check
-                            // above leaves room for U slots)
-#pragma unroll
-                            for (int u = 0; u < U; ++u) {
-                                *lp = (uint16_t)(kb + u);
-                                lp += ((keep >> u) & 1u) ? BS : 0;
-                            }
-                        }
+                const int count[1] = {screen_home(w0, wn, wmask, wbase)};
+                s_hc[tid] = (uint16_t)count[0];
+                int shift = 0;
+                while ((wn >> shift) > 256) ++shift;
+                deal_homes<BS, 1>(count, shift, s_bin, s_deal, s_cnt);
+                const int h = (int)s_deal[tid];
+                const int left = (int)s_hc[h];
+                if (left > 0) {
+                    Acc ab;
+                    ab.x = ax[h];
+                    ab.y = ay[h];
+                    ab.z = DIM == 3 ? az[h] : 0.0;
+                    ab.cnt = 0;
+                    ab.hash = 0ull;
+                    const uint2 hp = hxy[h];
+                    int j = s_wo[h];
+                    walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, left, [&](uint32_t &m, int &kb) {
+                        m = wmask[j];
+                        kb = wbase[j];
+                        ++j;
+                    }, hp.x, hp.y, DIM == 3 ? hzz[h] : 0u, (int)ht[h] * w.ntypes);
+                    ax[h] = ab.x;
+                    ay[h] = ab.y;
+                    if constexpr (DIM == 3) az[h] = ab.z;
+                    if constexpr (DEBUG) {
+                        dcnt[h] += ab.cnt;
+                        dhash[h] += ab.hash;
                     }
-                };
-                if constexpr (DIM == 3) {
-                    if (narrow) scan_rows(std::true_type{});
-                    else scan_rows(std::false_type{});
-                } else {
-                    scan_rows(std::false_type{});
+                    mycnt += (unsigned long long)ab.cnt;
                 }
-                flush();
                 __syncthreads();
+                w0 += wn;
+            }
+            if (active) {
+                acc.x = ax[tid];
+                acc.y = ay[tid];
+                if constexpr (DIM == 3) acc.z = az[tid];
+                if constexpr (DEBUG) {
+                    acc.cnt = dcnt[tid];
+                    acc.hash = dhash[tid];
+                }
+                finish_home<DIM, WRAP, DEBUG>(a, w, acc, hx, hy, hz, htype, ho, g);
             }
         }
     } else if (active) {
         home_global<DIM, WRAP, DEBUG, MLDS>(a, w, M, g, hx, hy, hz, mrow, acc);
-    }
-    if (!bal && active) {
         finish_home<DIM, WRAP, DEBUG>(a, w, acc, hx, hy, hz, htype, ho, g);
         mycnt = (unsigned long long)acc.cnt;
     }

@@ -135,6 +135,7 @@ struct WorldDev {
     int ntypes, moff;                // matrix size and offset (doubles) in the batch matrix
     int wrap;
     float r2hi;                      // screen bound, units 2^-64: (rmax 2^32)^2 (1 + 2^-20)
+    int sbias;                       // screen bound on 16-bit coordinates: -(bq + 1) (screen_hi)
     double cs;                       // cell size = rmax (Physics.java:312)
     double r2u;                      // fl(rmax*rmax) * 2^64: the reference's bound in units 2^-64
     double S;                        // 2^-32 / rmax: |rel| = |D| S with D in units 2^-32
