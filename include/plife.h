@@ -241,7 +241,7 @@ int plife_get_tuning(plife_physics *h, plife_tuning *t, int32_t *lds_bytes);
  * reference: it is for callers that cannot allocate -- code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It runs
  * plife_update's kernels, with every buffer they need beyond the state in a
- * static device array of the library (19.1 MB, held by each GPU the
+ * static device array of the library (21.0 MB, held by each GPU the
  * library runs on until the process ends); it calls no hipMalloc, hipFree
  * or memset/memcpy, only kernel launches.
  *   - State in the device layout (plife_update's): positions as 32-bit

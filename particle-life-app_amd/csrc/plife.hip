@@ -2,9 +2,9 @@
 //
 // Host orchestration of Physics.update() (backend/Physics.java:112-134) for a
 // batch of independent worlds; the single-world handle is a batch of one:
-//   bin (cell keys + cell histogram + first digit histogram) -> scans ->
-//   stable radix sort -> force + integrate (reads the pre-sort state through
-//   the permutation, writes the cell-sorted new state),
+//   bin (cell keys + cell histogram) -> cell scan -> place + rank (the stable
+//   counting sort; gathers sorted position records) -> force + integrate
+//   (writes the cell-sorted new state),
 // all enqueued on the handle's own stream.  No torch, no CPU fallback: every
 // step runs the HIP kernels of plife_kernels.hpp and plife_force.hpp.
 //
@@ -229,13 +229,15 @@ struct plife_physics {
     int pc = 0, ac = 0;
 
     // binning / sort scratch
-    uint32_t *keys0 = nullptr, *kA = nullptr, *kB = nullptr, *vA = nullptr, *vB = nullptr;
-    uint32_t *skeys = nullptr;         // batch cell key of each sorted slot (last radix pass)
-    uint32_t *perm = nullptr;          // points at vA or vB after a step
+    uint32_t *keys0 = nullptr;         // batch cell key of each pre-sort slot
+    uint32_t *kA = nullptr;            // the sort's arrival order; the one-launch step's second key buffer
+    uint32_t *skeys = nullptr;         // batch cell key of each sorted slot
+    uint32_t *perm = nullptr;          // sorted slot -> pre-sort slot (before that: arrival places)
+    uint4 *rec = nullptr;              // x, y, z, type of each sorted slot
     size_t cells_cap = 0;
     uint32_t *cell_count = nullptr, *cell_start = nullptr, *cell_end = nullptr;
-    size_t hist_cap = 0, bsum_cap = 0;
-    uint32_t *hist = nullptr, *bsum = nullptr;
+    size_t bsum_cap = 0;
+    uint32_t *bsum = nullptr;
     unsigned long long *bsq = nullptr;   // per-block sums of squares of the cell scan
     size_t bsq_cap = 0;
     // [0] interacting pairs, [1] sum of cell counts^2, [2 + w] pairs of world w
@@ -345,11 +347,9 @@ void free_state(plife_physics *h)
     free_state_arrays(h->px, h->py, h->pz, h->vx, h->vy, h->vz, h->type, h->id);
     dev_free(h->keys0);
     dev_free(h->kA);
-    dev_free(h->kB);
-    dev_free(h->vA);
-    dev_free(h->vB);
     dev_free(h->skeys);
-    h->perm = nullptr;
+    dev_free(h->perm);
+    dev_free(h->rec);
     h->cap = 0;
 }
 
@@ -410,10 +410,9 @@ int ensure_capacity(plife_physics *h, int need, bool keep)
     h->pc = 0;
     h->ac = 0;
     if ((rc = dev_alloc(&h->keys0, cap))) return rc;
-    if ((rc = dev_alloc(&h->kA, cap))) return rc;
-    if ((rc = dev_alloc(&h->kB, cap))) return rc;
-    if ((rc = dev_alloc(&h->vA, cap))) return rc;
-    if ((rc = dev_alloc(&h->vB, cap))) return rc;
+    if ((rc = dev_alloc(&h->kA, (size_t)cap + kRankPad))) return rc;
+    if ((rc = dev_alloc(&h->perm, cap))) return rc;
+    if ((rc = dev_alloc(&h->rec, cap))) return rc;
     if ((rc = dev_alloc(&h->skeys, cap))) return rc;
     h->cap = cap;
     return PLIFE_OK;
@@ -478,6 +477,7 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     const double rq = s.rmax * 65536.0 * (1.0 + 0x1p-20) + std::sqrt((double)(s.dim + 3));
     d.sbias = -(int)std::min(rq * rq + 2.0, 2147483646.0);
     d.cs = s.rmax;
+    d.ics = 1.0 / s.rmax;
     d.r2u = (s.rmax * s.rmax) * (kFix * kFix);         // Physics.java:432, exact 2^64 scaling
     d.S = 1.0 / R;
     d.R = R;
@@ -738,127 +738,60 @@ int ensure_blocks(plife_physics *h, int bs)
 // scans, sort, binning, force launches
 // ---------------------------------------------------------------------------
 
-struct RadixPlan {
-    int bits, passes, D, ntiles;
-    size_t hist_len;
-};
-
-RadixPlan radix_plan(long long ncells, int n)
+// The cell scan: one launch, two, or three by size.
+int scan_cells(plife_physics *h, int ncells, unsigned long long *sq)
 {
-    RadixPlan p;
-    p.bits = 0;
-    while ((1LL << p.bits) < ncells) ++p.bits;
-    if (p.bits == 0) p.bits = 1;
-    p.passes = (p.bits + 7) / 8;
-    p.D = (p.bits + p.passes - 1) / p.passes;
-    p.ntiles = ceil_div(std::max(n, 1), kRadixTile);
-    p.hist_len = (size_t)(1 << p.D) * (size_t)p.ntiles;
-    return p;
-}
-
-ScanJob no_job() { return ScanJob{nullptr, 0, nullptr, nullptr, 0, nullptr, nullptr}; }
-
-// One or two device-wide scans sharing three launches.
-int scan_jobs(plife_physics *h, ScanJob a, ScanJob b)
-{
-    if (a.n <= 0) std::swap(a, b);
-    if (a.n <= 0) return PLIFE_OK;
-    const int nb0 = ceil_div(a.n, kScanTile), nb1 = b.n > 0 ? ceil_div(b.n, kScanTile) : 0;
-    if (a.n <= kSmallScan && b.n <= kSmallScan) {
-        k_scan_small<<<nb1 ? 2 : 1, kSmallBlock, 0, h->stream>>>(a, b);
+    const ScanJob j{h->cell_count, ncells, h->cell_start, h->cell_end, sq, h->bsum, h->bsq};
+    const int nb = ceil_div(ncells, kScanTile);
+    if (ncells <= kSmallScan) {
+        k_scan_small<<<1, kSmallBlock, 0, h->stream>>>(j);
         LAUNCH_CHECK();
         return PLIFE_OK;
     }
-    if ((size_t)(nb0 + nb1) > h->bsum_cap || !h->bsum)
+    if (!h->bsum || (size_t)nb > h->bsum_cap || !h->bsq || (size_t)nb > h->bsq_cap)
         return fail(PLIFE_ERR_STATE, "scan scratch was not prepared");
-    if ((a.sq && (!h->bsq || (size_t)nb0 > h->bsq_cap)) || b.sq)
-        return fail(PLIFE_ERR_STATE, "scan scratch was not prepared");
-    a.bsum = h->bsum;
-    b.bsum = h->bsum + nb0;
-    a.sqb = h->bsq;
-    k_scan2_reduce<<<nb0 + nb1, kBlock, 0, h->stream>>>(a, b, nb0);
-    if (nb0 <= kFoldBlocks && nb1 <= kFoldBlocks) {
-        k_scan2_down_fold<<<nb0 + nb1, kBlock, 0, h->stream>>>(a, b, nb0);
-        LAUNCH_CHECK();
-        return PLIFE_OK;
+    k_scan_reduce<<<nb, kBlock, 0, h->stream>>>(j);
+    if (nb <= kFoldBlocks) {
+        k_scan_down_fold<<<nb, kBlock, 0, h->stream>>>(j);
+    } else {
+        k_scan_single<<<1, kBlock, 0, h->stream>>>(j);
+        k_scan_down<<<nb, kBlock, 0, h->stream>>>(j);
     }
-    k_scan2_single<<<nb1 ? 2 : 1, kBlock, 0, h->stream>>>(a, b);
-    k_scan2_down<<<nb0 + nb1, kBlock, 0, h->stream>>>(a, b, nb0);
     LAUNCH_CHECK();
     return PLIFE_OK;
 }
 
-template <int D>
-int radix_pass(plife_physics *h, const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
-               uint32_t *vout, int n, int shift, int ntiles, bool hist_ready)
+// Cell keys and histogram of n particles (Physics.java:319-340), clearing the
+// step's counters.
+int bin_cells(plife_physics *h, int dim, const PosBuf &P, int n, const uint16_t *world_of, int ncounters,
+              unsigned long long tag, unsigned long long *stat_out)
 {
-    int rc;
-    if (!hist_ready) {
-        k_radix_hist<D><<<ntiles, kBlock, 0, h->stream>>>(kin, n, shift, ntiles, h->hist);
-        if ((rc = scan_jobs(h, ScanJob{h->hist, (1 << D) * ntiles, h->hist, nullptr, 0, nullptr, nullptr},
-                            no_job())))
-            return rc;
-    }
-    k_radix_scatter<D><<<ntiles, kScatterBlock, 0, h->stream>>>(kin, vin, kout, vout, h->hist, n,
-                                                                 shift, ntiles);
+    const int nb = ceil_div(n, kBlock * kBinItems);
+    if (dim == 3)
+        k_bin<3><<<nb, kBlock, 0, h->stream>>>(P.x, P.y, P.z, n, h->d_worlds, world_of, h->keys0, h->perm,
+                                               h->cell_count, h->d_pairs, ncounters, tag, stat_out);
+    else
+        k_bin<2><<<nb, kBlock, 0, h->stream>>>(P.x, P.y, P.z, n, h->d_worlds, world_of, h->keys0, h->perm,
+                                               h->cell_count, h->d_pairs, ncounters, tag, stat_out);
     LAUNCH_CHECK();
     return PLIFE_OK;
 }
 
-// Stable sort of (keys0[i], i) by key -- the reference's counting-sort
-// permutation (Physics.java:342-353).  The first pass's tile histogram is
-// already scanned in h->hist (k_bin_tile).  Leaves the permutation (sorted
-// slot -> pre-sort index) in h->perm and the sorted keys in h->skeys.
-int radix_sort(plife_physics *h, int n, const RadixPlan &plan)
+// The stable counting sort (Physics.java:342-353) once the cells are scanned:
+// leaves the permutation (sorted slot -> pre-sort index) in h->perm, the sorted
+// keys in h->skeys and the sorted records in h->rec.
+int sort_cells(plife_physics *h, int dim, const PosBuf &P, const int32_t *type, int n)
 {
-    const uint32_t *kin = h->keys0;
-    const uint32_t *vin = nullptr;
-    int rc;
-    for (int p = 0; p < plan.passes; ++p) {
-        const bool last = p == plan.passes - 1;
-        uint32_t *kout = last ? h->skeys : ((p & 1) ? h->kB : h->kA);
-        uint32_t *vout = (p & 1) ? h->vB : h->vA;
-        const int shift = p * plan.D;
-        const bool hr = p == 0;
-        switch (plan.D) {
-            case 1: rc = radix_pass<1>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 2: rc = radix_pass<2>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 3: rc = radix_pass<3>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 4: rc = radix_pass<4>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 5: rc = radix_pass<5>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 6: rc = radix_pass<6>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            case 7: rc = radix_pass<7>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-            default: rc = radix_pass<8>(h, kin, vin, kout, vout, n, shift, plan.ntiles, hr); break;
-        }
-        if (rc) return rc;
-        kin = kout;
-        vin = vout;
-    }
-    h->perm = const_cast<uint32_t *>(vin);
+    const int nb = ceil_div(n, kBlock);
+    k_place<<<nb, kBlock, 0, h->stream>>>(n, h->keys0, h->perm, h->cell_start, h->kA);
+    if (dim == 3)
+        k_rank<3><<<nb, kBlock, 0, h->stream>>>(n, h->keys0, h->kA, h->cell_start, h->cell_end, P.x, P.y, P.z,
+                                                type, h->perm, h->skeys, h->rec);
+    else
+        k_rank<2><<<nb, kBlock, 0, h->stream>>>(n, h->keys0, h->kA, h->cell_start, h->cell_end, P.x, P.y, P.z,
+                                                type, h->perm, h->skeys, h->rec);
+    LAUNCH_CHECK();
     return PLIFE_OK;
-}
-
-template <int DIM>
-void launch_bin(plife_physics *h, int D, const PosBuf &P, int n, int ntiles)
-{
-    const uint16_t *wof = h->worlds.size() > 1 ? h->world_of : nullptr;
-    const int ncounters = 2 + (int)h->worlds.size();
-#define PLIFE_BIN(DD)                                                                          \
-    k_bin_tile<DIM, DD><<<ntiles, 1024, 0, h->stream>>>(P.x, P.y, P.z, n, h->d_worlds, wof,    \
-                                                          ntiles, h->keys0, h->cell_count,     \
-                                                          h->hist, h->d_pairs, ncounters,      \
-                                                          h->version + 1, h->stat_dev)
-    switch (D) {
-        case 1: PLIFE_BIN(1); break;
-        case 2: PLIFE_BIN(2); break;
-        case 3: PLIFE_BIN(3); break;
-        case 4: PLIFE_BIN(4); break;
-        case 5: PLIFE_BIN(5); break;
-        case 6: PLIFE_BIN(6); break;
-        case 7: PLIFE_BIN(7); break;
-        default: PLIFE_BIN(8); break;
-    }
-#undef PLIFE_BIN
 }
 
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS>
@@ -1340,13 +1273,9 @@ int prepare_step(plife_physics *h)
     // buffers are prepared either way
     h->small_ok = plan_small(h);
     h->small = h->small_ok && (h->tune.small_step == 2 || (h->small_meas == h->version && h->small_pref));
-    const RadixPlan rp = radix_plan(h->ncells, h->n);
-    if ((rc = ensure_dev(&h->hist, &h->hist_cap, rp.hist_len, &h->retired))) return rc;
-    const size_t nb = (size_t)ceil_div(h->ncells, kScanTile) +
-                      (size_t)ceil_div((long long)rp.hist_len, kScanTile);
+    const size_t nb = (size_t)ceil_div(h->ncells, kScanTile);
     if ((rc = ensure_dev(&h->bsum, &h->bsum_cap, nb, &h->retired))) return rc;
-    if ((rc = ensure_dev(&h->bsq, &h->bsq_cap, (size_t)ceil_div(h->ncells, kScanTile), &h->retired)))
-        return rc;
+    if ((rc = ensure_dev(&h->bsq, &h->bsq_cap, nb, &h->retired))) return rc;
     if (h->small) return ensure_small_blocks(h);
     if ((rc = ensure_blocks(h, h->plan.bs))) return rc;
     return balance_blocks(h);
@@ -1397,7 +1326,7 @@ int do_small_step(plife_physics *h, PhaseEvents *ev)
     a.dbg_count = h->dbg_count;
     a.dbg_hash = h->dbg_hash;
     a.dbg_acc = h->dbg_acc;
-    s.perm_out = h->vA;
+    s.perm_out = h->perm;
     // the last step's sorted keys: the incremental sort's hint (checked in the kernel)
     s.skeys_in = h->small_kbuf ? h->kA : h->skeys;
     s.skeys_out = h->small_kbuf ? h->skeys : h->kA;
@@ -1429,7 +1358,6 @@ int do_small_step(plife_physics *h, PhaseEvents *ev)
     LAUNCH_CHECK();
     h->stepped = true;
     h->last_ncells = h->ncells;
-    h->perm = h->vA;
     h->small_kbuf ^= 1;
     h->last_lds = lds;
     h->last_bs = h->small_homes;
@@ -1452,57 +1380,49 @@ int do_step(plife_physics *h, PhaseEvents *ev)
         return fail(PLIFE_ERR_STATE, "the step was not prepared");
 
     if ((rc = record(h, ev, 0))) return rc;
-    const RadixPlan plan = radix_plan(h->ncells, n);
     // A step that failed between binning and scanning may leave counts behind.
     if (h->cells_dirty) {
         k_fill_u32<<<ceil_div(nc, kBlock), kBlock, 0, h->stream>>>(h->cell_count, 0u, nc);
         LAUNCH_CHECK();
     }
     h->cells_dirty = true;
-    // 1. bin (Physics.java:319-340): cell keys, cell histogram, first radix
-    //    digit histogram; then the cell scan (start / end offsets, counters
-    //    cleared for the next step) and the digit scan in one launch
+    // 1. bin (Physics.java:319-340): cell keys and histogram; then the cell scan
+    //    (start / end offsets, counters cleared for the next step)
     const PosBuf P0 = h->P(h->pc);
     if (n > 0) {
-        if (h->dim == 3) launch_bin<3>(h, plan.D, P0, n, plan.ntiles);
-        else launch_bin<2>(h, plan.D, P0, n, plan.ntiles);
+        if ((rc = bin_cells(h, h->dim, P0, n, h->worlds.size() > 1 ? h->world_of : nullptr,
+                            2 + (int)h->worlds.size(), h->version + 1, h->stat_dev)))
+            return rc;
     } else {
         const int nz = 2 + (int)h->worlds.size();
         k_zero_u64<<<ceil_div(nz, kBlock), kBlock, 0, h->stream>>>(h->d_pairs, nz);
+        LAUNCH_CHECK();
     }
-    LAUNCH_CHECK();
-    if ((rc = scan_jobs(h, ScanJob{h->cell_count, nc, h->cell_start, h->cell_end, 1, nullptr,
-                                   h->d_pairs + 1},
-                        n > 0 ? ScanJob{h->hist, (int)plan.hist_len, h->hist, nullptr, 0, nullptr, nullptr}
-                              : no_job())))
-        return rc;
+    if ((rc = scan_cells(h, nc, h->d_pairs + 1))) return rc;
     h->cells_dirty = false;
     if ((rc = record(h, ev, 1))) return rc;
 
     h->stepped = true;
     h->last_ncells = h->ncells;
     if (n == 0) {
-        h->perm = h->vA;
         for (int k = 2; k < 5; ++k)
             if ((rc = record(h, ev, k))) return rc;
         return PLIFE_OK;
     }
 
     // 2. stable sort of (key, index) = the reference's counting-sort permutation
-    if ((rc = radix_sort(h, n, plan))) return rc;
+    if ((rc = sort_cells(h, h->dim, P0, h->type[h->ac], n))) return rc;
     if ((rc = record(h, ev, 2))) return rc;
     if ((rc = record(h, ev, 3))) return rc;
 
     // 3. force + integrate (Physics.java:122-131 fused: the update is Jacobi):
     //    reads the pre-sort state through the permutation and writes the new
     //    state in cell order (the array swap, Physics.java:350-353)
-    const int pi = h->pc, ai = h->ac, po = 1 - h->pc, ao = 1 - h->ac;
+    const int ai = h->ac, po = 1 - h->pc, ao = 1 - h->ac;
     const ForcePlan &fp = h->plan;
     ForceArgs a{};
+    a.rec = h->rec;
     a.perm = h->perm;
-    a.sx = h->px[pi];
-    a.sy = h->py[pi];
-    a.sz = h->pz[pi];
     a.vx = h->vx[ai];
     a.vy = h->vy[ai];
     a.vz = h->vz[ai];
@@ -1541,7 +1461,7 @@ int do_step(plife_physics *h, PhaseEvents *ev)
     h->last_bs = fp.bs;
     h->last_lcap = fp.lcap;
     if ((rc = launch_force_any(h, a, fp.bs, fp.lds))) return rc;
-    h->small_kbuf = 0;                 // the last radix pass wrote the sorted keys to skeys
+    h->small_kbuf = 0;                 // the sort wrote the sorted keys to skeys
     if ((rc = record(h, ev, 4))) return rc;
     h->pc = po;
     h->ac = ao;
@@ -1578,8 +1498,8 @@ std::vector<unsigned char> graph_key(const plife_physics *h)
     k.blocks_serial = h->blocks_serial;
     const void *p[] = {h->px[0], h->px[1], h->py[0], h->py[1], h->pz[0], h->pz[1], h->vx[0],
                        h->vx[1], h->vy[0], h->vy[1], h->vz[0], h->vz[1], h->type[0], h->type[1],
-                       h->id[0], h->id[1], h->keys0, h->kA, h->kB, h->vA, h->vB, h->cell_count,
-                       h->cell_start, h->cell_end, h->hist, h->bsum, h->bsq, h->dbg_count, h->dbg_hash, h->dbg_acc,
+                       h->id[0], h->id[1], h->keys0, h->kA, h->perm, h->rec, h->cell_count,
+                       h->cell_start, h->cell_end, h->bsum, h->bsq, h->dbg_count, h->dbg_hash, h->dbg_acc,
                        h->d_matrix, h->d_pairs, h->d_worlds, h->world_of, h->d_blocks,
                        h->stat_host, h->work_host, h->skeys, h->d_facc};
     std::memcpy(k.ptr, p, sizeof p);
@@ -2341,7 +2261,6 @@ void destroy_handle(plife_physics *h)
     dev_free(h->cell_count);
     dev_free(h->cell_start);
     dev_free(h->cell_end);
-    dev_free(h->hist);
     dev_free(h->bsum);
     dev_free(h->bsq);
     dev_free(h->d_pairs);
@@ -2436,8 +2355,8 @@ void report_tuning(const plife_physics *h, plife_tuning *t, int32_t *lds_bytes)
 //
 // Everything a step needs beyond the caller's state arrays lives in one
 // file-scope device array, `scratch`, of fixed size: the world's constants,
-// the workgroup table, the step's counters, the keys, radix buffers and
-// permutation, and the cell arrays.  Each GPU the library runs on holds its
+// the workgroup table, the step's counters, the keys, the sort's buffers and
+// the cell arrays.  Each GPU the library runs on holds its
 // own copy of the array until the process ends.  Host code never passes the
 // array's name to a kernel: the address each device holds it at comes from
 // hipGetSymbolAddress (na_scratch_base) and only that address is used.
@@ -2447,8 +2366,8 @@ constexpr long long kNaMaxCells = 1LL << 20;     // cells per call (nx^dim)
 constexpr int kNaMaxBlocks = kNaMaxN / 64;       // force workgroups (64 homes or more each)
 
 struct NaLayout {
-    size_t world, counters, blocks, work, keys0, kA, kB, vA, vB, skeys, count, start, end, hist,
-        bsum, bsq, total;
+    size_t world, counters, blocks, work, keys0, kA, perm, skeys, rec, count, start, end, bsum,
+        bsq, total;
 };
 
 constexpr size_t na_align(size_t o) { return (o + 255) & ~(size_t)255; }
@@ -2462,17 +2381,14 @@ constexpr NaLayout na_layout()
     L.blocks = o;   o = na_align(o + (size_t)kNaMaxBlocks * sizeof(uint2));
     L.work = o;     o = na_align(o + ((size_t)kNaMaxBlocks + 1) * sizeof(uint32_t));
     L.keys0 = o;    o = na_align(o + (size_t)kNaMaxN * 4);
-    L.kA = o;       o = na_align(o + (size_t)kNaMaxN * 4);
-    L.kB = o;       o = na_align(o + (size_t)kNaMaxN * 4);
-    L.vA = o;       o = na_align(o + (size_t)kNaMaxN * 4);
-    L.vB = o;       o = na_align(o + (size_t)kNaMaxN * 4);
+    L.kA = o;       o = na_align(o + (size_t)(kNaMaxN + kRankPad) * 4);
+    L.perm = o;     o = na_align(o + (size_t)kNaMaxN * 4);
     L.skeys = o;    o = na_align(o + (size_t)kNaMaxN * 4);
+    L.rec = o;      o = na_align(o + (size_t)kNaMaxN * 16);
     L.count = o;    o = na_align(o + (size_t)kNaMaxCells * 4);
     L.start = o;    o = na_align(o + (size_t)kNaMaxCells * 4);
     L.end = o;      o = na_align(o + (size_t)kNaMaxCells * 4);
-    // radix digit histograms: at most 2^8 digits per tile (passes of <= 8 bits)
-    L.hist = o;     o = na_align(o + (size_t)256 * ((kNaMaxN + kRadixTile - 1) / kRadixTile) * 4);
-    L.bsum = o;     o = na_align(o + (size_t)4096 * 4);
+    L.bsum = o;     o = na_align(o + (size_t)((kNaMaxCells + kScanTile - 1) / kScanTile) * 4);
     L.bsq = o;      o = na_align(o + (size_t)((kNaMaxCells + kScanTile - 1) / kScanTile) * 8);
     L.total = o;
     return L;
@@ -2569,7 +2485,6 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
     const double avg = (double)n / (double)nc;
     const ForcePlan fp = plan_force_for(s->dim, avg, false, false, plife_tuning{}, false, ntypes);
     const int nblocks = ceil_div(n, fp.bs);
-    const RadixPlan plan = radix_plan(nc, n);
 
     // a transient view of the scratch as the step helpers' buffers (no
     // allocation: plain pointers into the array)
@@ -2584,22 +2499,18 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
     t.d_blocks = reinterpret_cast<uint2 *>(base + kNa.blocks);
     t.keys0 = reinterpret_cast<uint32_t *>(base + kNa.keys0);
     t.kA = reinterpret_cast<uint32_t *>(base + kNa.kA);
-    t.kB = reinterpret_cast<uint32_t *>(base + kNa.kB);
-    t.vA = reinterpret_cast<uint32_t *>(base + kNa.vA);
-    t.vB = reinterpret_cast<uint32_t *>(base + kNa.vB);
+    t.perm = reinterpret_cast<uint32_t *>(base + kNa.perm);
+    t.rec = reinterpret_cast<uint4 *>(base + kNa.rec);
     t.skeys = reinterpret_cast<uint32_t *>(base + kNa.skeys);
     t.cell_count = reinterpret_cast<uint32_t *>(base + kNa.count);
     t.cell_start = reinterpret_cast<uint32_t *>(base + kNa.start);
     t.cell_end = reinterpret_cast<uint32_t *>(base + kNa.end);
-    t.hist = reinterpret_cast<uint32_t *>(base + kNa.hist);
     t.bsum = reinterpret_cast<uint32_t *>(base + kNa.bsum);
     t.bsum_cap = (kNa.bsq - kNa.bsum) / 4;
     t.bsq = reinterpret_cast<unsigned long long *>(base + kNa.bsq);
     t.bsq_cap = (kNa.total - kNa.bsq) / 8;
     uint32_t *work = reinterpret_cast<uint32_t *>(base + kNa.work);
-    if ((size_t)ceil_div(nc, kScanTile) + (size_t)ceil_div((long long)plan.hist_len, kScanTile) >
-            t.bsum_cap ||
-        plan.hist_len > (kNa.bsum - kNa.hist) / 4 || nblocks > kNaMaxBlocks)
+    if (nblocks > kNaMaxBlocks)
         return fail(PLIFE_ERR_STATE, "scratch layout too small for this world");
 
     const int setup_threads = std::max(nblocks + 1, 8);
@@ -2607,40 +2518,17 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
         wd, t.d_worlds, t.d_blocks, nblocks, fp.bs, t.d_pairs, work, t.cell_count, nc);
     LAUNCH_CHECK();
     if (n > 0) {
-        // 1. cell keys, histogram and first digit histogram; counters [0, 3)
-        //    cleared, tag in [3] (Physics.java:319-340)
-#define PLIFE_NA_BIN(DD)                                                                          \
-    do {                                                                                          \
-        if (d3) k_bin_tile<3, DD><<<plan.ntiles, 1024, 0, stream>>>(px, py, pz, n, t.d_worlds,   \
-                nullptr, plan.ntiles, t.keys0, t.cell_count, t.hist, t.d_pairs, 3, 1ull, nullptr); \
-        else k_bin_tile<2, DD><<<plan.ntiles, 1024, 0, stream>>>(px, py, pz, n, t.d_worlds,      \
-                nullptr, plan.ntiles, t.keys0, t.cell_count, t.hist, t.d_pairs, 3, 1ull, nullptr); \
-    } while (0)
-        switch (plan.D) {
-            case 1: PLIFE_NA_BIN(1); break;
-            case 2: PLIFE_NA_BIN(2); break;
-            case 3: PLIFE_NA_BIN(3); break;
-            case 4: PLIFE_NA_BIN(4); break;
-            case 5: PLIFE_NA_BIN(5); break;
-            case 6: PLIFE_NA_BIN(6); break;
-            case 7: PLIFE_NA_BIN(7); break;
-            default: PLIFE_NA_BIN(8); break;
-        }
-#undef PLIFE_NA_BIN
-        LAUNCH_CHECK();
-        // cell scan (clears the counts) and first digit scan
-        if ((rc = scan_jobs(&t, ScanJob{t.cell_count, nc, t.cell_start, t.cell_end, 1, nullptr,
-                                        t.d_pairs + 1},
-                            ScanJob{t.hist, (int)plan.hist_len, t.hist, nullptr, 0, nullptr, nullptr})))
-            return rc;
-        // 2. the stable sort: the reference's counting-sort permutation
-        if ((rc = radix_sort(&t, n, plan))) return rc;
+        // 1. cell keys and histogram; counters [0, 3) cleared, tag in [3]
+        //    (Physics.java:319-340); cell scan (clears the counts)
+        const PosBuf P{const_cast<uint32_t *>(px), const_cast<uint32_t *>(py), const_cast<uint32_t *>(pz)};
+        if ((rc = bin_cells(&t, s->dim, P, n, nullptr, 3, 1ull, nullptr))) return rc;
+        if ((rc = scan_cells(&t, nc, t.d_pairs + 1))) return rc;
+        // 2. the stable counting sort
+        if ((rc = sort_cells(&t, s->dim, P, type, n))) return rc;
         // 3. force + integrate into the caller's output arrays
         ForceArgs a{};
+        a.rec = t.rec;
         a.perm = t.perm;
-        a.sx = px;
-        a.sy = py;
-        a.sz = pz;
         a.vx = vx;
         a.vy = vy;
         a.vz = vz;

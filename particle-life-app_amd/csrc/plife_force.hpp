@@ -30,9 +30,10 @@
 namespace plife {
 
 struct ForceArgs {
+    const uint4 *rec;                // x, y, z, type of each sorted slot (multi-launch path)
     // step-start state in the pre-sort order, read through the permutation
     const uint32_t *perm;            // sorted slot -> pre-sort index
-    const uint32_t *sx, *sy, *sz;
+    const uint32_t *sx, *sy, *sz;    // (one-launch step)
     const float *vx, *vy, *vz;
     const int32_t *type, *id;
     // the new state, written in the sorted order (Physics.particles after the swap)
@@ -291,8 +292,8 @@ __device__ __forceinline__ void visit_run(const ForceArgs &a, const WorldDev &w,
 {
     for (int j = lo; j < hi; ++j) {
         if (j == g) continue;
-        const uint32_t jo = a.perm[j];
-        const uint32_t qx = a.sx[jo], qy = a.sy[jo], qz = DIM == 3 ? a.sz[jo] : 0u;
+        const uint4 q = a.rec[j];
+        const uint32_t qx = q.x, qy = q.y, qz = DIM == 3 ? q.z : 0u;
         const int dxi = (int)(qx - hx), dyi = (int)(qy - hy);
         const int dzi = DIM == 3 ? (int)(qz - hz) : 0;
         if (!WRAP) {
@@ -301,9 +302,9 @@ __device__ __forceinline__ void visit_run(const ForceArgs &a, const WorldDev &w,
             if (DIM == 3) ok &= ((dzi >= 0) == (qz >= hz));
             if (!ok) continue;
         }
-        const int idx = row + a.type[jo];
+        const int idx = row + (int)q.w;
         const double m = MLDS ? Mlds[idx] : a.matrix[w.moff + idx] * w.R;
-        pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m, DEBUG ? (uint32_t)a.id[jo] : 0u, w);
+        pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m, DEBUG ? (uint32_t)a.id[a.perm[j]] : 0u, w);
     }
 }
 
@@ -365,37 +366,46 @@ __device__ void home_global(const ForceArgs &a, const WorldDev &w, const double 
 constexpr int kMaxParts = 4;
 constexpr int kScreenPad = 32;   // candidates a screen step reads from one base
 
-// Starts (gs) of the NC staged cells and their exclusive prefix (off, NC + 1
-// entries) for a workgroup of T threads; returns the staged particle count,
-// the same in every thread.  Ends with a barrier.
+// A staged row's columns are consecutive cells, one run of the sorted order,
+// except where they wrap around the box in x: up to three runs (segments).
+constexpr int kMaxSegs = kMaxParts * 3;      // per stencil row
+
+// Exclusive prefix of the NC staged cells' counts (off, NC + 1 entries) for a
+// workgroup of T threads, and the segment table: entry k of segs holds the
+// first staged entry of segment k and the sorted slot minus the staged entry
+// of its particles.  An unused segment starts where the next one does.
+// Returns the staged particle count, the same in every thread.  Ends with a
+// barrier.
 template <int DIM, int T>
 __device__ __forceinline__ uint32_t stage_cells(const ForceArgs &a, const int (&p_base)[kMaxParts + 1],
                                                 const int (&p_w)[kMaxParts], const int (&p_row)[kMaxParts],
                                                 const int (&p_ca)[kMaxParts], int nx, uint32_t cb,
-                                                uint32_t *off, uint32_t *gs, uint32_t *s_cnt)
+                                                uint32_t *off, uint2 *segs, uint32_t *s_cnt)
 {
-    constexpr int NW = T / kWave;
+    constexpr int NW = T / kWave, NR = DIM == 3 ? 9 : 3;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
     const int NC = p_base[kMaxParts];
     uint32_t carry = 0;
     for (int f0 = 0; f0 < NC; f0 += T) {
         const int f = f0 + tid;
-        uint32_t c = 0;
+        uint32_t c = 0, s0 = 0;
+        int seg = 0, j = 0, pw = p_w[0], pc = p_ca[0];
         if (f < NC) {
-            int pb = p_base[0], pw = p_w[0], pr = p_row[0], pc = p_ca[0];
+            int pb = p_base[0], pr = p_row[0], part = 0;
 #pragma unroll
             for (int q = 1; q < kMaxParts; ++q)
-                if (f >= p_base[q] && p_w[q] > 0) { pb = p_base[q]; pw = p_w[q]; pr = p_row[q]; pc = p_ca[q]; }
-            const int r = (f - pb) / pw, j = (f - pb) - r * pw;
+                if (f >= p_base[q] && p_w[q] > 0) { pb = p_base[q]; pw = p_w[q]; pr = p_row[q]; pc = p_ca[q]; part = q; }
+            const int r = (f - pb) / pw;
+            j = (f - pb) - r * pw;
             const int oy = (r % 3) - 1, oz = DIM == 3 ? (r / 3) - 1 : 0;
             const int cy = pr % nx, cz = DIM == 3 ? pr / nx : 0;
             const int x = wrap_cell(pc - 1 + j, nx);
             const int y = wrap_cell(cy + oy, nx);
             const int z = DIM == 3 ? wrap_cell(cz + oz, nx) : 0;
             const uint32_t ci = cb + (uint32_t)(x + y * nx + z * nx * nx);
-            const uint32_t s0 = a.cell_start[ci];
+            s0 = a.cell_start[ci];
             c = a.cell_end[ci] - s0;
-            gs[f] = s0;
+            seg = (part * NR + r) * 3;
         }
         const uint32_t inc = wave_incl_scan(c);
         if (lane == kWave - 1) s_cnt[wv] = inc;
@@ -406,7 +416,20 @@ __device__ __forceinline__ uint32_t stage_cells(const ForceArgs &a, const int (&
             wbase0 += v < wv ? s_cnt[v] : 0u;
             tot += s_cnt[v];
         }
-        if (f < NC) off[f] = wbase0 + inc - c;
+        if (f < NC) {
+            const uint32_t o = wbase0 + inc - c;
+            const uint2 here = make_uint2(o, s0 - o);
+            off[f] = o;
+            // column 0 (wrapped or not), column 1 (a run of its own only after a
+            // wrapped column 0), the last column (only when it wraps)
+            const bool lw = pc == 0, rw = pc - 1 + pw - 1 == nx;
+            if (j == 0) {
+                segs[seg] = here;
+                if (!lw) segs[seg + 1] = here;
+            }
+            if (j == 1 && lw) segs[seg + 1] = here;
+            if (j == pw - 1) segs[seg + 2] = rw ? here : make_uint2(o + c, 0u);
+        }
         carry += tot;
         __syncthreads();
     }
@@ -423,25 +446,26 @@ struct Staged {
     uint8_t *type;
 };
 
-// Stages entries [w0, w0 + wn) of the neighbourhood (NC cells) with T threads.
+// Stages entries [w0, w0 + wn) of the neighbourhood (nsegs segments) with T
+// threads: one 16-byte record read per entry.
 template <int DIM, bool DEBUG, int T>
-__device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s, const uint32_t *off,
-                                             const uint32_t *gs, int NC, int w0, int wn)
+__device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s, const uint2 *segs, int nsegs,
+                                             int w0, int wn)
 {
     for (int t = threadIdx.x; t < wn; t += T) {
-        const int sg = w0 + t;
-        int lo = 0, hi = NC;           // off[lo] <= sg < off[hi]
+        const uint32_t sg = (uint32_t)(w0 + t);
+        int lo = 0, hi = nsegs;        // the last segment that starts at or before sg
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
-            if (off[mid] <= (uint32_t)sg) lo = mid;
+            if (segs[mid].x <= sg) lo = mid;
             else hi = mid;
         }
-        const uint32_t q = a.perm[gs[lo] + ((uint32_t)sg - off[lo])];
-        const uint32_t qx = a.sx[q], qy = a.sy[q];
-        s.xy[t] = make_uint2(high_halves(qx, qy), low_halves(qx, qy));
-        if constexpr (DIM == 3) s.z[t] = a.sz[q];
-        if constexpr (DEBUG) s.id[t] = (uint32_t)a.id[q];
-        s.type[t] = (uint8_t)a.type[q];
+        const uint32_t slot = sg + segs[lo].y;
+        const uint4 q = a.rec[slot];
+        s.xy[t] = make_uint2(high_halves(q.x, q.y), low_halves(q.x, q.y));
+        if constexpr (DIM == 3) s.z[t] = q.z;
+        if constexpr (DEBUG) s.id[t] = (uint32_t)a.id[a.perm[slot]];
+        s.type[t] = (uint8_t)q.w;
     }
 }
 
@@ -555,7 +579,7 @@ __device__ __forceinline__ void deal_homes(const int (&count)[HPT], int shift, u
 // The LDS of a staged workgroup: `cap` staged entries at most; the windowed
 // path streams a denser neighbourhood through it.
 struct ForceLds {
-    size_t m, sxy, words, wbase, ax, ay, az, dhash, hxy, hz, dcnt, words2, wbase2, ht, sz, sid, off, gs, st, total;
+    size_t m, sxy, words, wbase, ax, ay, az, dhash, hxy, hz, dcnt, words2, wbase2, ht, sz, sid, off, st, total;
 };
 
 // Bytes per home that several windows keep in LDS besides the mask words: the
@@ -592,7 +616,6 @@ __host__ __device__ inline ForceLds force_lds_layout(int dim, bool debug, int nt
     L.sz = o;    o += dim == 3 ? (size_t)(cap + kScreenPad) * 4 : 0;
     L.sid = o;   o += debug ? (size_t)cap * 4 : 0;
     L.off = o;   o += (size_t)(max_cells + 1) * 4;
-    L.gs = o;    o += (size_t)max_cells * 4;
     L.st = o;    o += (size_t)cap;
     L.total = (o + 15) & ~(size_t)15;
     return L;
@@ -622,6 +645,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     // per home: its staged index, kept candidates and first mask word
     __shared__ uint16_t s_si[BS], s_hc[BS], s_wo[BS];
     __shared__ uint32_t s_bin[256];
+    __shared__ uint2 s_seg[kMaxSegs * NR];
 
     const ForceLds L = force_lds_layout(DIM, DEBUG, a.ntypes_max, MLDS, a.cap, BS, a.max_cells,
                                         a.wpool, a.wpool2);
@@ -630,7 +654,6 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     uint32_t *szz = reinterpret_cast<uint32_t *>(smem + L.sz);
     uint32_t *sid = reinterpret_cast<uint32_t *>(smem + L.sid);
     uint32_t *off = reinterpret_cast<uint32_t *>(smem + L.off);
-    uint32_t *gs = reinterpret_cast<uint32_t *>(smem + L.gs);
     uint8_t *st = reinterpret_cast<uint8_t *>(smem + L.st);
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
@@ -652,8 +675,9 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     const bool active = tid < nact;
     const int g = g0 + (active ? tid : nact - 1);
     const uint32_t ho = a.perm[g];
-    const uint32_t hx = a.sx[ho], hy = a.sy[ho], hz = DIM == 3 ? a.sz[ho] : 0u;
-    const int htype = a.type[ho];
+    const uint4 hr = a.rec[g];
+    const uint32_t hx = hr.x, hy = hr.y, hz = DIM == 3 ? hr.z : 0u;
+    const int htype = (int)hr.w;
     const uint32_t hkey = a.skeys[g] - cb;
     const int hrow = (int)(hkey / (uint32_t)nx);
     const int hcx = (int)(hkey - (uint32_t)hrow * (uint32_t)nx);
@@ -697,7 +721,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     const bool use_lds = !w.all_global && a.cap > 0 && nparts <= (uint32_t)kMaxParts && NC <= a.max_cells;
 
     uint32_t carry = 0;
-    if (use_lds) carry = stage_cells<DIM, BS>(a, p_base, p_w, p_row, p_ca, nx, cb, off, gs, s_cnt);
+    if (use_lds) carry = stage_cells<DIM, BS>(a, p_base, p_w, p_row, p_ca, nx, cb, off, s_seg, s_cnt);
     else __syncthreads();
 
     const int mrow = htype * w.ntypes;
@@ -787,18 +811,18 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             return npass;
         };
 
-        const int S = (int)carry;
+        const int S = (int)carry, nsegs = (int)nparts * NR * 3;
         if (a.wpool > 0 && S <= a.cap && place_words(0, S) <= (uint32_t)a.wpool) {
             // ---- one window ----------------------------------------------
             uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words);
             uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase);
-            stage_window<DIM, DEBUG, BS>(a, stg, off, gs, NC, 0, S);
+            stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, 0, S);
             __syncthreads();
             const int count[1] = {screen_home(0, S, wmask, wbase)};
             int si = 0;
             if (active) {
                 const int f = pb + RMID * pw + jh;
-                si = (int)off[f] + (g - (int)gs[f]);
+                si = (int)off[f] + (g - (int)a.cell_start[cb + hkey]);
             }
             s_si[tid] = (uint16_t)si;
             s_hc[tid] = (uint16_t)count[0];
@@ -861,7 +885,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 // one entry needs a word per home at most, and wpool2 >= BS
                 int wn = min(a.cap, S - w0);
                 while (place_words(w0, wn) > (uint32_t)a.wpool2) wn = (wn + 1) >> 1;
-                stage_window<DIM, DEBUG, BS>(a, stg, off, gs, NC, w0, wn);
+                stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, w0, wn);
                 __syncthreads();
                 const int count[1] = {screen_home(w0, wn, wmask, wbase)};
                 s_hc[tid] = (uint16_t)count[0];
@@ -963,8 +987,9 @@ __global__ __launch_bounds__(kSparseBlock) void k_force_sparse(ForceArgs a)
     acc.hash = 0ull;
     if (active) {
         const uint32_t ho = a.perm[g];
-        const uint32_t hx = a.sx[ho], hy = a.sy[ho], hz = DIM == 3 ? a.sz[ho] : 0u;
-        const int htype = a.type[ho];
+        const uint4 hr = a.rec[g];
+        const uint32_t hx = hr.x, hy = hr.y, hz = DIM == 3 ? hr.z : 0u;
+        const int htype = (int)hr.w;
         home_global<DIM, WRAP, DEBUG, MLDS>(a, w, M, g, hx, hy, hz, htype * w.ntypes, acc);
         finish_home<DIM, WRAP, DEBUG>(a, w, acc, hx, hy, hz, htype, ho, g);
     }

@@ -1,12 +1,13 @@
 // plife_kernels.hpp -- gfx950 kernels of the particle-life physics step.
 //
 // One step (reference: backend/Physics.java:112-134):
-//   k_bin_tile               cell key per particle (Physics.java:362-375), cell histogram,
-//                            first radix-digit histogram
-//   k_scan2_*                exclusive/inclusive scans -> cell_start / cell_end
+//   k_bin                    cell key per particle (Physics.java:362-375), cell histogram, and
+//                            each particle's place among its cell's arrivals
+//   k_scan_*                 scan of the cell counts -> cell_start / cell_end
 //                            (cell_end is the reference's `containers` array, Physics.java:329-348)
-//   k_radix_hist/_scatter    stable LSD radix sort of (key, index): the reference's
-//                            stable counting-sort permutation (Physics.java:342-353)
+//   k_place, k_rank          the reference's stable counting-sort permutation
+//                            (Physics.java:342-353): particles placed in their cell in
+//                            arrival order, then ranked by index inside it
 //   k_force (plife_force.hpp) velocity phase + position phase fused (Physics.java:397-450);
 //                            legal because the update is Jacobi: velocities read only the
 //                            sorted step-start positions, new positions go to another buffer.
@@ -24,9 +25,6 @@ namespace plife {
 
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
-constexpr int kRadixTile = 2048;                 // elements per radix tile
-constexpr int kScatterBlock = 512;               // threads of the radix scatter
-constexpr int kRadixItems = kRadixTile / kScatterBlock;
 constexpr double kFix = 4294967296.0;       // 2^32
 constexpr double kInvFix = 1.0 / 4294967296.0;
 
@@ -136,7 +134,7 @@ struct WorldDev {
     int wrap;
     float r2hi;                      // screen bound, units 2^-64: (rmax 2^32)^2 (1 + 2^-20)
     int sbias;                       // screen bound on 16-bit coordinates: -(bq + 1) (screen_hi)
-    double cs;                       // cell size = rmax (Physics.java:312)
+    double cs, ics;                  // cell size = rmax (Physics.java:312), and 1 / cs
     double r2u;                      // fl(rmax*rmax) * 2^64: the reference's bound in units 2^-64
     double S;                        // 2^-32 / rmax: |rel| = |D| S with D in units 2^-32
     double R;                        // rmax * 2^32:  1/|rel| = R / |D|
@@ -166,14 +164,8 @@ __global__ void k_world_of(int n, const WorldDev *__restrict__ worlds, int nworl
     world_of[i] = (uint16_t)lo;
 }
 
-__device__ __forceinline__ int key_axis(uint32_t k, double cs, int nx)
-{
-    const double x = (double)k * kInvFix;   // exact
-    int c = (int)(x / cs);                   // IEEE FP64 division, x >= 0: trunc == floor
-    return c == nx ? nx - 1 : c;
-}
-
-// trunc(x / cs) for x = k 2^-32 without the division where that is safe:
+// trunc(x / cs) (IEEE FP64 division, x >= 0: trunc == floor) for x = k 2^-32
+// without the division where that is safe:
 // x * (1 / cs) is within 3 ulp of the rounded quotient, i.e. within 2^-35
 // for quotients below 2^16 cells, so its integer part is the division's
 // unless the product lies within 1e-9 of an integer -- then divide.
@@ -196,80 +188,123 @@ __device__ __forceinline__ int key_axis_fast(uint32_t k, double cs, double ics, 
 // Cell counts are accumulated with one atomic per run of equal keys inside a
 // wave: the input is the previous step's cell order, so most lanes of a wave
 // share a few keys and per-lane atomics would serialise on the same address.
-__device__ __forceinline__ void count_runs(uint32_t key, bool valid, uint32_t *__restrict__ cell_count)
+// Returns the lane's place among the cell's arrivals: what the run's atomic
+// found plus the lane's position in the run.
+__device__ __forceinline__ uint32_t count_runs(uint32_t key, bool valid, uint32_t *__restrict__ cell_count)
 {
     const int lane = __lane_id();
     const uint32_t prev = __shfl_up(key, 1, kWave);
     const bool head = valid && (lane == 0 || prev != key);
     const uint64_t heads = __ballot(head);
     const int nvalid = (int)__popcll(__ballot(valid));   // valid lanes are a prefix
+    uint32_t base = 0;
     if (head) {
         const uint64_t later = lane == 63 ? 0ull : (heads & (~0ull << (lane + 1)));
         const int next = later ? (int)__ffsll((long long)later) - 1 : nvalid;
-        atomicAdd(&cell_count[key], (uint32_t)(next - lane));
+        base = atomicAdd(&cell_count[key], (uint32_t)(next - lane));
     }
+    const uint64_t upto = heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
+    const int first = upto ? 63 - (int)__clzll((long long)upto) : 0;
+    return __shfl(base, first, kWave) + (uint32_t)(lane - first);
 }
 
-// Fused binning of one radix tile (kRadixTile elements in the radix kernels'
-// element order): cell keys, the cell histogram (run-aggregated atomics) and
-// this tile's histogram of the first radix digit.  Block 0 also clears the
-// pair counter of the step.
-template <int DIM, int D>
-__global__ __launch_bounds__(1024) void k_bin_tile(const uint32_t *__restrict__ px,
-                                                  const uint32_t *__restrict__ py,
-                                                  const uint32_t *__restrict__ pz, int n,
-                                                  const WorldDev *__restrict__ worlds,
-                                                  const uint16_t *__restrict__ world_of,
-                                                  int ntiles,
-                                                  uint32_t *__restrict__ keys,
-                                                  uint32_t *__restrict__ cell_count,
-                                                  uint32_t *__restrict__ hist,
-                                                  unsigned long long *__restrict__ counters,
-                                                  int ncounters, unsigned long long tag,
-                                                  unsigned long long *__restrict__ stat_out)
+// Binning: cell keys, the cell histogram (run-aggregated atomics) and each
+// particle's place among its cell's arrivals.  Block 0 also clears the step's
+// counters.
+constexpr int kBinItems = 1;
+
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_bin(const uint32_t *__restrict__ px, const uint32_t *__restrict__ py,
+                                                const uint32_t *__restrict__ pz, int n,
+                                                const WorldDev *__restrict__ worlds,
+                                                const uint16_t *__restrict__ world_of,
+                                                uint32_t *__restrict__ keys, uint32_t *__restrict__ arrival,
+                                                uint32_t *__restrict__ cell_count,
+                                                unsigned long long *__restrict__ counters, int ncounters,
+                                                unsigned long long tag, unsigned long long *__restrict__ stat_out)
 {
-    constexpr int R = 1 << D;
-    __shared__ uint32_t h[R];
-    for (int t = threadIdx.x; t < R; t += 1024) h[t] = 0;
     // the step's counters (pairs, sum of squares, per-world pairs) start at
     // zero, after the previous step's final values (and its layout tag) have
     // gone to the host's pinned copy (stat_out, when given)
     if (blockIdx.x == 0) {
-        for (int t = threadIdx.x; t <= ncounters; t += 1024) {
+        for (int t = threadIdx.x; t <= ncounters; t += kBlock) {
             if (stat_out) stat_out[t] = counters[t];
             counters[t] = t < ncounters ? 0ull : tag;   // [ncounters]: which layout the counts belong to
         }
     }
-    const double cs0 = worlds[0].cs;
-    const int nx0 = worlds[0].nx;
-    const uint32_t base0 = worlds[0].cell_base;
-    __syncthreads();
-    const int base = blockIdx.x * kRadixTile;
+    double cs = worlds[0].cs, ics = worlds[0].ics;
+    int nx = worlds[0].nx;
+    uint32_t cb = worlds[0].cell_base;
 #pragma unroll
-    for (int r = 0; r < kRadixTile / 1024; ++r) {
-        const int i = base + r * 1024 + threadIdx.x;
+    for (int r = 0; r < kBinItems; ++r) {
+        const int i = (blockIdx.x * kBinItems + r) * kBlock + threadIdx.x;
         const bool valid = i < n;
         uint32_t key = 0xFFFFFFFFu;
         if (valid) {
-            double cs = cs0;
-            int nx = nx0;
-            uint32_t cb = base0;
             if (world_of) {                            // several worlds: this slot's world
                 const WorldDev *w = worlds + world_of[i];
                 cs = w->cs;
+                ics = w->ics;
                 nx = w->nx;
                 cb = w->cell_base;
             }
-            key = (uint32_t)key_axis(px[i], cs, nx) + (uint32_t)key_axis(py[i], cs, nx) * (uint32_t)nx;
-            if constexpr (DIM == 3) key += (uint32_t)key_axis(pz[i], cs, nx) * (uint32_t)nx * (uint32_t)nx;
+            key = (uint32_t)key_axis_fast(px[i], cs, ics, nx) + (uint32_t)key_axis_fast(py[i], cs, ics, nx) * (uint32_t)nx;
+            if constexpr (DIM == 3) key += (uint32_t)key_axis_fast(pz[i], cs, ics, nx) * (uint32_t)nx * (uint32_t)nx;
             key += cb;
             keys[i] = key;
-            atomicAdd(&h[key & (R - 1)], 1u);
         }
-        count_runs(key, valid, cell_count);
+        const uint32_t at = count_runs(key, valid, cell_count);
+        if (valid) arrival[i] = at;
     }
-    __syncthreads();
-    for (int t = threadIdx.x; t < R; t += 1024) hist[t * ntiles + blockIdx.x] = h[t];
+}
+
+// Particle i to its cell's slots in arrival order.
+__global__ __launch_bounds__(kBlock) void k_place(int n, const uint32_t *__restrict__ keys,
+                                                  const uint32_t *__restrict__ arrival,
+                                                  const uint32_t *__restrict__ cell_start,
+                                                  uint32_t *__restrict__ order)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) order[cell_start[keys[i]] + arrival[i]] = (uint32_t)i;
+}
+
+// Stable order: each particle's rank among its cell's by index gives its
+// sorted slot, which gets the permutation, the key and the particle's record
+// (x, y, z, type), so that the force kernels read neighbours as contiguous
+// 16-byte entries.  The comparisons are the sum of count^2 over cells; the
+// force phase evaluates at least as many candidates at several times the cost
+// each, so that dense cells need no other sort.  Bound by the latency of its
+// dependent reads: threads go by pre-sort slot (coalesced keys and state, and
+// a wave's lanes share a few cells), and a cell is read sixteen indices at a
+// time, past its end too (`order` has kRankPad spare entries).
+constexpr int kRankPad = 16;
+
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_rank(int n, const uint32_t *__restrict__ keys,
+                                                 const uint32_t *__restrict__ order,
+                                                 const uint32_t *__restrict__ cell_start,
+                                                 const uint32_t *__restrict__ cell_end,
+                                                 const uint32_t *__restrict__ px, const uint32_t *__restrict__ py,
+                                                 const uint32_t *__restrict__ pz, const int32_t *__restrict__ type,
+                                                 uint32_t *__restrict__ perm, uint32_t *__restrict__ skeys,
+                                                 uint4 *__restrict__ rec)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (uint32_t)n) return;
+    const uint32_t key = keys[i];
+    const uint32_t s = cell_start[key], e = cell_end[key];
+    const uint4 p = make_uint4(px[i], py[i], DIM == 3 ? pz[i] : 0u, (uint32_t)type[i]);
+    uint32_t r = s;
+    for (uint32_t k = s; k < e; k += 16) {
+        uint32_t v[16];
+        __builtin_memcpy(v, order + k, sizeof v);
+        const int m = (int)min(e - k, 16u);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) r += ((v[u] < i) & (u < m)) ? 1u : 0u;
+    }
+    perm[r] = i;
+    skeys[r] = key;
+    rec[r] = p;
 }
 
 // ---------------------------------------------------------------------------
@@ -278,63 +313,67 @@ __global__ __launch_bounds__(1024) void k_bin_tile(const uint32_t *__restrict__ 
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kBlock * kScanItems;
 
-// Two independent device-wide scans in the same three launches: blocks
-// [0, nb0) scan job 0, blocks [nb0, nb0 + nb1) scan job 1.  excl may alias in;
-// with zero_in (requires in != excl) the input is cleared once read, which
-// leaves the cell counters ready for the next step's histogram.  With sq,
-// the sum of squared inputs is added to *sq (for cell counts: the number of
-// (particle, cell-mate) pairs, a clustering measure): the reduce pass stores
-// each block's sum in sqb and the block-sum scan adds them up, so the
-// device-wide total costs one atomic rather than one per block.
+// Exclusive scan of n cell counts into excl and inclusive into incl; the
+// counts are cleared once read, which leaves them ready for the next step's
+// histogram.  The sum of their squares (the number of (particle, cell-mate)
+// pairs, a clustering measure) is added to *sq: the reduce pass stores each
+// block's sum in sqb and one block adds them up, so the device-wide total
+// costs one atomic rather than one per block.
 struct ScanJob {
     uint32_t *in;
     int n;
-    uint32_t *excl;
-    uint32_t *incl;   // may be null
-    int zero_in;
-    uint32_t *bsum;   // ceil(n / kScanTile) block sums
-    unsigned long long *sq;   // may be null
-    unsigned long long *sqb;  // ceil(n / kScanTile) per-block sums of squares (with sq)
+    uint32_t *excl, *incl;
+    unsigned long long *sq;
+    uint32_t *bsum;           // ceil(n / kScanTile) block sums
+    unsigned long long *sqb;  // ceil(n / kScanTile) per-block sums of squares
 };
 
-__device__ __forceinline__ void scan_job_of(const ScanJob &j0, const ScanJob &j1, int nb0, int b,
-                                            ScanJob &j, int &blk)
+__device__ __forceinline__ void scan_load(const ScanJob &j, int i0, uint32_t (&v)[kScanItems], uint32_t &s)
 {
-    if (b < nb0) { j = j0; blk = b; }
-    else { j = j1; blk = b - nb0; }
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan2_reduce(ScanJob j0, ScanJob j1, int nb0)
-{
-    __shared__ uint32_t s_w[4];
-    __shared__ unsigned long long s_q[kBlock / kWave];
-    ScanJob j;
-    int blk;
-    scan_job_of(j0, j1, nb0, blockIdx.x, j, blk);
-    const int base = blk * kScanTile + threadIdx.x * kScanItems;
-    uint32_t s = 0;
-    unsigned long long q = 0;
+    s = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k)
-        if (base + k < j.n) {
-            const uint32_t v = j.in[base + k];
-            s += v;
-            q += (unsigned long long)v * v;
-        }
-    uint32_t total;
-    block_excl_scan(s, s_w, total);
-    if (threadIdx.x == 0) j.bsum[blk] = total;
-    if (j.sq) {                                    // uniform per block
-        q = block_sum_u64(q, s_q);
-        if (threadIdx.x == 0) j.sqb[blk] = q;
+    for (int k = 0; k < kScanItems; ++k) {
+        v[k] = (i0 + k < j.n) ? j.in[i0 + k] : 0u;
+        s += v[k];
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan2_single(ScanJob j0, ScanJob j1)
+__device__ __forceinline__ void scan_store(const ScanJob &j, int i0, const uint32_t (&v)[kScanItems], uint32_t off)
+{
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (i0 + k < j.n) {
+            j.in[i0 + k] = 0u;
+            j.excl[i0 + k] = off;
+            off += v[k];
+            j.incl[i0 + k] = off;
+        }
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_scan_reduce(ScanJob j)
 {
     __shared__ uint32_t s_w[4];
     __shared__ unsigned long long s_q[kBlock / kWave];
-    const ScanJob j = blockIdx.x == 0 ? j0 : j1;
+    uint32_t v[kScanItems], s;
+    scan_load(j, blockIdx.x * kScanTile + threadIdx.x * kScanItems, v, s);
+    unsigned long long q = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) q += (unsigned long long)v[k] * v[k];
+    uint32_t total;
+    block_excl_scan(s, s_w, total);
+    q = block_sum_u64(q, s_q);
+    if (threadIdx.x == 0) {
+        j.bsum[blockIdx.x] = total;
+        j.sqb[blockIdx.x] = q;
+    }
+}
+
+// The block sums of jobs of more than kFoldBlocks blocks.
+__global__ __launch_bounds__(kBlock) void k_scan_single(ScanJob j)
+{
+    __shared__ uint32_t s_w[4];
+    __shared__ unsigned long long s_q[kBlock / kWave];
     const int n = (j.n + kScanTile - 1) / kScanTile;
     uint32_t carry = 0;
     unsigned long long q = 0;
@@ -346,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_scan2_single(ScanJob j0, ScanJob j1)
         for (int k = 0; k < kScanItems; ++k) {
             v[k] = (i0 + k < n) ? j.bsum[i0 + k] : 0u;
             s += v[k];
-            if (j.sq && i0 + k < n) q += j.sqb[i0 + k];
+            if (i0 + k < n) q += j.sqb[i0 + k];
         }
         uint32_t total;
         uint32_t off = block_excl_scan(s, s_w, total) + carry;
@@ -357,76 +396,41 @@ __global__ __launch_bounds__(kBlock) void k_scan2_single(ScanJob j0, ScanJob j1)
         }
         carry += total;
     }
-    if (j.sq) {                                    // uniform per block
-        q = block_sum_u64(q, s_q);
-        if (threadIdx.x == 0 && q) atomicAdd(j.sq, q);
-    }
+    q = block_sum_u64(q, s_q);
+    if (threadIdx.x == 0 && q) atomicAdd(j.sq, q);
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan2_down(ScanJob j0, ScanJob j1, int nb0)
+__global__ __launch_bounds__(kBlock) void k_scan_down(ScanJob j)
 {
     __shared__ uint32_t s_w[4];
-    ScanJob j;
-    int blk;
-    scan_job_of(j0, j1, nb0, blockIdx.x, j, blk);
-    const int i0 = blk * kScanTile + threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
-    uint32_t s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        v[k] = (i0 + k < j.n) ? j.in[i0 + k] : 0u;
-        s += v[k];
-    }
-    uint32_t total;
-    uint32_t off = block_excl_scan(s, s_w, total) + j.bsum[blk];
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        if (i0 + k < j.n) {
-            if (j.zero_in) j.in[i0 + k] = 0u;
-            j.excl[i0 + k] = off;
-            off += v[k];
-            if (j.incl) j.incl[i0 + k] = off;
-        }
-    }
+    const int i0 = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+    uint32_t v[kScanItems], s, total;
+    scan_load(j, i0, v, s);
+    const uint32_t off = block_excl_scan(s, s_w, total) + j.bsum[blockIdx.x];
+    scan_store(j, i0, v, off);
 }
 
 // Down-sweep for jobs of at most kFoldBlocks blocks, with the block-sum scan
 // folded in: each block adds up the sums of the blocks before it (at most
-// kFoldBlocks / kBlock loads per thread), and block 0 adds the job's sum of
+// kFoldBlocks / kBlock loads per thread), and block 0 adds the sum of
 // squares -- two launches instead of three, same outputs.
 constexpr int kFoldBlocks = 1024;
 
-__global__ __launch_bounds__(kBlock) void k_scan2_down_fold(ScanJob j0, ScanJob j1, int nb0)
+__global__ __launch_bounds__(kBlock) void k_scan_down_fold(ScanJob j)
 {
     __shared__ uint32_t s_w[4];
     __shared__ unsigned long long s_q[kBlock / kWave];
-    ScanJob j;
-    int blk;
-    scan_job_of(j0, j1, nb0, blockIdx.x, j, blk);
+    const int blk = blockIdx.x;
     uint32_t pre = 0;
     for (int b = threadIdx.x; b < blk; b += kBlock) pre += j.bsum[b];
     uint32_t before;
     block_excl_scan(pre, s_w, before);             // `before` = the sum over all threads
     const int i0 = blk * kScanTile + threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
-    uint32_t s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        v[k] = (i0 + k < j.n) ? j.in[i0 + k] : 0u;
-        s += v[k];
-    }
-    uint32_t total;
-    uint32_t off = block_excl_scan(s, s_w, total) + before;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        if (i0 + k < j.n) {
-            if (j.zero_in) j.in[i0 + k] = 0u;
-            j.excl[i0 + k] = off;
-            off += v[k];
-            if (j.incl) j.incl[i0 + k] = off;
-        }
-    }
-    if (j.sq && blk == 0) {                        // uniform per block
+    uint32_t v[kScanItems], s, total;
+    scan_load(j, i0, v, s);
+    const uint32_t off = block_excl_scan(s, s_w, total) + before;
+    scan_store(j, i0, v, off);
+    if (blk == 0) {
         const int nb = (j.n + kScanTile - 1) / kScanTile;
         unsigned long long q = 0;
         for (int b = threadIdx.x; b < nb; b += kBlock) q += j.sqb[b];
@@ -435,70 +439,30 @@ __global__ __launch_bounds__(kBlock) void k_scan2_down_fold(ScanJob j0, ScanJob 
     }
 }
 
-// Both jobs in one launch when they are small (at most kSmallScan entries):
-// workgroup j scans job j alone, kScanItems entries per thread per pass,
-// carrying the running sum -- one launch instead of three, for arrays whose
-// scan time is launch latency.  Same outputs as the three-launch scan.
+// The whole scan by one workgroup when the job is small (at most kSmallScan
+// entries, at most two passes), carrying the running sum -- one launch instead
+// of two, for arrays whose scan time is launch latency.  Same outputs.
 constexpr int kSmallBlock = 1024;
-constexpr int kSmallScan = 8192;            // at most two passes of the workgroup
+constexpr int kSmallScan = 8192;
 
-__global__ __launch_bounds__(kSmallBlock) void k_scan_small(ScanJob j0, ScanJob j1)
+__global__ __launch_bounds__(kSmallBlock) void k_scan_small(ScanJob j)
 {
     __shared__ uint32_t s_w[kSmallBlock / kWave];
     __shared__ unsigned long long s_q[kSmallBlock / kWave];
-    const ScanJob j = blockIdx.x == 0 ? j0 : j1;
     uint32_t carry = 0;
     unsigned long long q = 0;
     for (int base = 0; base < j.n; base += kSmallBlock * kScanItems) {
         const int i0 = base + threadIdx.x * kScanItems;
-        uint32_t v[kScanItems];
-        uint32_t s = 0;
+        uint32_t v[kScanItems], s, total;
+        scan_load(j, i0, v, s);
 #pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            v[k] = (i0 + k < j.n) ? j.in[i0 + k] : 0u;
-            s += v[k];
-            q += (unsigned long long)v[k] * v[k];
-        }
-        uint32_t total;
-        uint32_t off = block_excl_scan<kSmallBlock>(s, s_w, total) + carry;
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            if (i0 + k < j.n) {
-                if (j.zero_in) j.in[i0 + k] = 0u;
-                j.excl[i0 + k] = off;
-                off += v[k];
-                if (j.incl) j.incl[i0 + k] = off;
-            }
-        }
+        for (int k = 0; k < kScanItems; ++k) q += (unsigned long long)v[k] * v[k];
+        const uint32_t off = block_excl_scan<kSmallBlock>(s, s_w, total) + carry;
+        scan_store(j, i0, v, off);
         carry += total;
     }
-    if (j.sq) {                                    // uniform per block
-        q = block_sum_u64<kSmallBlock>(q, s_q);
-        if (threadIdx.x == 0 && q) atomicAdd(j.sq, q);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// stable LSD radix sort of (key, value) -- reduce-then-scan per digit pass
-// ---------------------------------------------------------------------------
-
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t *__restrict__ keys, int n,
-                                                       int shift, int ntiles,
-                                                       uint32_t *__restrict__ hist)
-{
-    constexpr int R = 1 << D;
-    __shared__ uint32_t h[R];
-    for (int t = threadIdx.x; t < R; t += kBlock) h[t] = 0;
-    __syncthreads();
-    const int base = blockIdx.x * kRadixTile;
-#pragma unroll 4
-    for (int k = 0; k < kRadixTile / kBlock; ++k) {
-        const int i = base + k * kBlock + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & (R - 1)], 1u);
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < R; t += kBlock) hist[t * ntiles + blockIdx.x] = h[t];
+    q = block_sum_u64<kSmallBlock>(q, s_q);
+    if (threadIdx.x == 0 && q) atomicAdd(j.sq, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -823,104 +787,6 @@ struct AuxBuf {
     float *vx, *vy, *vz;
     int32_t *type, *id;
 };
-
-// Stable scatter.  Elements are ranked in index order: round r covers indices
-// base + r*256 + tid, and inside a round waves go in order and lanes go in
-// order (wave-level match by digit ballots).  gofs is the digit-major
-// exclusive scan of the per-tile histograms.  vin == nullptr means value = index.
-template <int D>
-__global__ __launch_bounds__(kScatterBlock) void k_radix_scatter(const uint32_t *__restrict__ kin,
-                                                                 const uint32_t *__restrict__ vin,
-                                                                 uint32_t *__restrict__ kout,
-                                                                 uint32_t *__restrict__ vout,
-                                                                 const uint32_t *__restrict__ gofs,
-                                                                 int n, int shift, int ntiles)
-{
-    constexpr int R = 1 << D;
-    constexpr int NW = kScatterBlock / kWave;
-    __shared__ uint32_t s_k[kRadixTile];
-    __shared__ uint32_t s_v[kRadixTile];
-    __shared__ uint32_t s_cnt[NW][R];
-    __shared__ uint32_t s_off[NW][R];
-    __shared__ uint32_t s_start[R];
-    __shared__ uint32_t s_gb[R];
-    __shared__ uint32_t s_w[NW];
-
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int base = blockIdx.x * kRadixTile;
-    for (int t = tid; t < NW * R; t += kScatterBlock) (&s_cnt[0][0])[t] = 0;
-    uint32_t running = 0;
-    uint32_t key[kRadixItems], val[kRadixItems], rank[kRadixItems];
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    __syncthreads();
-
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-        const int i = base + r * kScatterBlock + tid;
-        const bool valid = i < n;
-        const uint32_t k = valid ? kin[i] : 0u;
-        const uint32_t v = valid ? (vin ? vin[i] : (uint32_t)i) : 0u;
-        const uint32_t d = (k >> shift) & (R - 1);
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < D; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bb = __ballot(bit);
-            peers &= bit ? bb : ~bb;
-        }
-        const uint32_t lr = (uint32_t)__popcll(peers & lt);
-        if (valid && lr == 0) s_cnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (tid < R) {
-            uint32_t o = running;
-#pragma unroll
-            for (int ww = 0; ww < NW; ++ww) {
-                s_off[ww][tid] = o;
-                o += s_cnt[ww][tid];
-                s_cnt[ww][tid] = 0;
-            }
-            running = o;
-        }
-        __syncthreads();
-        key[r] = k;
-        val[r] = v;
-        rank[r] = valid ? s_off[w][d] + lr : 0u;
-    }
-
-    // exclusive scan of the tile's digit counts (threads tid < R hold them)
-    const uint32_t rv = tid < R ? running : 0u;
-    const uint32_t rinc = wave_incl_scan(rv);
-    if (lane == 63) s_w[w] = rinc;
-    __syncthreads();
-    uint32_t wb = 0;
-#pragma unroll
-    for (int ww = 0; ww < NW; ++ww) wb += ww < w ? s_w[ww] : 0u;
-    const uint32_t st = wb + rinc - rv;
-    if (tid < R) {
-        s_start[tid] = st;
-        s_gb[tid] = gofs[tid * ntiles + blockIdx.x];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-        const int i = base + r * kScatterBlock + tid;
-        if (i < n) {
-            const uint32_t d = (key[r] >> shift) & (R - 1);
-            const uint32_t lp = s_start[d] + rank[r];
-            s_k[lp] = key[r];
-            s_v[lp] = val[r];
-        }
-    }
-    __syncthreads();
-    const int nvalid = min(kRadixTile, n - base);
-    for (int j = tid; j < nvalid; j += kScatterBlock) {
-        const uint32_t k = s_k[j];
-        const uint32_t d = (k >> shift) & (R - 1);
-        const uint32_t g = s_gb[d] + (uint32_t)j - s_start[d];
-        if (kout) kout[g] = k;
-        vout[g] = s_v[j];
-    }
-}
 
 // Slots [off, off + n) of up to kPackMax device arrays of 32-bit words,
 // gathered chunk-major for a chunked download: chunk c (slots c*chunk ...)
