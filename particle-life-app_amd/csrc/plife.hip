@@ -464,7 +464,12 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     d.off = w.off;
     d.n = w.n;
     d.nx = gr.nx;
-    d.all_global = gr.nx < 3 ? 1 : 0;   // repeated stencil cells (Physics.java:377-395)
+    // repeated stencil cells (Physics.java:377-395), or matrix entries whose
+    // product with R is not finite: the summed force law needs finite ones
+    d.all_global = gr.nx < 3 ? 1 : 0;
+    for (const double m : w.matrix)
+        if (!std::isfinite(m * R)) d.all_global = 1;
+    d.exact_d2 = s.rmax <= 0x1p-6 ? 1 : 0;
     d.cell_base = cell_base;
     d.ntypes = w.ntypes;
     d.moff = moff;
@@ -2426,12 +2431,19 @@ int na_scratch_base(int dev, unsigned char **out)
 // b * bs), and zeros where the step expects them -- the counters, the tag
 // slot of the workgroup work record, and the first ncells cell counts (a
 // previous call may have stopped between binning and the cell scan).
-__global__ void k_na_setup(WorldDev wd, WorldDev *world, uint2 *blocks, int nblocks, int bs,
-                           unsigned long long *counters, uint32_t *work, uint32_t *cell_count,
+// Block 0 also looks the matrix over (it is in device memory): entries that
+// are not finite times R send the world down the literal path, as world_dev does.
+__global__ void k_na_setup(WorldDev wd, const double *matrix, WorldDev *world, uint2 *blocks, int nblocks,
+                           int bs, unsigned long long *counters, uint32_t *work, uint32_t *cell_count,
                            int ncells)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) *world = wd;
+    if (blockIdx.x == 0) {
+        bool bad = false;
+        for (int t = threadIdx.x; t < wd.ntypes * wd.ntypes; t += blockDim.x) bad |= !isfinite(matrix[t] * wd.R);
+        if (__syncthreads_or(bad)) wd.all_global = 1;
+        if (i == 0) *world = wd;
+    }
     if (i < 8) counters[i] = 0ull;
     if (i < nblocks) blocks[i] = make_uint2(0u, (uint32_t)(i * bs));
     if (i == 0) work[nblocks] = 0u;
@@ -2515,7 +2527,7 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
 
     const int setup_threads = std::max(nblocks + 1, 8);
     k_na_setup<<<std::min(ceil_div(std::max(setup_threads, nc), kBlock), 1024), kBlock, 0, stream>>>(
-        wd, t.d_worlds, t.d_blocks, nblocks, fp.bs, t.d_pairs, work, t.cell_count, nc);
+        wd, matrix, t.d_worlds, t.d_blocks, nblocks, fp.bs, t.d_pairs, work, t.cell_count, nc);
     LAUNCH_CHECK();
     if (n > 0) {
         // 1. cell keys and histogram; counters [0, 3) cleared, tag in [3]

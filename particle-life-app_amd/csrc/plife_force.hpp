@@ -123,18 +123,48 @@ __device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, doub
     }
 }
 
+// pair_d2 where every square of a pair in range is below 2^52 (rmax <= 2^-6,
+// WorldDev::exact_d2): squares and sums of integers below 2^53 are exact, so
+// FMAs give the same value in one instruction less per axis; a pair whose sum
+// is past 2^53 is out of range either way.
+template <int DIM, bool EXACT>
+__device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
+{
+    if constexpr (!EXACT) return pair_d2<DIM>(dx, dy, dz);
+    else return DIM == 3 ? fma(dx, dx, fma(dy, dy, dz * dz)) : fma(dx, dx, dy * dy);
+}
+
+// pair_coef with its branches summed in place of selected, for a finite mR:
+// below beta g is negative, at and above it 1/beta - 1/dist is not, so that of
+// max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
+// zero to the other branch's value -- two instructions where the compare, the
+// two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
+// free on its FMA, is max(g, 0).)
+__device__ __forceinline__ double pair_coef_sum(double d2, double mR, const WorldDev &a)
+{
+    const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
+    const double e = d2 * y0;
+    const double h = fma(-e, y0, 1.0);
+    const double y = fma(0.5 * y0, h, y0);
+    const double u = d2 * y;
+    const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
+    const double g = fmin(fmax(fma(t, -a.inv_1mb, 1.0), 0.0), 1.0);
+    const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);
+    return fma(mR * g, y, rep);
+}
+
 // pair64 with no branch: the coefficient of a pair out of range (or
 // rejected by the caller, ok = false) is selected to 0, which leaves the sums
 // bit-identical (a sum that starts at +0 is never -0), so that the chains of
 // neighbouring candidates can overlap.
-template <int DIM, bool DEBUG>
+template <int DIM, bool DEBUG, bool EXACT>
 __device__ __forceinline__ void pair64_sel(Acc &acc, bool ok, int dxi, int dyi, int dzi, double mR,
                                            uint32_t qid, const WorldDev &a)
 {
     const double dx = (double)dxi, dy = (double)dyi, dz = (double)dzi;
-    const double d2 = pair_d2<DIM>(dx, dy, dz);
+    const double d2 = pair_d2_of<DIM, EXACT>(dx, dy, dz);
     const bool in = ok & (d2 != 0.0) & (d2 <= a.r2u);    // Physics.java:432
-    double cf = pair_coef(d2, mR, a);
+    double cf = pair_coef_sum(d2, mR, a);
     asm volatile("" : "+v"(cf));        // computed for every candidate: no branch
     const double c = in ? cf : 0.0;
     acc.x = fma(c, dx, acc.x);
@@ -496,8 +526,8 @@ __device__ __forceinline__ uint32_t low_bits(int n)
 // candidates, word by word in candidate order, two per iteration (half the
 // loop's bookkeeping; their force laws overlap).  load(m, kb) fetches the
 // next non-zero mask word and its first candidate.
-template <int DIM, bool WRAP, bool DEBUG, bool MLDS, typename Load>
-__device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w, const Staged &s,
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS, bool EXACT, typename Load>
+__device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev &w, const Staged &s,
                                           const double *M, Acc &ab, int left, Load &&load, uint32_t px,
                                           uint32_t py, uint32_t pz, int mrow)
 {
@@ -516,7 +546,7 @@ __device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w,
         }
         const int idx = mrow + (int)s.type[k];
         const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-        pair64_sel<DIM, DEBUG>(ab, ok, dxi, dyi, dzi, m, DEBUG ? s.id[k] : 0u, w);
+        pair64_sel<DIM, DEBUG, EXACT>(ab, ok, dxi, dyi, dzi, m, DEBUG ? s.id[k] : 0u, w);
     };
     uint32_t m = 0;
     int kb = 0;
@@ -534,6 +564,15 @@ __device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w,
         visit(k2);
     }
     if (left > 0) visit(next());
+}
+
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS, typename Load>
+__device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w, const Staged &s,
+                                          const double *M, Acc &ab, int left, Load &&load, uint32_t px,
+                                          uint32_t py, uint32_t pz, int mrow)
+{
+    if (w.exact_d2) walk_home_of<DIM, WRAP, DEBUG, MLDS, true>(a, w, s, M, ab, left, load, px, py, pz, mrow);
+    else walk_home_of<DIM, WRAP, DEBUG, MLDS, false>(a, w, s, M, ab, left, load, px, py, pz, mrow);
 }
 
 // Counting sort of the HPT * T homes of a workgroup by their kept-candidate

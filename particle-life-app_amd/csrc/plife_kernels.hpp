@@ -128,11 +128,12 @@ __global__ void k_zero_u64(unsigned long long *p, int n)
 // world exactly as stepping it alone would.
 struct WorldDev {
     int off, n;                      // particle slots
-    int nx, all_global;              // cells per axis; 1 when nx < 3 (literal stencil)
+    int nx, all_global;              // cells per axis; 1: literal stencil and force law (home_global)
     uint32_t cell_base;              // first batch cell of this world
     int ntypes, moff;                // matrix size and offset (doubles) in the batch matrix
     int wrap;
     float r2hi;                      // screen bound, units 2^-64: (rmax 2^32)^2 (1 + 2^-20)
+    int exact_d2;                    // 1: squared distances in range are exact (pair_d2_of)
     int sbias;                       // screen bound on 16-bit coordinates: -(bq + 1) (screen_hi)
     double cs, ics;                  // cell size = rmax (Physics.java:312), and 1 / cs
     double r2u;                      // fl(rmax*rmax) * 2^64: the reference's bound in units 2^-64
