@@ -126,6 +126,10 @@ constexpr int kDlChunks = 8;           // downloads move in at most this many ch
 constexpr int kFlightSlots = 64;       // events marking queued launches of plife_update
 constexpr double kStopWindowMs = 20.0; // device work plife_update keeps queued (stop latency)
 constexpr int kDlMinChunk = 65536;     // slots; smaller downloads are one chunk
+// bytes; downloads up to it are written to pinned memory by k_pack (1k-particle
+// app frame 79 -> 64 us, 64 worlds of 1k to 8k 1.1 ms less; 512 worlds of up to
+// 64k particles 191.5 ms by copies, 185.3 at 256 KiB, 182.4 at 1 MiB, 182.0 at 4)
+constexpr size_t kDlDirect = (size_t)1 << 20;
 
 // Grow-only device array: reallocated (contents dropped) when too small.  The
 // old array goes to `retired` when given and small enough, else is freed.
@@ -249,6 +253,7 @@ struct plife_physics {
     size_t stat_cap = 0;
     std::vector<void *> retired_host;  // replaced pinned buffers, freed at destroy
     unsigned char *pin = nullptr;      // pinned staging of state downloads
+    uint32_t *pin_dev = nullptr;       // the device's address of pin
     size_t pin_cap = 0;
     uint32_t *dl_dev = nullptr;        // device staging of state downloads (chunk-major)
     size_t dl_cap = 0;
@@ -1942,6 +1947,14 @@ int ensure_pin(plife_physics *h, size_t bytes)
         h->pin = nullptr;
         return fail(PLIFE_ERR_MEMORY, "hipHostMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
     }
+    void *dev = nullptr;
+    const hipError_t e2 = hipHostGetDevicePointer(&dev, h->pin, 0);
+    if (e2 != hipSuccess) {
+        (void)hipHostFree(h->pin);
+        h->pin = nullptr;
+        return fail(PLIFE_ERR_DEVICE, "hipHostGetDevicePointer: %s", hipGetErrorString(e2));
+    }
+    h->pin_dev = (uint32_t *)dev;
     h->pin_cap = bytes;
     return PLIFE_OK;
 }
@@ -2108,16 +2121,20 @@ int set_slots(plife_physics *h, WorldHost &w, int32_t k, const int32_t *slots, c
     return PLIFE_OK;
 }
 
-// Downloads slots [off, off + n) of the current buffers.  k_pack gathers the
-// requested arrays chunk by chunk into device staging, one DMA per chunk moves
-// it to pinned memory, and host threads convert each chunk to the caller's
-// FP64 triples as soon as its DMA has completed, while later chunks are still
-// in flight.
+// Downloads slots [off, off + n) of the current buffers.  A small download's
+// k_pack writes the requested arrays straight into pinned host memory: one
+// launch and one wait, where a copy adds an enqueue, a DMA start and an event.
+// A larger one's gathers them chunk by chunk into device staging, one DMA per
+// chunk moves it to pinned memory, and host threads convert each chunk to the
+// caller's FP64 triples as soon as its DMA has completed, while later chunks
+// are still in flight.
 int download_particles(plife_physics *h, int off, int n, double *pos, double *vel, int32_t *types,
                        int32_t *ids, bool d3)
 {
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    if (n == 0) return PLIFE_OK;
+    if (n == 0 || !(pos || vel || types || ids)) {
+        HIP_TRY(hipStreamSynchronize(h->stream));
+        return PLIFE_OK;
+    }
     const PosBuf P = h->P(h->pc);
     const AuxBuf A = h->A(h->ac);
     PackArgs pk{};
@@ -2130,12 +2147,12 @@ int download_particles(plife_physics *h, int off, int n, double *pos, double *ve
     const int ix = add(pos, P.x), iy = add(pos, P.y), iz = add(pos && d3, P.z);
     const int ivx = add(vel, A.vx), ivy = add(vel, A.vy), ivz = add(vel && d3, A.vz);
     const int it = add(types, A.type), ii = add(ids, A.id);
-    if (na == 0) return PLIFE_OK;
     const size_t words = (size_t)na * (size_t)n;
-    int rc = ensure_dev(&h->dl_dev, &h->dl_cap, words);
+    int rc = ensure_pin(h, words * 4);
     if (rc) return rc;
-    if ((rc = ensure_pin(h, words * 4))) return rc;
-    const int chunk = n >= 2 * kDlMinChunk
+    const bool direct = words * 4 <= kDlDirect;
+    if (!direct && (rc = ensure_dev(&h->dl_dev, &h->dl_cap, words))) return rc;
+    const int chunk = !direct && n >= 2 * kDlMinChunk
                           ? (int)std::min<long long>(n, ((long long)ceil_div(n, kDlChunks) + 255) / 256 * 256)
                           : n;
     const int nchunks = ceil_div(n, chunk);
@@ -2143,10 +2160,11 @@ int download_particles(plife_physics *h, int off, int n, double *pos, double *ve
     pk.off = off;
     pk.n = n;
     pk.chunk = chunk;
-    k_pack<<<ceil_div(n, kBlock), kBlock, 0, h->stream>>>(pk, h->dl_dev);
-    LAUNCH_CHECK();
     uint32_t *const stage = (uint32_t *)h->pin;
-    for (int c = 0; c < nchunks; ++c) {
+    k_pack<<<ceil_div(n, kBlock), kBlock, 0, h->stream>>>(pk, direct ? h->pin_dev : h->dl_dev);
+    LAUNCH_CHECK();
+    if (direct) HIP_TRY(hipStreamSynchronize(h->stream));
+    for (int c = 0; !direct && c < nchunks; ++c) {
         const size_t first = (size_t)c * chunk * na;
         const size_t len = (size_t)std::min(chunk, n - c * chunk);
         HIP_TRY(hipMemcpyAsync(stage + first, h->dl_dev + first, len * na * 4, hipMemcpyDeviceToHost,
@@ -2203,7 +2221,7 @@ int download_particles(plife_physics *h, int off, int n, double *pos, double *ve
         });
     hipError_t err = hipSuccess;
     for (int c = 0; c < nchunks; ++c) {
-        err = hipEventSynchronize(h->dl_ev[c]);
+        if (!direct) err = hipEventSynchronize(h->dl_ev[c]);
         if (err != hipSuccess) {
             failed.store(true, std::memory_order_release);
             ready.store(nchunks, std::memory_order_release);
