@@ -1100,15 +1100,21 @@ int balance_blocks(plife_physics *h)
 }
 
 // Which force kernel steps each world.  A world goes to the sparse-world
-// kernel when a staged workgroup of its homes would span more than two grid
-// rows or more cells than the staged cell table holds; the span follows from
-// the occupancy of the cells its particles sit in, estimated from the
-// neighbours per particle of the last measured step (a uniform world's count
-// before that): local density nb / V(rmax) times the cell volume rmax^dim.
+// kernel when the cells its particles sit in hold fewer than kSparseOcc
+// particles, estimated from the neighbours per particle of the last measured
+// step (a uniform world's count before that): local density nb / V(rmax) times
+// the cell volume rmax^dim; or when a staged workgroup would span more cells
+// than its cell table holds.  Below the line a staged workgroup spans many rows
+// and stages far more than it uses; above it one thread per home is a long
+// chain of dependent reads (us a step, staged vs sparse: 2D 300k particles 74.6
+// vs 63.0 at 0.7 a cell, 64.1 vs 63.9 at 1.5, 62.9 vs 66.3 at 2.5; 1k 26.9 vs
+// 36.2 at 2.5; 3D 500k 181 vs 115 at 1, 240 vs 140 at 2, 169 vs 194 at 4).
 // Grids of fewer than 3 cells per axis always take it (literal stencil over
-// repeated cells).  Hysteresis keeps worlds near the threshold from
-// switching kernels, and so recapturing, at every update.  Results do not
-// depend on the class.
+// repeated cells).  Hysteresis keeps worlds near the threshold from switching
+// kernels, and so recapturing, at every update.  Results do not depend on the
+// class.
+constexpr double kSparseOcc2 = 1.5, kSparseOcc3 = 3.0;
+
 void classify_worlds(plife_physics *h)
 {
     const int dim = h->dim == 3 ? 3 : 2;
@@ -1133,7 +1139,7 @@ void classify_worlds(plife_physics *h)
             const double occ = std::max({avg, nb * cell / ball, 1e-9});
             const double span = bs / occ;              // cells spanned by a workgroup's homes
             const double k = w.sparse ? 0.75 : 1.0;
-            sparse = span > 2.0 * gr.nx * k || NR * (span + 6.0) > 2048.0 * k;
+            sparse = occ * k < (dim == 3 ? kSparseOcc3 : kSparseOcc2) || NR * (span + 6.0) > 2048.0 * k;
         }
         if (sparse != w.sparse) {
             w.sparse = sparse;

@@ -320,21 +320,29 @@ __device__ __forceinline__ void visit_run(const ForceArgs &a, const WorldDev &w,
                                           int g, uint32_t hx, uint32_t hy, uint32_t hz, int row,
                                           Acc &acc, int lo, int hi)
 {
-    for (int j = lo; j < hi; ++j) {
-        if (j == g) continue;
-        const uint4 q = a.rec[j];
-        const uint32_t qx = q.x, qy = q.y, qz = DIM == 3 ? q.z : 0u;
-        const int dxi = (int)(qx - hx), dyi = (int)(qy - hy);
-        const int dzi = DIM == 3 ? (int)(qz - hz) : 0;
-        if (!WRAP) {
-            // plain difference of the clamped world: skip |D| >= 1/2
-            bool ok = ((dxi >= 0) == (qx >= hx)) & ((dyi >= 0) == (qy >= hy));
-            if (DIM == 3) ok &= ((dzi >= 0) == (qz >= hz));
+    constexpr int G = 4;               // records read together
+#pragma unroll 1
+    for (int j0 = lo; j0 < hi; j0 += G) {
+        uint4 q[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u) q[u] = a.rec[min(j0 + u, hi - 1)];
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+            const int j = j0 + u;
+            const uint32_t qx = q[u].x, qy = q[u].y, qz = DIM == 3 ? q[u].z : 0u;
+            const int dxi = (int)(qx - hx), dyi = (int)(qy - hy);
+            const int dzi = DIM == 3 ? (int)(qz - hz) : 0;
+            bool ok = (j < hi) & (j != g);
+            if (!WRAP) {
+                // plain difference of the clamped world: skip |D| >= 1/2
+                ok &= ((dxi >= 0) == (qx >= hx)) & ((dyi >= 0) == (qy >= hy));
+                if (DIM == 3) ok &= ((dzi >= 0) == (qz >= hz));
+            }
             if (!ok) continue;
+            const int idx = row + (int)q[u].w;
+            const double m = MLDS ? Mlds[idx] : a.matrix[w.moff + idx] * w.R;
+            pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m, DEBUG ? (uint32_t)a.id[a.perm[j]] : 0u, w);
         }
-        const int idx = row + (int)q.w;
-        const double m = MLDS ? Mlds[idx] : a.matrix[w.moff + idx] * w.R;
-        pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m, DEBUG ? (uint32_t)a.id[a.perm[j]] : 0u, w);
     }
 }
 
