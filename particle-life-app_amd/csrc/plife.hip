@@ -72,7 +72,11 @@ constexpr int kMaxWorlds = 65535;     // the world index of a slot is a u16
 constexpr int kMaxLds = 65536;
 constexpr int kTuneSteps = 24;         // an update long enough to time two configurations
 constexpr int kTuneMax = 22;           // steps such a timing takes at most (4 x 4 + 3 switches + 3)
-constexpr size_t kWordLds = 24576;    // most LDS for the balanced path's mask words
+constexpr size_t kWordLds = 32768;    // most LDS for the mask words of one window
+constexpr double kStageSlack = 1.25, kPoolSlack = 1.1;   // over the expected staged entries and mask words
+constexpr double kMaxSlack = 1.6;     // over those, where LDS is free
+constexpr int kCus = 256;             // gfx950: CUs, LDS per CU, and what a workgroup uses besides the layout
+constexpr size_t kCuLds = 163840, kStaticLds = 5120;
 
 struct ForcePlan {
     int wpool = 0;                    // mask words per workgroup with one window (0: always several)
@@ -891,28 +895,61 @@ int record(plife_physics *h, PhaseEvents *ev, int k)
 // mixed: worlds of several densities share the launch.  The plan never changes
 // results: every home visits its candidates in the same order whatever the
 // windows and workgroup size.
-ForcePlan plan_force_for(int dim, double avg, bool clustered, bool mixed, const plife_tuning &t, bool dbg,
-                         int ntypes_max)
+ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustered, bool mixed,
+                         const plife_tuning &t, bool dbg, int ntypes_max)
 {
     const int NR = dim == 3 ? 9 : 3;
     ForcePlan p;
     p.bs = t.block_homes ? t.block_homes : (clustered ? 128 : 256);
+    // a workgroup takes the global path when its homes lie in more rows than the
+    // part table holds: worlds of few cells per row take fewer homes (force
+    // kernel, us, 64 / 128 / 256 homes: 1k particles in 20 x 20 cells 15.6 / 16.9
+    // / 27.4, in 13 x 13 17.8 / 18.8 / 37.5; 30k in 16^3 40 / 35 / 53), and small
+    // ones a little sooner, where more workgroups fill more CUs
+    if (!t.block_homes && !clustered && nx > 0)
+        while (p.bs > 64 && p.bs / std::max(avg, 1e-9) > (n <= 100000 ? 1.5 : 2.0) * nx) p.bs /= 2;
     // a workgroup of bs homes spans ~bs/avg + 1 cells of a row; it stages NR
     // rows of (span + 2) cells.  Clustered worlds keep a short cell table: the
     // few sparse workgroups that span more cells take the global path.
     const double span = p.bs / std::max(avg, 1e-9) + 1.0;
-    // one window (uniform worlds): a home's stencil row is a run of three cells,
-    // ~3 avg candidates, ceil(run / 32) mask words; the workgroup's pool holds
-    // 10% more than the expected total (workgroups needing more take several
-    // windows)
-    if (!clustered && !t.windowed_only) {
-        const double run = 3.0 * avg;
-        const long long pool = (long long)std::ceil(p.bs * NR * (run / 32.0 + 0.5) * 1.1) + 64;
-        if (pool <= 65535 && (size_t)pool * 6 <= kWordLds) p.wpool = (int)pool;
-    }
     p.max_cells = (int)std::min<double>(std::max(64.0, std::ceil(NR * (span + 2.0) * 1.5 + 16)),
                                         clustered ? 384.0 : 2048.0);
-    // several windows: mask words per home (32 candidates each).  Where one
+    const bool m_in_lds = ntypes_max <= kMaxTypesLds;
+    auto total = [&](const ForcePlan &q, long long c) {
+        return force_lds_layout(dim, dbg, ntypes_max, m_in_lds, (int)c, p.bs, q.max_cells, q.wpool,
+                                q.wpool2).total;
+    };
+    auto entries = [&](double slack) {
+        const long long want = (long long)std::ceil(NR * (span + 2.0) * avg * slack) + 64;
+        return std::min<long long>((want + 63) / 64 * 64, 65472);
+    };
+    // One window (uniform worlds): a home's stencil row is a run of three cells,
+    // ~3 avg candidates, ceil(run / 32) mask words; the pool holds the expected
+    // total and some slack (workgroups needing more take several windows).
+    const double words = p.bs * NR * (3.0 * avg / 32.0 + 0.5);
+    auto pool = [&](double slack) { return (long long)std::ceil(words * slack) + 64; };
+    long long want = 64;
+    if (!clustered && !t.windowed_only && pool(kPoolSlack) * 6 <= (long long)kWordLds) {
+        p.wpool = (int)pool(kPoolSlack);
+        want = entries(t.stage_slack > 0.0 ? t.stage_slack : kStageSlack);
+        // A launch that leaves CUs room for all its workgroups at once pays
+        // nothing for a larger layout, and its time is that of its slowest
+        // workgroup: as much slack as fits, so that none takes several windows.
+        if (t.stage_slack == 0.0 && n > 0) {
+            const long long per_cu = (ceil_div(n, p.bs) + kCus - 1) / kCus;
+            const size_t room = std::min<size_t>(kMaxLds, kCuLds / (size_t)per_cu - kStaticLds);
+            for (double more = kMaxSlack; more > 1.0 && kCuLds / (size_t)per_cu > kStaticLds; more -= 0.05) {
+                ForcePlan q = p;
+                q.wpool = (int)pool(kPoolSlack * more);
+                const long long c = entries(kStageSlack * more);
+                if (q.wpool > 65535 || total(q, c) > room) continue;
+                p.wpool = q.wpool;
+                want = c;
+                break;
+            }
+        }
+    }
+    // Several windows: mask words per home (32 candidates each).  Where one
     // window is the rule (a single uniform world), no more than fit the space of
     // its pool: LDS per workgroup sets how many share a CU (1M 2D world: 0.218 ms
     // a step within the pool, 0.231 at 7 words).  Worlds of several densities in
@@ -926,24 +963,18 @@ ForcePlan plan_force_for(int dim, double avg, bool clustered, bool mixed, const 
                             : std::max(mixed || p.wpool == 0 ? 9 : 4, std::min(fit, 16));
     p.lcap = std::min(p.lcap, 32768 / (6 * p.bs));                       // words stay within 32 KB of LDS
     p.wpool2 = p.lcap * p.bs;
-    const size_t budget = kMaxLds;
-    const double slack = t.stage_slack > 0.0 ? t.stage_slack : 1.25;
-    long long want = (long long)std::ceil(NR * (span + 2.0) * avg * slack) + 64;
     // where every workgroup streams windows, stage no more than its words cover
-    if (p.wpool == 0) want = std::min<long long>(clustered ? 65535 : want, 32ll * (p.lcap - 1));
-    want = std::min<long long>((want + 63) / 64 * 64, 65535);
-    const bool m_in_lds = ntypes_max <= kMaxTypesLds;
-    auto total = [&](long long c) {
-        return force_lds_layout(dim, dbg, ntypes_max, m_in_lds, (int)c, p.bs, p.max_cells,
-                                p.wpool, p.wpool2).total;
-    };
+    if (p.wpool == 0) {
+        want = (32ll * (p.lcap - 1) + 63) / 64 * 64;
+        if (!clustered) want = std::min(want, entries(t.stage_slack > 0.0 ? t.stage_slack : kStageSlack));
+    }
     // keep room for a useful staging window: shrink the cell table first
     const long long min_cap = std::min<long long>(want, 256);
-    while (p.max_cells > 64 && total(min_cap) > budget) p.max_cells = std::max(64, p.max_cells * 3 / 4);
+    while (p.max_cells > 64 && total(p, min_cap) > kMaxLds) p.max_cells = std::max(64, p.max_cells * 3 / 4);
     // then shrink the staging capacity until the layout fits the LDS budget
-    while (want > 64 && total(want) > budget) want -= 64;
-    p.cap = (int)std::max(0LL, want);
-    p.lds = total(p.cap);
+    while (want > 64 && total(p, want) > kMaxLds) want -= 64;
+    p.cap = (int)want;
+    p.lds = total(p, p.cap);
     return p;
 }
 
@@ -961,17 +992,20 @@ ForcePlan plan_force(const plife_physics *h)
     const int dim = h->dim == 3 ? 3 : 2;
     // density of the worlds the staged kernel steps (all of them if none is)
     long long sn = 0, sc = 0;
+    int nx = 0;                        // cells per row of a single world
     for (const WorldHost &w : h->worlds)
         if (!w.sparse) {
             sn += w.n;
             sc += grid_of(w.st).ncells;
+            if (h->worlds.size() == 1) nx = grid_of(w.st).nx;
         }
     if (sc == 0) {
         sn = h->n;
         sc = h->ncells;
     }
     const double avg = (double)sn / (double)std::max(sc, 1LL);
-    return plan_force_for(dim, avg, h->clustered, h->worlds.size() > 1, plan_tuning(h), h->debug != 0, h->ntypes_max);
+    return plan_force_for(dim, avg, sn, nx, h->clustered, h->worlds.size() > 1, plan_tuning(h), h->debug != 0,
+                          h->ntypes_max);
 }
 
 // The class of a layout for the measured homes per workgroup: dimension,
@@ -1727,7 +1761,7 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
     // times the planner's choice (256, or 128 for clustered 3D) against the
     // other (time_pair) and keeps the faster for every layout of the class.
     if (shape_tune_due(h) && nsteps >= kTuneSteps && nsteps - k >= kTuneMax) {
-        const int cand[2] = {h->clustered ? 128 : 256, h->clustered ? 256 : 128};   // the planner's first
+        const int cand[2] = {h->plan.bs, h->plan.bs == 128 ? 256 : 128};            // the planner's first
         float t[2];
         rc = time_pair([&](int p) {
             h->auto_bs = cand[p];
@@ -2519,7 +2553,7 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
     const WorldDev wd = world_dev(wh, 0u, 0);
     const int nc = (int)gr.ncells;
     const double avg = (double)n / (double)nc;
-    const ForcePlan fp = plan_force_for(s->dim, avg, false, false, plife_tuning{}, false, ntypes);
+    const ForcePlan fp = plan_force_for(s->dim, avg, n, gr.nx, false, false, plife_tuning{}, false, ntypes);
     const int nblocks = ceil_div(n, fp.bs);
 
     // a transient view of the scratch as the step helpers' buffers (no
