@@ -33,6 +33,7 @@
 #include "../../include/plife.h"
 #include "plife_force.hpp"
 #include "plife_small.hpp"
+#include "plife_split.hpp"
 
 using namespace plife;
 
@@ -83,6 +84,11 @@ struct ForcePlan {
     int wpool2 = 0;                   // mask words per workgroup with several windows
     int bs, lcap, max_cells, cap;
     size_t lds;
+};
+
+struct SplitPlan {
+    int cap = 0, max_cells = 0;
+    size_t lds = 0;
 };
 
 template <typename T>
@@ -172,6 +178,11 @@ Grid grid_of(const plife_settings &s)
 
 }  // namespace
 
+// The force kernels of the multi-launch path: k_force, k_force_sparse and
+// k_force_split.  Each steps whole worlds.
+enum ForceKind { kStaged, kSparse, kSplit, kForceKinds };
+constexpr int kSegments = 2 * kForceKinds;   // (periodic, clamped) x kernel
+
 // One world as the host keeps it.
 struct WorldHost {
     int32_t id = 0;
@@ -183,7 +194,8 @@ struct WorldHost {
     bool live = true;                  // false once removed (dropped at the next layout)
     double nb = -1.0;                  // neighbours per particle in the last measured step
     int max_type = -1;                 // highest type of its particles (must stay < ntypes to step)
-    bool sparse = false;               // stepped by the sparse-world force kernel
+    double hot = -1.0;                 // neighbours per particle of its densest workgroup, ditto
+    int kind = kStaged;                // the force kernel that steps it
 };
 
 struct plife_physics {
@@ -219,7 +231,7 @@ struct plife_physics {
     uint2 *d_blocks = nullptr;
     size_t blocks_cap = 0;
     int blocks_bs = 0, nb_total = 0;
-    int seg[4] = {};                   // blocks of (periodic, clamped) x (staged, sparse) worlds
+    int seg[kSegments] = {};           // blocks of (periodic, clamped) x ForceKind worlds
     uint64_t blocks_version = ~0ull, blocks_classes = ~0ull;
     uint64_t blocks_serial = 0;        // bumped whenever the table's content or order changes
     std::vector<uint64_t> block_key;   // per entry: world id, sparse kernel, first home in the world
@@ -300,6 +312,7 @@ struct plife_physics {
     // launch tuning (0 = automatic), the current plan, what the last launch used
     plife_tuning tune{};
     ForcePlan plan{};
+    SplitPlan split{};
     size_t last_lds = 0;
     int last_cap = 0, last_bs = 0, last_lcap = 0;
 
@@ -673,9 +686,11 @@ int sync_layout(plife_physics *h)
     return PLIFE_OK;
 }
 
-// Force workgroup table: segments of periodic staged, periodic sparse,
-// clamped staged and clamped sparse worlds (one launch each), bs homes per
-// staged block and kSparseBlock per sparse block.
+// Homes per workgroup of a force kernel; bs: the staged kernel's.
+int kind_homes(int kind, int bs) { return kind == kSparse ? kSparseBlock : kind == kSplit ? kSplitHomes : bs; }
+
+// Force workgroup table: segments of periodic staged, sparse and split worlds,
+// then clamped ones (one launch each).
 int ensure_blocks(plife_physics *h, int bs)
 {
     if (h->blocks_bs == bs && h->blocks_version == h->version && h->blocks_classes == h->classes)
@@ -691,19 +706,20 @@ int ensure_blocks(plife_physics *h, int bs)
     h->blocks.clear();
     h->block_key.clear();
     h->block_est.clear();
-    for (int s = 0; s < 4; ++s) {
-        const bool wrap = s < 2, sparse = (s & 1) != 0;
+    for (int s = 0; s < kSegments; ++s) {
+        const bool wrap = s < kForceKinds;
+        const int kind = s % kForceKinds;
         const size_t before = h->blocks.size();
         for (int w = 0; w < (int)h->worlds.size(); ++w) {
             const WorldHost &wh = h->worlds[w];
-            if ((wh.st.wrap != 0) != wrap || wh.sparse != sparse) continue;
-            const int step = sparse ? kSparseBlock : bs;
+            if ((wh.st.wrap != 0) != wrap || wh.kind != kind) continue;
+            const int step = kind_homes(kind, bs);
             // expected pairs per home where no measurement carries over
             const double r = wh.st.rmax;
             const double ball = wh.st.dim == 3 ? 4.0 / 3.0 * M_PI * r * r * r : M_PI * r * r;
             const double nb = wh.nb >= 0.0 ? wh.nb : std::max(wh.n - 1, 0) * ball;
             for (int g = 0; g < wh.n; g += step) {
-                const uint64_t key = ((uint64_t)(uint32_t)wh.id << 33) | ((uint64_t)sparse << 32) | (uint32_t)g;
+                const uint64_t key = ((uint64_t)(uint32_t)wh.id << 33) | ((uint64_t)kind << 31) | (uint32_t)g;
                 const auto it = prev.find(key);
                 const double homes = std::min(step, wh.n - g);
                 h->blocks.push_back(make_uint2((uint32_t)w, (uint32_t)(wh.off + g)));
@@ -833,19 +849,39 @@ void launch_sparse(plife_physics *h, const ForceArgs &a, int nblocks)
     else k_force_sparse<DIM, WRAP, DEBUG, false><<<nblocks, kSparseBlock, 0, h->stream>>>(a);
 }
 
-// One launch per segment of the block table present in the batch: periodic
-// staged, periodic sparse, clamped staged, clamped sparse.
+template <int DIM, bool WRAP, bool DEBUG>
+void launch_split(plife_physics *h, ForceArgs a, int nblocks)
+{
+    a.cap = h->split.cap;
+    a.max_cells = h->split.max_cells;
+    if (a.m_in_lds) k_force_split<DIM, WRAP, DEBUG, true><<<nblocks, kSplitThreads, h->split.lds, h->stream>>>(a);
+    else k_force_split<DIM, WRAP, DEBUG, false><<<nblocks, kSplitThreads, h->split.lds, h->stream>>>(a);
+}
+
+// One launch per segment of the block table present in the batch.
 int launch_force_any(plife_physics *h, ForceArgs a, int bs, size_t lds)
 {
     const bool dbg = h->debug != 0;
     int base = 0;
-    for (int s = 0; s < 4; ++s) {
-        const bool wrap = s < 2, sparse = (s & 1) != 0;
+    for (int s = 0; s < kSegments; ++s) {
+        const bool wrap = s < kForceKinds;
+        const int kind = s % kForceKinds;
         const int nb = h->seg[s];
         a.block_base = base;
         base += nb;
         if (nb <= 0) continue;
-        if (sparse) {
+        if (kind == kSplit) {
+            if (h->dim == 3) {
+                if (wrap) dbg ? launch_split<3, true, true>(h, a, nb) : launch_split<3, true, false>(h, a, nb);
+                else dbg ? launch_split<3, false, true>(h, a, nb) : launch_split<3, false, false>(h, a, nb);
+            } else {
+                if (wrap) dbg ? launch_split<2, true, true>(h, a, nb) : launch_split<2, true, false>(h, a, nb);
+                else dbg ? launch_split<2, false, true>(h, a, nb) : launch_split<2, false, false>(h, a, nb);
+            }
+            LAUNCH_CHECK();
+            continue;
+        }
+        if (kind == kSparse) {
             if (h->dim == 3) {
                 if (wrap) dbg ? launch_sparse<3, true, true>(h, a, nb) : launch_sparse<3, true, false>(h, a, nb);
                 else dbg ? launch_sparse<3, false, true>(h, a, nb) : launch_sparse<3, false, false>(h, a, nb);
@@ -904,10 +940,10 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
     // a workgroup takes the global path when its homes lie in more rows than the
     // part table holds: worlds of few cells per row take fewer homes (force
     // kernel, us, 64 / 128 / 256 homes: 1k particles in 20 x 20 cells 15.6 / 16.9
-    // / 27.4, in 13 x 13 17.8 / 18.8 / 37.5; 30k in 16^3 40 / 35 / 53), and small
-    // ones a little sooner, where more workgroups fill more CUs
+    // / 27.4, in 13 x 13 17.8 / 18.8 / 37.5; 30k in 16^3 40 / 35 / 53; 300k in 42^3
+    // 168 / 112 / 167, in 33^3 186 / 132 / 108)
     if (!t.block_homes && !clustered && nx > 0)
-        while (p.bs > 64 && p.bs / std::max(avg, 1e-9) > (n <= 100000 ? 1.5 : 2.0) * nx) p.bs /= 2;
+        while (p.bs > 64 && p.bs / std::max(avg, 1e-9) > 1.5 * nx) p.bs /= 2;
     // a workgroup of bs homes spans ~bs/avg + 1 cells of a row; it stages NR
     // rows of (span + 2) cells.  Clustered worlds keep a short cell table: the
     // few sparse workgroups that span more cells take the global path.
@@ -987,6 +1023,22 @@ plife_tuning plan_tuning(const plife_physics *h)
     return t;
 }
 
+// Launch shape of the split kernel: windows of kSplitWindow candidates (dense
+// 196k 2D world: 1.98 ms a step at 256, 2.03 at 128, 2.48 at 384), and a cell
+// table for workgroups of 64 homes (the few that span more take the global
+// path).
+constexpr int kSplitWindow = 256;
+
+SplitPlan plan_split_for(int dim, bool dbg, int ntypes_max)
+{
+    SplitPlan p;
+    p.max_cells = dim == 3 ? 768 : 384;
+    for (p.cap = kSplitWindow;; p.cap -= 32) {
+        p.lds = split_lds_layout(dim, dbg, ntypes_max, ntypes_max <= kMaxTypesLds, p.cap, p.max_cells).total;
+        if (p.cap <= 64 || p.lds + kStaticLds <= (size_t)kMaxLds) return p;
+    }
+}
+
 ForcePlan plan_force(const plife_physics *h)
 {
     const int dim = h->dim == 3 ? 3 : 2;
@@ -994,7 +1046,7 @@ ForcePlan plan_force(const plife_physics *h)
     long long sn = 0, sc = 0;
     int nx = 0;                        // cells per row of a single world
     for (const WorldHost &w : h->worlds)
-        if (!w.sparse) {
+        if (w.kind == kStaged) {
             sn += w.n;
             sc += grid_of(w.st).ncells;
             if (h->worlds.size() == 1) nx = grid_of(w.st).nx;
@@ -1015,7 +1067,7 @@ uint64_t shape_class(const plife_physics *h)
 {
     long long sn = 0, sc = 0;
     for (const WorldHost &w : h->worlds)
-        if (!w.sparse) {
+        if (w.kind == kStaged) {
             sn += w.n;
             sc += grid_of(w.st).ncells;
         }
@@ -1035,7 +1087,7 @@ bool shape_tune_due(const plife_physics *h)
         h->bs_meas == h->version)
         return false;
     for (const WorldHost &w : h->worlds)
-        if (!w.sparse && w.n > 0) return true;
+        if (w.kind == kStaged && w.n > 0) return true;
     return false;
 }
 
@@ -1091,7 +1143,7 @@ int balance_blocks(plife_physics *h)
         for (int i = 0; i < nb; ++i) work[i] = __atomic_load_n(h->work_host + i, __ATOMIC_RELAXED);
     bool changed = false;
     int base = 0;
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < kSegments; ++s) {
         const int n = h->seg[s];
         const int b0 = base;
         base += n;
@@ -1148,6 +1200,13 @@ int balance_blocks(plife_physics *h)
 // kernels, and so recapturing, at every update.  Results do not depend on the
 // class.
 constexpr double kSparseOcc2 = 1.5, kSparseOcc3 = 3.0;
+// The split kernel's line: a home's chain of neighbours on the staged kernel
+// (us a neighbour), the device's time for a pair at its full rate (1M 2D world:
+// 78 M pairs in 167 us), and what a launch of its own costs.  64 clustered
+// worlds of 1k to 8k particles, us a step: 427 -> 198 with worlds of 500
+// neighbours split, 868 -> 415 at 110 neighbours on average; before they
+// cluster 73 -> 92 where the line was 15 us, unchanged at 45.
+constexpr double kChainUs = 0.38, kPairUs = 2.1e-6, kSplitFloorUs = 45.0;
 
 void classify_worlds(plife_physics *h)
 {
@@ -1156,27 +1215,51 @@ void classify_worlds(plife_physics *h)
     const int mode = h->tune.sparse_worlds;
     const plife_tuning pt = plan_tuning(h);
     const double bs = pt.block_homes ? pt.block_homes : (h->clustered ? 128 : 256);
+    // neighbours per particle of each world's densest workgroup in the last
+    // measured step of the current table, and the step's pairs
+    double pairs = 0.0;
+    const int nb = h->nb_total;
+    const bool measured = nb > 0 && h->blocks_bs > 0 && h->blocks_version == h->version && h->work_host &&
+                          h->work_host_cap > (size_t)nb && (int)h->blocks.size() == nb &&
+                          __atomic_load_n(h->work_host + nb, __ATOMIC_RELAXED) == (uint32_t)(h->blocks_serial + 1);
+    if (measured) {
+        for (WorldHost &w : h->worlds) w.hot = 0.0;
+        for (int i = 0; i < nb; ++i) {
+            WorldHost &w = h->worlds[h->blocks[i].x];
+            const int first = (int)h->blocks[i].y - w.off;
+            const int homes = std::max(1, std::min(kind_homes(w.kind, h->blocks_bs), w.n - first));
+            w.hot = std::max(w.hot, (double)__atomic_load_n(h->work_host + i, __ATOMIC_RELAXED) / homes);
+        }
+    }
+    for (const WorldHost &w : h->worlds) pairs += std::max(w.nb, 0.0) * w.n;
+    // the split kernel has its own launch shape: a caller's shape means k_force
+    const plife_tuning &t = h->tune;
+    const bool shaped = t.block_homes || t.list_cap || t.stage_slack > 0.0 || t.windowed_only;
     bool changed = false;
     for (WorldHost &w : h->worlds) {
         const Grid gr = grid_of(w.st);
-        bool sparse;
+        int kind = kStaged;
         if (gr.nx < 3) {
-            sparse = true;
+            kind = kSparse;
         } else if (mode != 0) {
-            sparse = mode == 2;
+            kind = mode == 2 ? kSparse : kStaged;
         } else {
             const double r = w.st.rmax;
             const double cell = dim == 3 ? r * r * r : r * r;
             const double ball = dim == 3 ? 4.0 / 3.0 * M_PI * r * r * r : M_PI * r * r;
-            const double nb = w.nb >= 0.0 ? w.nb : std::max(w.n - 1, 0) * ball;
+            const double nb1 = w.nb >= 0.0 ? w.nb : std::max(w.n - 1, 0) * ball;
             const double avg = (double)w.n / (double)gr.ncells;
-            const double occ = std::max({avg, nb * cell / ball, 1e-9});
+            const double occ = std::max({avg, nb1 * cell / ball, 1e-9});
             const double span = bs / occ;              // cells spanned by a workgroup's homes
-            const double k = w.sparse ? 0.75 : 1.0;
-            sparse = occ * k < (dim == 3 ? kSparseOcc3 : kSparseOcc2) || NR * (span + 6.0) > 2048.0 * k;
+            const double k = w.kind == kSparse ? 0.75 : 1.0;
+            if (occ * k < (dim == 3 ? kSparseOcc3 : kSparseOcc2) || NR * (span + 6.0) > 2048.0 * k) kind = kSparse;
         }
-        if (sparse != w.sparse) {
-            w.sparse = sparse;
+        // the densest homes' chain against the whole launch at the device's rate
+        if (kind != kSparse && !shaped && mode == 0 && w.hot > 0.0 && w.nb >= 0.0 &&
+            w.hot * kChainUs * (w.kind == kSplit ? 1.25 : 1.0) > pairs * kPairUs + kSplitFloorUs)
+            kind = kSplit;
+        if (kind != w.kind) {
+            w.kind = kind;
             changed = true;
         }
     }
@@ -1316,6 +1399,7 @@ int prepare_step(plife_physics *h)
             }
     }
     h->plan = plan_force(h);
+    h->split = plan_split_for(h->dim == 3 ? 3 : 2, h->debug != 0, h->ntypes_max);
     if ((rc = ensure_cells(h, h->ncells))) return rc;
     if ((rc = ensure_debug(h))) return rc;
     // the one-launch step where it fits: forced by the tuning, or chosen by
@@ -1526,7 +1610,8 @@ std::vector<unsigned char> graph_key(const plife_physics *h)
         uint64_t version;
         plife_tuning tune;
         ForcePlan plan;
-        int seg[4];
+        SplitPlan split;
+        int seg[kSegments];
         int small, small_homes, small_kbuf, pad2;
         uint64_t blocks_serial;
         const void *ptr[40];
@@ -1541,6 +1626,7 @@ std::vector<unsigned char> graph_key(const plife_physics *h)
     k.version = h->version;
     k.tune = h->tune;
     k.plan = h->plan;
+    k.split = h->split;
     k.small = h->small ? 1 : 0;
     k.small_homes = h->small_homes;
     k.small_kbuf = h->small_kbuf;
@@ -2106,7 +2192,7 @@ int apply_preset(plife_physics *h, WorldHost &w, bool positions, int preset, uin
     else k_set_types<<<ceil_div(w.n, kBlock), kBlock, 0, h->stream>>>(g);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(h->stream));
-    w.nb = -1.0;             // the world's clustering is no longer known
+    w.nb = w.hot = -1.0;     // the world's clustering is no longer known
     if (!positions) w.max_type = w.ntypes - 1;
     h->stepped = false;      // cell by-products describe the old state
     return PLIFE_OK;
@@ -2371,7 +2457,7 @@ void reset_planner(plife_physics *h)
     std::memset(h->stat_host, 0, h->stat_cap * sizeof(uint64_t));
     h->occupancy = 0.0;
     h->clustered = false;
-    for (WorldHost &w : h->worlds) w.nb = -1.0;
+    for (WorldHost &w : h->worlds) w.nb = w.hot = -1.0;
 }
 
 int check_single(plife_physics *h)

@@ -153,26 +153,33 @@ __device__ __forceinline__ double pair_coef_sum(double d2, double mR, const Worl
     return fma(mR * g, y, rep);
 }
 
-// pair64 with no branch: the coefficient of a pair out of range (or
-// rejected by the caller, ok = false) is selected to 0, which leaves the sums
-// bit-identical (a sum that starts at +0 is never -0), so that the chains of
-// neighbouring candidates can overlap.
-template <int DIM, bool DEBUG, bool EXACT>
-__device__ __forceinline__ void pair64_sel(Acc &acc, bool ok, int dxi, int dyi, int dzi, double mR,
-                                           uint32_t qid, const WorldDev &a)
+// G lanes share a home (G = 4: a quad of lanes; G = 16: a row of 16): lane k of
+// the group holds candidate k's coefficient and difference, and every lane adds
+// the G terms in candidate order, acc = fma(c_k, D_k, acc) for k = 0 .. G-1,
+// each lane's values broadcast across the group by DPP -- the operations and
+// the order of one lane stepping them all (a term with c = 0 leaves a sum
+// unchanged: a sum that starts at +0 is never -0).
+template <int G, int K>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v)
 {
-    const double dx = (double)dxi, dy = (double)dyi, dz = (double)dzi;
-    const double d2 = pair_d2_of<DIM, EXACT>(dx, dy, dz);
-    const bool in = ok & (d2 != 0.0) & (d2 <= a.r2u);    // Physics.java:432
-    double cf = pair_coef_sum(d2, mR, a);
-    asm volatile("" : "+v"(cf));        // computed for every candidate: no branch
-    const double c = in ? cf : 0.0;
-    acc.x = fma(c, dx, acc.x);
-    acc.y = fma(c, dy, acc.y);
-    if constexpr (DIM == 3) acc.z = fma(c, dz, acc.z);
-    acc.cnt += in ? 1 : 0;
-    if constexpr (DEBUG)
-        if (in) acc.hash += id_hash(qid);
+    static_assert(G == 4 || G == 16, "groups are DPP quads or rows");
+    if constexpr (G == 4) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, K * 0x55, 0xf, 0xf, false);  // quad_perm:[K,K,K,K]
+    else return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + K, 0xf, 0xf, false);  // row_newbcast:K
+}
+
+template <int DIM, int G, int K = 0>
+__device__ __forceinline__ void group_terms(Acc &acc, double c, int dx, int dy, int dz)
+{
+    if constexpr (K < G) {
+        const unsigned long long cb = (unsigned long long)__double_as_longlong(c);
+        const unsigned long long kb = (unsigned long long)group_bcast<G, K>((uint32_t)cb) |
+                                      ((unsigned long long)group_bcast<G, K>((uint32_t)(cb >> 32)) << 32);
+        const double ck = __longlong_as_double((long long)kb);
+        acc.x = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dx), acc.x);
+        acc.y = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dy), acc.y);
+        if constexpr (DIM == 3) acc.z = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dz), acc.z);
+        group_terms<DIM, G, K + 1>(acc, c, dx, dy, dz);
+    }
 }
 
 // The block's pairs, for the host to order the next updates' blocks
@@ -530,31 +537,55 @@ __device__ __forceinline__ uint32_t low_bits(int n)
     return n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
 }
 
+// Staged candidate k against a home at (px, py, pz) with matrix row mrow: the
+// coefficient (0 when the pair does not interact or !ok) and the difference.
+// No branch, so that the chains of neighbouring candidates can overlap; a
+// coefficient of 0 leaves the sums bit-identical.
+template <int DIM, bool WRAP, bool MLDS, bool EXACT>
+__device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev &w, const Staged &s,
+                                              const double *M, int k, bool ok, uint32_t px, uint32_t py,
+                                              uint32_t pz, int mrow, int &dxi, int &dyi, int &dzi, bool &in)
+{
+    const uint2 hl = s.xy[k];
+    const uint32_t qx = join_x(hl), qy = join_y(hl), qz = DIM == 3 ? s.z[k] : 0u;
+    dxi = (int)(qx - px);
+    dyi = (int)(qy - py);
+    dzi = DIM == 3 ? (int)(qz - pz) : 0;
+    if constexpr (!WRAP) {
+        // plain difference of the clamped world: |D| >= 1/2 unless the
+        // int32 difference has the sign of the unsigned order
+        ok &= ((dxi >= 0) == (qx >= px)) & ((dyi >= 0) == (qy >= py));
+        if (DIM == 3) ok &= ((dzi >= 0) == (qz >= pz));
+    }
+    const int idx = mrow + (int)s.type[k];
+    const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
+    const double d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
+    in = ok & (d2 != 0.0) & (d2 <= w.r2u);               // Physics.java:432
+    double cf = pair_coef_sum(d2, m, w);
+    asm volatile("" : "+v"(cf));        // computed for every candidate: no branch
+    return in ? cf : 0.0;
+}
+
 // Phase B of one home at (px, py, pz) with matrix row mrow: its `left` kept
 // candidates, word by word in candidate order, two per iteration (half the
 // loop's bookkeeping; their force laws overlap).  load(m, kb) fetches the
 // next non-zero mask word and its first candidate.
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS, bool EXACT, typename Load>
 __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                          const double *M, Acc &ab, int left, Load &&load, uint32_t px,
-                                          uint32_t py, uint32_t pz, int mrow)
+                                             const double *M, Acc &ab, int left, Load &&load, uint32_t px,
+                                             uint32_t py, uint32_t pz, int mrow)
 {
-    // one candidate k: the reference's FP64 predicate and force law
     auto visit = [&](int k) {
-        const uint2 hl = s.xy[k];
-        const uint32_t qx = join_x(hl), qy = join_y(hl), qz = DIM == 3 ? s.z[k] : 0u;
-        const int dxi = (int)(qx - px), dyi = (int)(qy - py);
-        const int dzi = DIM == 3 ? (int)(qz - pz) : 0;
-        bool ok = true;
-        if constexpr (!WRAP) {
-            // plain difference of the clamped world: |D| >= 1/2 unless the
-            // int32 difference has the sign of the unsigned order
-            ok = ((dxi >= 0) == (qx >= px)) & ((dyi >= 0) == (qy >= py));
-            if (DIM == 3) ok &= ((dzi >= 0) == (qz >= pz));
-        }
-        const int idx = mrow + (int)s.type[k];
-        const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-        pair64_sel<DIM, DEBUG, EXACT>(ab, ok, dxi, dyi, dzi, m, DEBUG ? s.id[k] : 0u, w);
+        int dxi, dyi, dzi;
+        bool in;
+        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, true, px, py, pz, mrow, dxi, dyi,
+                                                             dzi, in);
+        ab.x = fma(c, (double)dxi, ab.x);
+        ab.y = fma(c, (double)dyi, ab.y);
+        if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);
+        ab.cnt += in ? 1 : 0;
+        if constexpr (DEBUG)
+            if (in) ab.hash += id_hash(s.id[k]);
     };
     uint32_t m = 0;
     int kb = 0;

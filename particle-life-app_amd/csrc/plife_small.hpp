@@ -153,29 +153,6 @@ __device__ __forceinline__ void small_run(const ForceArgs &a, const WorldDev &w,
 // never -0), so the sums are bit-identical, while one home's chain of
 // dependent loads and FP64 steps is shared by G lanes.  Interacting pairs
 // (and the debug hash) are counted per lane; the caller sums the group.
-template <int G, int K>
-__device__ __forceinline__ uint32_t group_bcast(uint32_t v)
-{
-    static_assert(G == 4 || G == 16, "groups are DPP quads or rows");
-    if constexpr (G == 4) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, K * 0x55, 0xf, 0xf, false);  // quad_perm:[K,K,K,K]
-    else return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + K, 0xf, 0xf, false);  // row_newbcast:K
-}
-
-template <int DIM, int G, int K = 0>
-__device__ __forceinline__ void group_terms(Acc &acc, double c, int dx, int dy, int dz)
-{
-    if constexpr (K < G) {
-        const unsigned long long cb = (unsigned long long)__double_as_longlong(c);
-        const unsigned long long kb = (unsigned long long)group_bcast<G, K>((uint32_t)cb) |
-                                      ((unsigned long long)group_bcast<G, K>((uint32_t)(cb >> 32)) << 32);
-        const double ck = __longlong_as_double((long long)kb);
-        acc.x = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dx), acc.x);
-        acc.y = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dy), acc.y);
-        if constexpr (DIM == 3) acc.z = fma(ck, (double)(int)group_bcast<G, K>((uint32_t)dz), acc.z);
-        group_terms<DIM, G, K + 1>(acc, c, dx, dy, dz);
-    }
-}
-
 template <int DIM, bool DEBUG, bool MLDS, int G>
 __device__ __forceinline__ void small_run_split(const ForceArgs &a, const WorldDev &w, bool wrap,
                                                 const double *M, const uint32_t *SX, const uint32_t *SY,
