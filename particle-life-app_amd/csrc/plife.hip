@@ -201,6 +201,8 @@ struct WorldHost {
 struct plife_physics {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t side_stream = nullptr;     // a second force launch of a step (launch_force_any)
+    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     bool batch = false;                // created by plife_batch_create
     bool have_settings = false;        // single-world handle: plife_set_settings was called
     int dim = 0;                       // shared by all worlds
@@ -761,6 +763,13 @@ int ensure_blocks(plife_physics *h, int bs)
     h->blocks_bs = bs;
     h->blocks_version = h->version;
     h->blocks_classes = h->classes;
+    int segments = 0;
+    for (const int nb : h->seg) segments += nb > 0;
+    if (segments > 1 && !h->side_stream) {
+        HIP_TRY(hipStreamCreateWithFlags(&h->side_stream, hipStreamNonBlocking));
+        HIP_TRY(hipEventCreateWithFlags(&h->fork_ev, hipEventDisableTiming));
+        HIP_TRY(hipEventCreateWithFlags(&h->join_ev, hipEventDisableTiming));
+    }
     return PLIFE_OK;
 }
 
@@ -858,50 +867,75 @@ void launch_split(plife_physics *h, ForceArgs a, int nblocks)
     else k_force_split<DIM, WRAP, DEBUG, false><<<nblocks, kSplitThreads, h->split.lds, h->stream>>>(a);
 }
 
-// One launch per segment of the block table present in the batch.
+// One segment of the block table on h->stream.
+int launch_segment(plife_physics *h, const ForceArgs &a, int s, int bs, size_t lds, bool dbg)
+{
+    const bool wrap = s < kForceKinds;
+    const int kind = s % kForceKinds, nb = h->seg[s];
+    if (kind == kSplit) {
+        if (h->dim == 3) {
+            if (wrap) dbg ? launch_split<3, true, true>(h, a, nb) : launch_split<3, true, false>(h, a, nb);
+            else dbg ? launch_split<3, false, true>(h, a, nb) : launch_split<3, false, false>(h, a, nb);
+        } else {
+            if (wrap) dbg ? launch_split<2, true, true>(h, a, nb) : launch_split<2, true, false>(h, a, nb);
+            else dbg ? launch_split<2, false, true>(h, a, nb) : launch_split<2, false, false>(h, a, nb);
+        }
+        LAUNCH_CHECK();
+        return PLIFE_OK;
+    }
+    if (kind == kSparse) {
+        if (h->dim == 3) {
+            if (wrap) dbg ? launch_sparse<3, true, true>(h, a, nb) : launch_sparse<3, true, false>(h, a, nb);
+            else dbg ? launch_sparse<3, false, true>(h, a, nb) : launch_sparse<3, false, false>(h, a, nb);
+        } else {
+            if (wrap) dbg ? launch_sparse<2, true, true>(h, a, nb) : launch_sparse<2, true, false>(h, a, nb);
+            else dbg ? launch_sparse<2, false, true>(h, a, nb) : launch_sparse<2, false, false>(h, a, nb);
+        }
+        LAUNCH_CHECK();
+        return PLIFE_OK;
+    }
+    if (h->dim == 3) {
+        if (wrap) dbg ? launch_force<3, true, true>(h, a, nb, bs, lds) : launch_force<3, true, false>(h, a, nb, bs, lds);
+        else dbg ? launch_force<3, false, true>(h, a, nb, bs, lds) : launch_force<3, false, false>(h, a, nb, bs, lds);
+    } else {
+        if (wrap) dbg ? launch_force<2, true, true>(h, a, nb, bs, lds) : launch_force<2, true, false>(h, a, nb, bs, lds);
+        else dbg ? launch_force<2, false, true>(h, a, nb, bs, lds) : launch_force<2, false, false>(h, a, nb, bs, lds);
+    }
+    LAUNCH_CHECK();
+    return PLIFE_OK;
+}
+
+// One launch per segment of the block table present in the batch.  The
+// segments step different worlds, so where there are several they go to the
+// handle's side stream in turn with its own, between a fork and a join: a
+// segment's last workgroups leave CUs that the next one's can use.  (A handle
+// without a side stream launches them in order.)
 int launch_force_any(plife_physics *h, ForceArgs a, int bs, size_t lds)
 {
     const bool dbg = h->debug != 0;
-    int base = 0;
-    for (int s = 0; s < kSegments; ++s) {
-        const bool wrap = s < kForceKinds;
-        const int kind = s % kForceKinds;
+    int base = 0, many = 0;
+    for (const int nb : h->seg) many += nb > 0;
+    const bool fork = many > 1 && h->join_ev;
+    hipStream_t const main_stream = h->stream;
+    if (fork) {
+        HIP_TRY(hipEventRecord(h->fork_ev, main_stream));
+        HIP_TRY(hipStreamWaitEvent(h->side_stream, h->fork_ev, 0));
+    }
+    int rc = PLIFE_OK, turn = 0;
+    for (int s = 0; s < kSegments && !rc; ++s) {
         const int nb = h->seg[s];
         a.block_base = base;
         base += nb;
         if (nb <= 0) continue;
-        if (kind == kSplit) {
-            if (h->dim == 3) {
-                if (wrap) dbg ? launch_split<3, true, true>(h, a, nb) : launch_split<3, true, false>(h, a, nb);
-                else dbg ? launch_split<3, false, true>(h, a, nb) : launch_split<3, false, false>(h, a, nb);
-            } else {
-                if (wrap) dbg ? launch_split<2, true, true>(h, a, nb) : launch_split<2, true, false>(h, a, nb);
-                else dbg ? launch_split<2, false, true>(h, a, nb) : launch_split<2, false, false>(h, a, nb);
-            }
-            LAUNCH_CHECK();
-            continue;
-        }
-        if (kind == kSparse) {
-            if (h->dim == 3) {
-                if (wrap) dbg ? launch_sparse<3, true, true>(h, a, nb) : launch_sparse<3, true, false>(h, a, nb);
-                else dbg ? launch_sparse<3, false, true>(h, a, nb) : launch_sparse<3, false, false>(h, a, nb);
-            } else {
-                if (wrap) dbg ? launch_sparse<2, true, true>(h, a, nb) : launch_sparse<2, true, false>(h, a, nb);
-                else dbg ? launch_sparse<2, false, true>(h, a, nb) : launch_sparse<2, false, false>(h, a, nb);
-            }
-            LAUNCH_CHECK();
-            continue;
-        }
-        if (h->dim == 3) {
-            if (wrap) dbg ? launch_force<3, true, true>(h, a, nb, bs, lds) : launch_force<3, true, false>(h, a, nb, bs, lds);
-            else dbg ? launch_force<3, false, true>(h, a, nb, bs, lds) : launch_force<3, false, false>(h, a, nb, bs, lds);
-        } else {
-            if (wrap) dbg ? launch_force<2, true, true>(h, a, nb, bs, lds) : launch_force<2, true, false>(h, a, nb, bs, lds);
-            else dbg ? launch_force<2, false, true>(h, a, nb, bs, lds) : launch_force<2, false, false>(h, a, nb, bs, lds);
-        }
-        LAUNCH_CHECK();
+        if (fork) h->stream = (turn++ & 1) ? h->side_stream : main_stream;
+        rc = launch_segment(h, a, s, bs, lds, dbg);
     }
-    return PLIFE_OK;
+    h->stream = main_stream;
+    if (fork) {                            // also after a failed launch: a capture must not end forked
+        HIP_TRY(hipEventRecord(h->join_ev, h->side_stream));
+        HIP_TRY(hipStreamWaitEvent(main_stream, h->join_ev, 0));
+    }
+    return rc;
 }
 
 // Events bracketing the phases of one step (optional).
@@ -940,10 +974,10 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
     // a workgroup takes the global path when its homes lie in more rows than the
     // part table holds: worlds of few cells per row take fewer homes (force
     // kernel, us, 64 / 128 / 256 homes: 1k particles in 20 x 20 cells 15.6 / 16.9
-    // / 27.4, in 13 x 13 17.8 / 18.8 / 37.5; 30k in 16^3 40 / 35 / 53; 300k in 42^3
-    // 168 / 112 / 167, in 33^3 186 / 132 / 108)
+    // / 27.4, in 13 x 13 17.8 / 18.8 / 37.5; 30k in 16^3 40 / 35 / 53), and small
+    // ones a little sooner, where more workgroups fill more CUs
     if (!t.block_homes && !clustered && nx > 0)
-        while (p.bs > 64 && p.bs / std::max(avg, 1e-9) > 1.5 * nx) p.bs /= 2;
+        while (p.bs > 64 && p.bs / std::max(avg, 1e-9) > (n <= 100000 ? 1.5 : 2.0) * nx) p.bs /= 2;
     // a workgroup of bs homes spans ~bs/avg + 1 cells of a row; it stages NR
     // rows of (span + 2) cells.  Clustered worlds keep a short cell table: the
     // few sparse workgroups that span more cells take the global path.
@@ -2448,6 +2482,9 @@ void destroy_handle(plife_physics *h)
         if (s.done) (void)hipEventDestroy(s.done);
         s = UploadSlot{};
     }
+    if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
+    if (h->join_ev) (void)hipEventDestroy(h->join_ev);
+    if (h->side_stream) (void)hipStreamDestroy(h->side_stream);
     if (h->stream) (void)hipStreamDestroy(h->stream);
 }
 
