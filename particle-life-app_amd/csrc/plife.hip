@@ -2752,7 +2752,7 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
         a.block_work = work;
         a.work_tag = 1u;
         a.nb_total = nblocks;
-        t.seg[s->wrap ? 0 : 2] = nblocks;
+        t.seg[(s->wrap ? 0 : kForceKinds) + kStaged] = nblocks;
         if ((rc = launch_force_any(&t, a, fp.bs, fp.lds))) return rc;
     }
     if (pairs) {
