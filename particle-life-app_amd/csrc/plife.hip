@@ -1281,7 +1281,10 @@ void classify_worlds(plife_physics *h)
             const double r = w.st.rmax;
             const double cell = dim == 3 ? r * r * r : r * r;
             const double ball = dim == 3 ? 4.0 / 3.0 * M_PI * r * r * r : M_PI * r * r;
-            const double nb1 = w.nb >= 0.0 ? w.nb : std::max(w.n - 1, 0) * ball;
+            // (a single world's clustering may be known ahead of its first step)
+            const double nb1 = w.nb >= 0.0                                      ? w.nb
+                               : h->worlds.size() == 1 && h->occupancy > 0.0 ? (h->occupancy - 1.0) * ball / cell
+                                                                             : std::max(w.n - 1, 0) * ball;
             const double avg = (double)w.n / (double)gr.ncells;
             const double occ = std::max({avg, nb1 * cell / ball, 1e-9});
             const double span = bs / occ;              // cells spanned by a workgroup's homes
@@ -1764,6 +1767,29 @@ int throttle(plife_physics *h, int k, int limit)
     return PLIFE_OK;
 }
 
+// The clustering measure of the current state, ahead of a step: bins and scans
+// it (as the step will again) and waits for the sum of the squared counts.
+int measure_cells(plife_physics *h)
+{
+    int rc;
+    const int nc = (int)h->ncells;
+    if (h->cells_dirty) {
+        k_fill_u32<<<ceil_div(nc, kBlock), kBlock, 0, h->stream>>>(h->cell_count, 0u, nc);
+        LAUNCH_CHECK();
+    }
+    h->cells_dirty = true;
+    if ((rc = bin_cells(h, h->dim, h->P(h->pc), h->n, h->worlds.size() > 1 ? h->world_of : nullptr,
+                        2 + (int)h->worlds.size(), h->version + 1, nullptr)))
+        return rc;
+    if ((rc = scan_cells(h, nc, h->d_pairs + 1))) return rc;
+    h->cells_dirty = false;
+    k_copy_u64<<<1, kBlock, 0, h->stream>>>(h->d_pairs + 1, h->stat_dev + 1, 1);
+    LAUNCH_CHECK();
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    h->stepped = false;                // the cell by-products are of no step
+    return PLIFE_OK;
+}
+
 // nsteps steps: pairs of steps replay a captured graph, the rest launch
 // directly.  A graph is captured once the same configuration comes back on a
 // second update (or when one update runs many steps); a configuration that
@@ -1785,12 +1811,18 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
         count_steps(h, steps);
         return bounded ? throttle(h, steps, limit) : PLIFE_OK;
     };
-    // The first update of a 3D handle: the launch plan follows the clustering
-    // of the cells, which only a step measures, so a long first update steps
-    // once, waits for that step's counters and re-plans the rest (C3: the
-    // clustered plan is 1.6x faster than the uniform one it would otherwise run).
-    if (h->dim == 3 && h->occupancy <= 0.0 && !h->small && nsteps - k >= 3 && h->n > 0 &&
-        h->tune.block_homes == 0) {
+    // The first update of a fresh state.  In 3D the launch plan follows the
+    // clustering of the cells: binned and scanned ahead of the first step, so
+    // that it need not run on the uniform plan (4M clustered world: 78 ms there,
+    // 31 on the clustered plan).  Then a long update steps once, waits for that
+    // step's counters and re-plans the rest from its neighbours per particle and
+    // per workgroup (a single world; a batch's updates do not wait).
+    const bool fresh = h->n > 0 && !h->small && h->tune.block_homes == 0;
+    if (fresh && h->dim == 3 && h->occupancy <= 0.0 && nsteps - k >= 3) {
+        if ((rc = measure_cells(h))) return rc;
+        if ((rc = prepare_step(h))) return rc;
+    }
+    if (fresh && !h->batch && h->worlds[0].nb < 0.0 && nsteps - k >= (h->dim == 3 ? 3 : 8)) {
         if (honour_stop && h->stop.load()) return PLIFE_STOPPED;
         if ((rc = do_step(h, nullptr))) return rc;
         ++k;
