@@ -488,15 +488,11 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     d.off = w.off;
     d.n = w.n;
     d.nx = gr.nx;
-    // the sums are in units of beta; a beta below 2^-33 has no particle pair
-    // closer than beta rmax (|D| >= 1, R <= 2^32) and scales by 1 instead
-    const double c = s.beta >= 0x1p-33 ? s.beta : 1.0;
-    d.mk = 2.0 * c / (1.0 - s.beta);
     // repeated stencil cells (Physics.java:377-395), or matrix entries whose
-    // product with mk is not finite: the summed force law needs finite ones
+    // product with R is not finite: the summed force law needs finite ones
     d.all_global = gr.nx < 3 ? 1 : 0;
     for (const double m : w.matrix)
-        if (!std::isfinite(m * d.mk)) d.all_global = 1;
+        if (!std::isfinite(m * R)) d.all_global = 1;
     d.exact_d2 = s.rmax <= 0x1p-6 ? 1 : 0;
     d.cell_base = cell_base;
     d.ntypes = w.ntypes;
@@ -512,11 +508,17 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     d.cs = s.rmax;
     d.ics = 1.0 / s.rmax;
     d.r2u = (s.rmax * s.rmax) * (kFix * kFix);         // Physics.java:432, exact 2^64 scaling
-    d.hR = 0.5 * R;
-    d.nbR = -0.5 * (s.beta * R);
+    d.S = 1.0 / R;
+    d.R = R;
+    d.beta = s.beta;
+    d.one_plus_beta = 1.0 + s.beta;
+    d.inv_1mb = 1.0 / (1.0 - s.beta);
+    d.inv_beta = 1.0 / s.beta;
+    d.m2S = -2.0 * d.S;
+    d.betaR = s.beta * R;
     d.ff = std::pow(s.friction, 60 * s.dt);            // Physics.java:401
-    d.ka = s.force * kInvFix / c;
-    d.kdt = s.force * s.dt / kFix / c;
+    d.ka = s.force * kInvFix;
+    d.kdt = s.force * s.dt / kFix;
     d.dt = s.dt;
     return d;
 }
@@ -2643,7 +2645,7 @@ int na_scratch_base(int dev, unsigned char **out)
 // slot of the workgroup work record, and the first ncells cell counts (a
 // previous call may have stopped between binning and the cell scan).
 // Block 0 also looks the matrix over (it is in device memory): entries that
-// are not finite times mk send the world down the literal path, as world_dev does.
+// are not finite times R send the world down the literal path, as world_dev does.
 __global__ void k_na_setup(WorldDev wd, const double *matrix, WorldDev *world, uint2 *blocks, int nblocks,
                            int bs, unsigned long long *counters, uint32_t *work, uint32_t *cell_count,
                            int ncells)
@@ -2651,7 +2653,7 @@ __global__ void k_na_setup(WorldDev wd, const double *matrix, WorldDev *world, u
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == 0) {
         bool bad = false;
-        for (int t = threadIdx.x; t < wd.ntypes * wd.ntypes; t += blockDim.x) bad |= !isfinite(matrix[t] * wd.mk);
+        for (int t = threadIdx.x; t < wd.ntypes * wd.ntypes; t += blockDim.x) bad |= !isfinite(matrix[t] * wd.R);
         if (__syncthreads_or(bad)) wd.all_global = 1;
         if (i == 0) *world = wd;
     }

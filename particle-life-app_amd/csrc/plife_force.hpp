@@ -79,10 +79,10 @@ __device__ __forceinline__ unsigned long long id_hash(uint32_t id)
 // the reference adds rel*(f/dist)*(rmax*force*dt) = D*(f/dist)*(force*dt) where
 //   f/dist = 1/beta - 1/dist                             (dist <  beta)
 //          = a*(1 - |1 + beta - 2 dist|/(1 - beta))/dist (dist >= beta)
-// (app/Main.java:275-280).  With v = 1/dist = R/|D| (R = rmax 2^32) these are
-//   s/beta and (2 a/(1 - beta)) min(s, v - 1),  s = 1 - beta v,
-// so acc accumulates c D*(f/dist) with c = beta (WorldDev::mk, kdt), in units
-// of 2^-32: s alone below beta, mk a min(s, v - 1) above it.
+// (app/Main.java:275-280).  acc accumulates D*(f/dist) in units of 2^-32.
+// With u = |D| = dist R (R = rmax 2^32) and y = 1/|D|: 1/dist = R y, and the
+// attractive branch is (a R) (1 - |1 + beta - 2 S u|/(1 - beta)) y, so the
+// caller passes mR = a * R (staged that way with the matrix).
 template <int DIM>
 __device__ __forceinline__ double pair_d2(double dx, double dy, double dz)
 {
@@ -91,34 +91,30 @@ __device__ __forceinline__ double pair_d2(double dx, double dy, double dz)
     return DIM == 3 ? dx * dx + (dy * dy + dz * dz) : dx * dx + dy * dy;
 }
 
-// s = 1 - beta v and t = v - 1 of the force law, from the squared distance:
-// 2/|D| by one Newton step from FP32, y0 (3 - d2 y0^2).
-__device__ __forceinline__ void pair_terms(double d2, const WorldDev &a, double &s, double &t)
+// f/dist of the force law for a pair in range (0 < d2 <= rmax^2).
+__device__ __forceinline__ double pair_coef(double d2, double mR, const WorldDev &a)
 {
     const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
     const double e = d2 * y0;
-    const double y = y0 * fma(-e, y0, 3.0);
-    s = fma(a.nbR, y, 1.0);
-    t = fma(a.hR, y, -1.0);
-}
-
-// c f/dist of the force law for a pair in range (0 < d2 <= rmax^2); m = mk a.
-__device__ __forceinline__ double pair_coef(double d2, double m, const WorldDev &a)
-{
-    double s, t;
-    pair_terms(d2, a, s, t);
-    return s < 0.0 ? s : m * fmin(fmax(fmin(s, t), 0.0), 1.0);
+    const double h = fma(-e, y0, 1.0);
+    const double y = fma(0.5 * y0, h, y0);        // 1/|D|, one Newton step from FP32
+    const double u = d2 * y;                       // |D| = dist R
+    const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
+    const double g = fma(t, -a.inv_1mb, 1.0);
+    const double att = (mR * g) * y;
+    const double rep = fma(-a.R, y, a.inv_beta);   // 1/beta - 1/dist
+    return u < a.betaR ? rep : att;
 }
 
 template <int DIM, bool DEBUG>
-__device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, double m, uint32_t qid,
+__device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, double mR, uint32_t qid,
                                        const WorldDev &a)
 {
     const double dx = (double)dxi, dy = (double)dyi, dz = (double)dzi;
     const double d2 = pair_d2<DIM>(dx, dy, dz);
     const bool in = (d2 != 0.0) & (d2 <= a.r2u);     // Physics.java:432
     if (in) {
-        const double c = pair_coef(d2, m, a);
+        const double c = pair_coef(d2, mR, a);
         acc.x = fma(c, dx, acc.x);
         acc.y = fma(c, dy, acc.y);
         if constexpr (DIM == 3) acc.z = fma(c, dz, acc.z);
@@ -138,19 +134,23 @@ __device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
     else return DIM == 3 ? fma(dx, dx, fma(dy, dy, dz * dz)) : fma(dx, dx, dy * dy);
 }
 
-// pair_coef with its branches summed in place of selected, for a finite m: of
-// min(s, 0) and max(min(s, t), 0) one is zero, so the FMA adds an exact zero
-// to the other branch's value.  No predicate either: past rmax t is not
-// positive and s is, so both are zero, and where d2 = 0 s and t are NaN, which
-// fmin and fmax drop.  (min(s, t) <= 1, so the clamp to [0, 1], free on its
-// instruction, is the max.)  With the Newton step, 8 FP64 instructions a
-// candidate in place of 14, a compare and two selects (1M 2D world, 32 steps:
-// 7.19 -> 6.89 ms).
-__device__ __forceinline__ double pair_coef_sum(double d2, double m, const WorldDev &a)
+// pair_coef with its branches summed in place of selected, for a finite mR:
+// below beta g is negative, at and above it 1/beta - 1/dist is not, so that of
+// max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
+// zero to the other branch's value -- two instructions where the compare, the
+// two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
+// free on its FMA, is max(g, 0).)
+__device__ __forceinline__ double pair_coef_sum(double d2, double mR, const WorldDev &a)
 {
-    double s, t;
-    pair_terms(d2, a, s, t);
-    return fma(m, fmin(fmax(fmin(s, t), 0.0), 1.0), fmin(s, 0.0));
+    const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
+    const double e = d2 * y0;
+    const double h = fma(-e, y0, 1.0);
+    const double y = fma(0.5 * y0, h, y0);
+    const double u = d2 * y;
+    const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
+    const double g = fmin(fmax(fma(t, -a.inv_1mb, 1.0), 0.0), 1.0);
+    const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);
+    return fma(mR * g, y, rep);
 }
 
 // G lanes share a home (G = 4: a quad of lanes; G = 16: a row of 16): lane k of
@@ -347,7 +347,7 @@ __device__ __forceinline__ void visit_run(const ForceArgs &a, const WorldDev &w,
             }
             if (!ok) continue;
             const int idx = row + (int)q[u].w;
-            const double m = MLDS ? Mlds[idx] : a.matrix[w.moff + idx] * w.mk;
+            const double m = MLDS ? Mlds[idx] : a.matrix[w.moff + idx] * w.R;
             pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m, DEBUG ? (uint32_t)a.id[a.perm[j]] : 0u, w);
         }
     }
@@ -483,23 +483,6 @@ __device__ __forceinline__ uint32_t stage_cells(const ForceArgs &a, const int (&
     return carry;
 }
 
-// A staged coordinate, and the difference of two.  Periodic worlds: the
-// coordinate itself; its differences modulo 2^32 are minimum-image differences.
-// Clamped worlds: with the top bit flipped, so that a saturating signed
-// subtraction gives the plain difference where |D| < 1/2 and +-2^31 where it is
-// not: past any rmax that has a staged grid (at most 1/3), with no sign test.
-template <bool WRAP>
-__device__ __forceinline__ uint32_t staged_axis(uint32_t x)
-{
-    return WRAP ? x : x ^ 0x80000000u;
-}
-template <bool WRAP>
-__device__ __forceinline__ int staged_diff(uint32_t q, uint32_t h)
-{
-    if constexpr (WRAP) return (int)(q - h);
-    else return __builtin_elementwise_sub_sat((int)q, (int)h);
-}
-
 // Staged candidates in LDS: high and low halves of x and y, z, type and
 // (debug) id.
 struct Staged {
@@ -510,7 +493,7 @@ struct Staged {
 
 // Stages entries [w0, w0 + wn) of the neighbourhood (nsegs segments) with T
 // threads: one 16-byte record read per entry.
-template <int DIM, bool WRAP, bool DEBUG, int T>
+template <int DIM, bool DEBUG, int T>
 __device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s, const uint2 *segs, int nsegs,
                                              int w0, int wn)
 {
@@ -524,9 +507,8 @@ __device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s
         }
         const uint32_t slot = sg + segs[lo].y;
         const uint4 q = a.rec[slot];
-        const uint32_t x = staged_axis<WRAP>(q.x), y = staged_axis<WRAP>(q.y);
-        s.xy[t] = make_uint2(high_halves(x, y), low_halves(x, y));
-        if constexpr (DIM == 3) s.z[t] = staged_axis<WRAP>(q.z);
+        s.xy[t] = make_uint2(high_halves(q.x, q.y), low_halves(q.x, q.y));
+        if constexpr (DIM == 3) s.z[t] = q.z;
         if constexpr (DEBUG) s.id[t] = (uint32_t)a.id[a.perm[slot]];
         s.type[t] = (uint8_t)q.w;
     }
@@ -555,52 +537,55 @@ __device__ __forceinline__ uint32_t low_bits(int n)
     return n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
 }
 
-// Staged candidate k against a home at (px, py, pz) (staged_axis) with matrix
-// row mrow: the coefficient (0 where the pair does not interact), the difference
-// and its square.
+// Staged candidate k against a home at (px, py, pz) with matrix row mrow: the
+// coefficient (0 when the pair does not interact or !ok) and the difference.
+// No branch, so that the chains of neighbouring candidates can overlap; a
+// coefficient of 0 leaves the sums bit-identical.
 template <int DIM, bool WRAP, bool MLDS, bool EXACT>
 __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                              const double *M, int k, uint32_t px, uint32_t py, uint32_t pz,
-                                              int mrow, int &dxi, int &dyi, int &dzi, double &d2)
+                                              const double *M, int k, bool ok, uint32_t px, uint32_t py,
+                                              uint32_t pz, int mrow, int &dxi, int &dyi, int &dzi, bool &in)
 {
     const uint2 hl = s.xy[k];
-    dxi = staged_diff<WRAP>(join_x(hl), px);
-    dyi = staged_diff<WRAP>(join_y(hl), py);
-    dzi = DIM == 3 ? staged_diff<WRAP>(s.z[k], pz) : 0;
+    const uint32_t qx = join_x(hl), qy = join_y(hl), qz = DIM == 3 ? s.z[k] : 0u;
+    dxi = (int)(qx - px);
+    dyi = (int)(qy - py);
+    dzi = DIM == 3 ? (int)(qz - pz) : 0;
+    if constexpr (!WRAP) {
+        // plain difference of the clamped world: |D| >= 1/2 unless the
+        // int32 difference has the sign of the unsigned order
+        ok &= ((dxi >= 0) == (qx >= px)) & ((dyi >= 0) == (qy >= py));
+        if (DIM == 3) ok &= ((dzi >= 0) == (qz >= pz));
+    }
     const int idx = mrow + (int)s.type[k];
-    const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.mk;
-    d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
-    return pair_coef_sum(d2, m, w);
+    const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
+    const double d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
+    in = ok & (d2 != 0.0) & (d2 <= w.r2u);               // Physics.java:432
+    double cf = pair_coef_sum(d2, m, w);
+    asm volatile("" : "+v"(cf));        // computed for every candidate: no branch
+    return in ? cf : 0.0;
 }
 
 // Phase B of one home at (px, py, pz) with matrix row mrow: its `left` kept
 // candidates, word by word in candidate order, two per iteration (half the
 // loop's bookkeeping; their force laws overlap).  load(m, kb) fetches the
-// next non-zero mask word and its first candidate.  ab.cnt counts the
-// lane's interacting pairs in debug mode; else, on the scalar unit, `loop`
-// those of all the wave's lanes while this lane is in the loop (the wave's
-// total is its largest) and ab.cnt the lane's odd last one.
+// next non-zero mask word and its first candidate.
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS, bool EXACT, typename Load>
 __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                             const double *M, Acc &ab, int &loop, int left, Load &&load, uint32_t px,
+                                             const double *M, Acc &ab, int left, Load &&load, uint32_t px,
                                              uint32_t py, uint32_t pz, int mrow)
 {
-    auto visit = [&](int k, bool last) {
+    auto visit = [&](int k) {
         int dxi, dyi, dzi;
-        double d2;
-        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, d2);
+        bool in;
+        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, true, px, py, pz, mrow, dxi, dyi,
+                                                             dzi, in);
         ab.x = fma(c, (double)dxi, ab.x);
         ab.y = fma(c, (double)dyi, ab.y);
         if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);
-        // Physics.java:432
-        if (DEBUG || last) {
-            const bool in = (d2 != 0.0) & (d2 <= w.r2u);
-            ab.cnt += in ? 1 : 0;
-            if constexpr (DEBUG)
-                if (in) ab.hash += id_hash(s.id[k]);
-        } else {
-            loop += __popcll(__ballot(d2 != 0.0) & __ballot(d2 <= w.r2u));
-        }
+        ab.cnt += in ? 1 : 0;
+        if constexpr (DEBUG)
+            if (in) ab.hash += id_hash(s.id[k]);
     };
     uint32_t m = 0;
     int kb = 0;
@@ -614,19 +599,19 @@ __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev 
     for (; left >= 2; left -= 2) {
         const int k1 = next();
         const int k2 = next();
-        visit(k1, false);
-        visit(k2, false);
+        visit(k1);
+        visit(k2);
     }
-    if (left > 0) visit(next(), true);
+    if (left > 0) visit(next());
 }
 
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS, typename Load>
 __device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                          const double *M, Acc &ab, int &loop, int left, Load &&load, uint32_t px,
+                                          const double *M, Acc &ab, int left, Load &&load, uint32_t px,
                                           uint32_t py, uint32_t pz, int mrow)
 {
-    if (w.exact_d2) walk_home_of<DIM, WRAP, DEBUG, MLDS, true>(a, w, s, M, ab, loop, left, load, px, py, pz, mrow);
-    else walk_home_of<DIM, WRAP, DEBUG, MLDS, false>(a, w, s, M, ab, loop, left, load, px, py, pz, mrow);
+    if (w.exact_d2) walk_home_of<DIM, WRAP, DEBUG, MLDS, true>(a, w, s, M, ab, left, load, px, py, pz, mrow);
+    else walk_home_of<DIM, WRAP, DEBUG, MLDS, false>(a, w, s, M, ab, left, load, px, py, pz, mrow);
 }
 
 // Counting sort of the HPT * T homes of a workgroup by their kept-candidate
@@ -759,7 +744,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     const int nact = min(BS, w.off + w.n - g0);
 
     if constexpr (MLDS)
-        for (int t = tid; t < w.ntypes * w.ntypes; t += BS) M[t] = a.matrix[w.moff + t] * w.mk;
+        for (int t = tid; t < w.ntypes * w.ntypes; t += BS) M[t] = a.matrix[w.moff + t] * w.R;
 
     // Thread tid stands for home g0 + tid (sorted order).  Parts: grid rows (2D:
     // cy; 3D: cy + cz*nx) and columns of the homes.
@@ -819,6 +804,11 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
 
     const int mrow = htype * w.ntypes;
 
+    // The force law's two additive constants held in VGPRs: each meets
+    // another scalar operand in an FMA, which reads one scalar at most.
+    WorldDev wf = w;
+    asm volatile("" : "+v"(wf.one_plus_beta));
+    asm volatile("" : "+v"(wf.inv_beta));
     const Staged stg{sxy, szz, sid, st};
 
     Acc acc;
@@ -843,8 +833,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
         if (cy == nx - 1) q2y = stencil_origin(hy, w.cs) == nx;
         if (DIM == 3 && cz == nx - 1) q2z = stencil_origin(hz, w.cs) == nx;
         const int j_lo = jh - 1 + (q2x ? 1 : 0);
-        const uint32_t bx = staged_axis<WRAP>(hx), by = staged_axis<WRAP>(hy), bz = staged_axis<WRAP>(hz);
-        const uint32_t hq = high_halves(bx, by);
+        const uint32_t hq = high_halves(hx, hy);
 
         // The home's run of stencil row r inside the window [w0, w0 + wn),
         // window-relative: returns its length, its first entry in lo.
@@ -887,7 +876,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                     uint32_t word = 0;
 #pragma unroll
                     for (int gq = 3; gq >= 0; --gq)
-                        if (i + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, bz, w.sbias, word);
+                        if (i + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, hz, w.sbias, word);
                     word &= low_bits(len - i);
                     if (word) {
                         wmask[at] = word;
@@ -900,18 +889,12 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             return npass;
         };
 
-        // this thread's share of the pairs walk_home counted
-        auto wave_pairs = [&](int loop, int cnt) -> unsigned long long {
-            const int most = wave_max(loop);
-            return (unsigned long long)cnt + (lane == 0 ? (unsigned long long)most : 0ull);
-        };
-
         const int S = (int)carry, nsegs = (int)nparts * NR * 3;
         if (a.wpool > 0 && S <= a.cap && place_words(0, S) <= (uint32_t)a.wpool) {
             // ---- one window ----------------------------------------------
             uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words);
             uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase);
-            stage_window<DIM, WRAP, DEBUG, BS>(a, stg, s_seg, nsegs, 0, S);
+            stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, 0, S);
             __syncthreads();
             const int count[1] = {screen_home(0, S, wmask, wbase)};
             int si = 0;
@@ -925,7 +908,6 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             // scan order, so its sums do not depend on the windows.
             deal_homes<BS, 1>(count, 0, s_bin, s_deal, s_cnt);
             const int h = (int)s_deal[tid];
-            int wloop = 0, wcnt = 0;
             if (h < nact) {
                 const int hsi = s_si[h];
                 const uint2 hhl = sxy[hsi];
@@ -937,17 +919,15 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 ab.cnt = 0;
                 ab.hash = 0ull;
                 int j = s_wo[h];
-                walk_home<DIM, WRAP, DEBUG, MLDS>(a, w, stg, M, ab, wloop, (int)s_hc[h], [&](uint32_t &m, int &kb) {
+                walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, (int)s_hc[h], [&](uint32_t &m, int &kb) {
                     m = wmask[j];
                     kb = wbase[j];
                     ++j;
                 }, hp.x, hp.y, bhz, btype * w.ntypes);
                 const int gh = g0 + h;
-                finish_home<DIM, WRAP, DEBUG>(a, w, ab, staged_axis<WRAP>(hp.x), staged_axis<WRAP>(hp.y),
-                                              staged_axis<WRAP>(bhz), btype, a.perm[gh], gh);
-                wcnt = ab.cnt;
+                finish_home<DIM, WRAP, DEBUG>(a, w, ab, hp.x, hp.y, bhz, btype, a.perm[gh], gh);
+                mycnt = (unsigned long long)ab.cnt;
             }
-            mycnt = wave_pairs(wloop, wcnt);
         } else {
             // ---- several windows -----------------------------------------
             // The staged neighbourhood streams through LDS in windows of at most
@@ -969,11 +949,11 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words2);
             uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase2);
             ax[tid] = ay[tid] = 0.0;
-            hxy[tid] = make_uint2(bx, by);
+            hxy[tid] = make_uint2(hx, hy);
             ht[tid] = (uint8_t)htype;
             if constexpr (DIM == 3) {
                 az[tid] = 0.0;
-                hzz[tid] = bz;
+                hzz[tid] = hz;
             }
             if constexpr (DEBUG) {
                 dhash[tid] = 0ull;
@@ -983,7 +963,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 // one entry needs a word per home at most, and wpool2 >= BS
                 int wn = min(a.cap, S - w0);
                 while (place_words(w0, wn) > (uint32_t)a.wpool2) wn = (wn + 1) >> 1;
-                stage_window<DIM, WRAP, DEBUG, BS>(a, stg, s_seg, nsegs, w0, wn);
+                stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, w0, wn);
                 __syncthreads();
                 const int count[1] = {screen_home(w0, wn, wmask, wbase)};
                 s_hc[tid] = (uint16_t)count[0];
@@ -992,7 +972,6 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 deal_homes<BS, 1>(count, shift, s_bin, s_deal, s_cnt);
                 const int h = (int)s_deal[tid];
                 const int left = (int)s_hc[h];
-                int wloop = 0, wcnt = 0;
                 if (left > 0) {
                     Acc ab;
                     ab.x = ax[h];
@@ -1002,7 +981,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                     ab.hash = 0ull;
                     const uint2 hp = hxy[h];
                     int j = s_wo[h];
-                    walk_home<DIM, WRAP, DEBUG, MLDS>(a, w, stg, M, ab, wloop, left, [&](uint32_t &m, int &kb) {
+                    walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, left, [&](uint32_t &m, int &kb) {
                         m = wmask[j];
                         kb = wbase[j];
                         ++j;
@@ -1014,9 +993,8 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                         dcnt[h] += ab.cnt;
                         dhash[h] += ab.hash;
                     }
-                    wcnt = ab.cnt;
+                    mycnt += (unsigned long long)ab.cnt;
                 }
-                mycnt += wave_pairs(wloop, wcnt);
                 __syncthreads();
                 w0 += wn;
             }
@@ -1076,7 +1054,7 @@ __global__ __launch_bounds__(kSparseBlock) void k_force_sparse(ForceArgs a)
     const uint2 bw = a.blocks[a.block_base + blk];
     const WorldDev w = a.worlds[bw.x];
     if constexpr (MLDS) {
-        for (int t = tid; t < w.ntypes * w.ntypes; t += kSparseBlock) M[t] = a.matrix[w.moff + t] * w.mk;
+        for (int t = tid; t < w.ntypes * w.ntypes; t += kSparseBlock) M[t] = a.matrix[w.moff + t] * w.R;
         __syncthreads();
     }
     const int g = (int)bw.y + tid;

@@ -137,14 +137,14 @@ struct WorldDev {
     int sbias;                       // screen bound on 16-bit coordinates: -(bq + 1) (screen_hi)
     double cs, ics;                  // cell size = rmax (Physics.java:312), and 1 / cs
     double r2u;                      // fl(rmax*rmax) * 2^64: the reference's bound in units 2^-64
-    // force law (pair_coef), with R = rmax 2^32 and c the scale of the sums
-    // (beta, or 1 where no distance is below beta rmax)
-    double hR;                       // R / 2
-    double nbR;                      // -beta R / 2
-    double mk;                       // 2 c / (1 - beta): factor of the matrix entries
+    double S;                        // 2^-32 / rmax: |rel| = |D| S with D in units 2^-32
+    double R;                        // rmax * 2^32:  1/|rel| = R / |D|
+    double beta, one_plus_beta, inv_1mb, inv_beta;
+    double m2S;                      // -2 S
+    double betaR;                    // beta R: |D| below it is the repulsion zone
     double ff;                       // friction^(60 dt) (host FP64 pow, Physics.java:401)
-    double kdt;                      // force * dt * 2^-32 / c
-    double ka;                       // force * 2^-32 / c: acceleration per unit of accumulated c D (f/dist)
+    double kdt;                      // force * dt * 2^-32
+    double ka;                       // force * 2^-32: acceleration per unit of accumulated D (f/dist)
     double dt;
 };
 

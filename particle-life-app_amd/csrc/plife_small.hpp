@@ -134,7 +134,7 @@ __device__ __forceinline__ void small_run(const ForceArgs &a, const WorldDev &w,
                 if (!ok) continue;
             }
             const int idx = row + ST[j];
-            const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.mk;
+            const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
             pair64<DIM, DEBUG>(acc, dxi, dyi, dzi, m,
                                DEBUG ? (uint32_t)a.id[w.off + min((int)(P[j] & 0xFFFFu), w.n - 1)] : 0u, w);
         }
@@ -166,7 +166,7 @@ __device__ __forceinline__ void small_run_split(const ForceArgs &a, const WorldD
         const int jc = min(j, hi - 1);
         const uint32_t qx = SX[jc], qy = SY[jc], qz = DIM == 3 ? SZ[jc] : 0u;
         const int idx = row + ST[jc];
-        const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.mk;
+        const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
         const int dxi = (int)(qx - hx), dyi = (int)(qy - hy);
         const int dzi = DIM == 3 ? (int)(qz - hz) : 0;
         bool in = j < hi;
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_step_small(SmallArgs s)
     const int nrounds = (n + kSmallL * kSmallThreads - 1) / (kSmallL * kSmallThreads);
 
     if constexpr (MLDS)
-        for (int t = tid; t < w.ntypes * w.ntypes; t += kSmallThreads) M[t] = a.matrix[w.moff + t] * w.mk;
+        for (int t = tid; t < w.ntypes * w.ntypes; t += kSmallThreads) M[t] = a.matrix[w.moff + t] * w.R;
 
     // 1. cell keys in the pre-sort order (Physics.java:362-375), packed with
     //    the index, and the previous step's keys of the same slots (O, in P1)

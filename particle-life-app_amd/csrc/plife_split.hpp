@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
     uint16_t *const list = reinterpret_cast<uint16_t *>(smem + L.list) + home * split_list_stride(a.cap);
 
     if constexpr (MLDS)
-        for (int t = tid; t < w.ntypes * w.ntypes; t += T) M[t] = a.matrix[w.moff + t] * w.mk;
+        for (int t = tid; t < w.ntypes * w.ntypes; t += T) M[t] = a.matrix[w.moff + t] * w.R;
 
     const bool active = home < nact;
     const int g = g0 + (active ? home : nact - 1);
@@ -147,19 +147,22 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
         if (cy == nx - 1) q2y = stencil_origin(hy, w.cs) == nx;
         if (DIM == 3 && cz == nx - 1) q2z = stencil_origin(hz, w.cs) == nx;
         const int j_lo = jh - 1 + (q2x ? 1 : 0);
-        const uint32_t bx = staged_axis<WRAP>(hx), by = staged_axis<WRAP>(hy), bz = staged_axis<WRAP>(hz);
-        const uint32_t hq = high_halves(bx, by);
+        const uint32_t hq = high_halves(hx, hy);
+        WorldDev wf = w;
+        asm volatile("" : "+v"(wf.one_plus_beta));
+        asm volatile("" : "+v"(wf.inv_beta));
+
         auto step_list = [&](auto exact, int n) {
             constexpr bool EXACT = decltype(exact)::value;
             auto coef = [&](int p, int &dx, int &dy, int &dz) -> double {
                 const int k = list[min(p, n - 1)];
-                double d2;
-                const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, stg, M, k, bx, by, bz, mrow, dx, dy, dz, d2);
-                const bool in = (p < n) & (d2 != 0.0) & (d2 <= w.r2u);      // Physics.java:432
+                bool in;
+                const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, p < n, hx, hy, hz, mrow, dx,
+                                                                     dy, dz, in);
                 acc.cnt += in ? 1 : 0;
                 if constexpr (DEBUG)
                     if (in) acc.hash += id_hash(stg.id[k]);
-                return p < n ? c : 0.0;
+                return c;
             };
 #pragma unroll 1
             for (int s = 0; s < n; s += 2 * G) {
@@ -173,7 +176,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
 
         for (int w0 = 0; w0 < S; w0 += a.cap) {
             const int wn = min(a.cap, S - w0);
-            stage_window<DIM, WRAP, DEBUG, T>(a, stg, s_seg, nsegs, w0, wn);
+            stage_window<DIM, DEBUG, T>(a, stg, s_seg, nsegs, w0, wn);
             __syncthreads();
             // ---- phase A: the home's kept candidates, in order, into its list
             int n = 0;
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
                     uint32_t word = 0;
 #pragma unroll
                     for (int gq = 3; gq >= 0; --gq)
-                        if (i0 + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, bz, w.sbias, word);
+                        if (i0 + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, hz, w.sbias, word);
                     word &= low_bits(len - i);
                     const uint32_t c = (uint32_t)__popc(word);
                     const uint32_t c0 = group_bcast<G, 0>(c), c1 = group_bcast<G, 1>(c), c2 = group_bcast<G, 2>(c),
