@@ -54,7 +54,7 @@ typedef struct {
 typedef struct {
     double step_ms;     /* wall time per step, event-to-event over all steps */
     double bin_ms;      /* cell keys + cell histogram + cell scan */
-    double sort_ms;     /* stable radix sort passes */
+    double sort_ms;     /* the stable counting sort */
     double gather_ms;   /* 0: the force kernel reads the pre-sort state through the permutation */
     double force_ms;    /* force + integrate kernel (average launch duration) */
     int64_t pairs;      /* interacting ordered pairs in the last step */

@@ -70,14 +70,18 @@ constexpr int kMaxTypes = 256;        // the app caps the matrix size at 256 (ap
 constexpr int kMaxTypesLds = 32;      // matrix staged in LDS up to 32x32 (8 KB of FP64)
 constexpr long long kMaxCells = 1LL << 28;
 constexpr int kMaxWorlds = 65535;     // the world index of a slot is a u16
-constexpr int kMaxLds = 65536;
+constexpr int kMaxLds = 81920;        // two workgroups a CU
 constexpr int kTuneSteps = 24;         // an update long enough to time two configurations
 constexpr int kTuneMax = 22;           // steps such a timing takes at most (4 x 4 + 3 switches + 3)
 constexpr size_t kWordLds = 32768;    // most LDS for the mask words of one window
+// Clustered 3D worlds of fewer particles take 128 homes per workgroup, so that
+// more workgroups fill the CUs (us a step, 128 / 256 homes: 200k 1466 / 1545, 500k
+// 1990 / 1947, 1M 1948 / 1993 and 911 / 826, 4M 31.3 / 28.1 ms).
+constexpr long long kClusteredWide = 1000000;
 constexpr double kStageSlack = 1.25, kPoolSlack = 1.1;   // over the expected staged entries and mask words
 constexpr double kMaxSlack = 1.6;     // over those, where LDS is free
 constexpr int kCus = 256;             // gfx950: CUs, LDS per CU, and what a workgroup uses besides the layout
-constexpr size_t kCuLds = 163840, kStaticLds = 5120;
+constexpr size_t kCuLds = 163840, kStaticLds = 2048, kLdsGrain = 1280;
 
 struct ForcePlan {
     int wpool = 0;                    // mask words per workgroup with one window (0: always several)
@@ -833,13 +837,24 @@ int sort_cells(plife_physics *h, int dim, const PosBuf &P, const int32_t *type, 
     return PLIFE_OK;
 }
 
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS, int BS>
+void launch_staged(plife_physics *h, const ForceArgs &a, int nblocks, size_t lds)
+{
+    // (a launch with more dynamic LDS than 64 KB needs the limit raised; an
+    // error shows at the launch)
+    if (lds > 65536)
+        (void)hipFuncSetAttribute((const void *)k_force<DIM, WRAP, DEBUG, MLDS, BS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    k_force<DIM, WRAP, DEBUG, MLDS, BS><<<nblocks, BS, lds, h->stream>>>(a);
+}
+
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS>
 void launch_force_bs(plife_physics *h, const ForceArgs &a, int nblocks, int bs, size_t lds)
 {
     switch (bs) {
-        case 64: k_force<DIM, WRAP, DEBUG, MLDS, 64><<<nblocks, 64, lds, h->stream>>>(a); break;
-        case 128: k_force<DIM, WRAP, DEBUG, MLDS, 128><<<nblocks, 128, lds, h->stream>>>(a); break;
-        default: k_force<DIM, WRAP, DEBUG, MLDS, 256><<<nblocks, 256, lds, h->stream>>>(a); break;
+        case 64: launch_staged<DIM, WRAP, DEBUG, MLDS, 64>(h, a, nblocks, lds); break;
+        case 128: launch_staged<DIM, WRAP, DEBUG, MLDS, 128>(h, a, nblocks, lds); break;
+        default: launch_staged<DIM, WRAP, DEBUG, MLDS, 256>(h, a, nblocks, lds); break;
     }
 }
 
@@ -959,18 +974,28 @@ int record(plife_physics *h, PhaseEvents *ev, int k)
 // cell a particle sits in) measured by an earlier step:
 //   * uniform worlds: 256 homes per workgroup and a staging buffer that holds
 //     the whole neighbourhood (one window);
-//   * clustered 3D worlds (occupancy far above the mean N / cells): 128 homes
-//     per workgroup and a small staging buffer, so that many workgroups share
+//   * clustered 3D worlds (occupancy far above the mean N / cells): 128 or 256
+//     homes per workgroup and a small staging buffer, so that many workgroups share
 //     a CU while the dense neighbourhoods stream through it in windows.
 // mixed: worlds of several densities share the launch.  The plan never changes
 // results: every home visits its candidates in the same order whatever the
 // windows and workgroup size.
+// Expected mask words of a stencil row run of `mean` candidates (Poisson).
+double run_words(double mean)
+{
+    const double dev = std::sqrt(std::max(mean, 1e-9));
+    if (mean > 40.0 * kWordCands) return mean / kWordCands + 0.5;
+    double sum = 0.0;                  // P(run > k words), k = 0, 1, ...: normal, with a continuity correction
+    for (int k = 0; k < 64; ++k) sum += 0.5 * std::erfc((k * kWordCands + 0.5 - mean) / (dev * std::sqrt(2.0)));
+    return sum;
+}
+
 ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustered, bool mixed,
                          const plife_tuning &t, bool dbg, int ntypes_max)
 {
     const int NR = dim == 3 ? 9 : 3;
     ForcePlan p;
-    p.bs = t.block_homes ? t.block_homes : (clustered ? 128 : 256);
+    p.bs = t.block_homes ? t.block_homes : (clustered && n < kClusteredWide ? 128 : 256);
     // a workgroup takes the global path when its homes lie in more rows than the
     // part table holds: worlds of few cells per row take fewer homes (force
     // kernel, us, 64 / 128 / 256 homes: 1k particles in 20 x 20 cells 15.6 / 16.9
@@ -991,24 +1016,25 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
     };
     auto entries = [&](double slack) {
         const long long want = (long long)std::ceil(NR * (span + 2.0) * avg * slack) + 64;
-        return std::min<long long>((want + 63) / 64 * 64, 65472);
+        return std::min<long long>((want + 63) / 64 * 64, kMaxStaged);
     };
     // One window (uniform worlds): a home's stencil row is a run of three cells,
-    // ~3 avg candidates, ceil(run / 32) mask words; the pool holds the expected
-    // total and some slack (workgroups needing more take several windows).
-    const double words = p.bs * NR * (3.0 * avg / 32.0 + 0.5);
+    // ~3 avg candidates, ceil(run / kWordCands) mask words; the pool holds the
+    // expected total and some slack (workgroups needing more take several windows).
+    const double words = p.bs * NR * run_words(3.0 * avg);
     auto pool = [&](double slack) { return (long long)std::ceil(words * slack) + 64; };
     long long want = 64;
-    if (!clustered && !t.windowed_only && pool(kPoolSlack) * 6 <= (long long)kWordLds) {
+    if (!clustered && !t.windowed_only && pool(kPoolSlack) * 4 <= (long long)kWordLds) {
         p.wpool = (int)pool(kPoolSlack);
         want = entries(t.stage_slack > 0.0 ? t.stage_slack : kStageSlack);
-        // A launch that leaves CUs room for all its workgroups at once pays
-        // nothing for a larger layout, and its time is that of its slowest
-        // workgroup: as much slack as fits, so that none takes several windows.
+        // LDS up to what the same number of workgroups on a CU (or all of the
+        // launch's, where that is fewer) can share costs nothing: as much slack
+        // as fits, so that fewer workgroups take several windows.
         if (t.stage_slack == 0.0 && n > 0) {
             const long long per_cu = (ceil_div(n, p.bs) + kCus - 1) / kCus;
-            const size_t room = std::min<size_t>(kMaxLds, kCuLds / (size_t)per_cu - kStaticLds);
-            for (double more = kMaxSlack; more > 1.0 && kCuLds / (size_t)per_cu > kStaticLds; more -= 0.05) {
+            const long long fit = std::max<long long>(1, (long long)(kCuLds / std::max<size_t>(total(p, want), 1)));
+            const size_t room = std::min<size_t>(kMaxLds, kCuLds / (size_t)std::min(per_cu, fit) / kLdsGrain * kLdsGrain);
+            for (double more = kMaxSlack; more > 1.0; more -= 0.05) {
                 ForcePlan q = p;
                 q.wpool = (int)pool(kPoolSlack * more);
                 const long long c = entries(kStageSlack * more);
@@ -1019,20 +1045,21 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
             }
         }
     }
-    // Several windows: mask words per home (32 candidates each).  Where one
+    // Several windows: mask words per home (in units of 32 candidates).  Where one
     // window is the rule (a single uniform world), no more than fit the space of
     // its pool: LDS per workgroup sets how many share a CU (1M 2D world: 0.218 ms
     // a step within the pool, 0.231 at 7 words).  Worlds of several densities in
     // one launch stream windows in the denser half of them: 9 words (512-world
-    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9).  Clustered worlds: 5 (4M
-    // 3D world: 35.1 ms at 5, 35.7 at 7, 36.5 at 9).
+    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9).  Clustered worlds: 7 (4M
+    // 3D world, 256 homes: 30.3 ms at 5, 28.1 at 7, 30.1 at 9; 1M, 128 homes: 1078
+    // us at 5, 911 at 7).
     const int fixed = force_home_bytes(dim, dbg);
-    const int fit = (int)(((long long)p.wpool * 6 / p.bs - fixed) / 6);
+    const int fit = (int)(((long long)p.wpool * 4 / p.bs - fixed) / 6.4);
     p.lcap = t.list_cap > 0 ? std::max(t.list_cap, 2)
-             : clustered    ? 5
+             : clustered    ? 7
                             : std::max(mixed || p.wpool == 0 ? 9 : 4, std::min(fit, 16));
-    p.lcap = std::min(p.lcap, 32768 / (6 * p.bs));                       // words stay within 32 KB of LDS
-    p.wpool2 = p.lcap * p.bs;
+    p.lcap = std::min(p.lcap, 32768 / (7 * p.bs));                       // words stay within 32 KB of LDS
+    p.wpool2 = ceil_div(32 * p.lcap, kWordCands) * p.bs;
     // where every workgroup streams windows, stage no more than its words cover
     if (p.wpool == 0) {
         want = (32ll * (p.lcap - 1) + 63) / 64 * 64;
@@ -1069,7 +1096,7 @@ SplitPlan plan_split_for(int dim, bool dbg, int ntypes_max)
     p.max_cells = dim == 3 ? 768 : 384;
     for (p.cap = kSplitWindow;; p.cap -= 32) {
         p.lds = split_lds_layout(dim, dbg, ntypes_max, ntypes_max <= kMaxTypesLds, p.cap, p.max_cells).total;
-        if (p.cap <= 64 || p.lds + kStaticLds <= (size_t)kMaxLds) return p;
+        if (p.cap <= 64 || p.lds + kStaticLds <= (size_t)65536) return p;
     }
 }
 
@@ -1089,7 +1116,10 @@ ForcePlan plan_force(const plife_physics *h)
         sn = h->n;
         sc = h->ncells;
     }
-    const double avg = (double)sn / (double)std::max(sc, 1LL);
+    // Where a single 3D world has drawn together, but not into clusters, the
+    // particles' own cells set a workgroup's neighbourhood, not the mean cell.
+    double avg = (double)sn / (double)std::max(sc, 1LL);
+    if (dim == 3 && !h->clustered && h->worlds.size() == 1) avg = std::max(avg, h->occupancy - 1.0);
     return plan_force_for(dim, avg, sn, nx, h->clustered, h->worlds.size() > 1, plan_tuning(h), h->debug != 0,
                           h->ntypes_max);
 }
@@ -1248,7 +1278,7 @@ void classify_worlds(plife_physics *h)
     const int NR = dim == 3 ? 9 : 3;
     const int mode = h->tune.sparse_worlds;
     const plife_tuning pt = plan_tuning(h);
-    const double bs = pt.block_homes ? pt.block_homes : (h->clustered ? 128 : 256);
+    const double bs = pt.block_homes ? pt.block_homes : (h->clustered && h->n < kClusteredWide ? 128 : 256);
     // neighbours per particle of each world's densest workgroup in the last
     // measured step of the current table, and the step's pairs
     double pairs = 0.0;

@@ -139,10 +139,12 @@ __device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
 // max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
 // zero to the other branch's value -- two instructions where the compare, the
 // two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
-// free on its FMA, is max(g, 0).)
+// free on its FMA, is max(g, 0).)  No predicate either: past rmax g is negative
+// and 1/beta - 1/dist is not, so both are zero; where d2 = 0 the square root's
+// argument of 1/2 keeps every term finite, and the difference it multiplies is 0.
 __device__ __forceinline__ double pair_coef_sum(double d2, double mR, const WorldDev &a)
 {
-    const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
+    const double y0 = (double)__builtin_amdgcn_rsqf(fmaxf((float)d2, 0.5f));
     const double e = d2 * y0;
     const double h = fma(-e, y0, 1.0);
     const double y = fma(0.5 * y0, h, y0);
@@ -409,7 +411,7 @@ __device__ void home_global(const ForceArgs &a, const WorldDev &w, const double 
 // p_base[q] on.  A workgroup's homes span a few consecutive cells of one grid
 // row, or (at row ends) of a few rows; each distinct row is a part.
 constexpr int kMaxParts = 4;
-constexpr int kScreenPad = 32;   // candidates a screen step reads from one base
+constexpr int kScreenPad = 40;   // candidates a screen step reads from one base, at most
 
 // A staged row's columns are consecutive cells, one run of the sorted order,
 // except where they wrap around the box in x: up to three runs (segments).
@@ -483,17 +485,56 @@ __device__ __forceinline__ uint32_t stage_cells(const ForceArgs &a, const int (&
     return carry;
 }
 
+// A staged coordinate, and the difference of two.  Periodic worlds: the
+// coordinate itself; its differences modulo 2^32 are minimum-image differences.
+// Clamped worlds: with the top bit flipped, so that a saturating signed
+// subtraction gives the plain difference where |D| < 1/2 and +-2^31 where it is
+// not: past any rmax that has a staged grid (at most 1/3), with no sign test.
+template <bool WRAP>
+__device__ __forceinline__ uint32_t staged_axis(uint32_t x)
+{
+    return WRAP ? x : x ^ 0x80000000u;
+}
+template <bool WRAP>
+__device__ __forceinline__ int staged_diff(uint32_t q, uint32_t h)
+{
+    if constexpr (WRAP) return (int)(q - h);
+    else return __builtin_elementwise_sub_sat((int)q, (int)h);
+}
+
 // Staged candidates in LDS: high and low halves of x and y, z, type and
 // (debug) id.
+struct StagedAt {                    // LDS addresses of entry 0, less 8 (xy) or 4 (z) times the types'
+    uint32_t type, xy, z;
+};
 struct Staged {
     uint2 *xy;
     uint32_t *z, *id;
     uint8_t *type;
+    StagedAt at;
 };
+
+#define PLIFE_LDS __attribute__((address_space(3)))
+template <typename T>
+__device__ __forceinline__ uint32_t lds_address(T *p)
+{
+    return (uint32_t)(uintptr_t)(PLIFE_LDS unsigned char *)(unsigned char *)p;
+}
+template <typename T>
+__device__ __forceinline__ T lds_read(uint32_t at)
+{
+    return *(PLIFE_LDS const T *)(uintptr_t)at;
+}
+
+__device__ __forceinline__ Staged staged_at(uint2 *xy, uint32_t *z, uint32_t *id, uint8_t *type)
+{
+    const uint32_t t = lds_address(type);
+    return Staged{xy, z, id, type, StagedAt{t, lds_address(xy) - 8u * t, lds_address(z) - 4u * t}};
+}
 
 // Stages entries [w0, w0 + wn) of the neighbourhood (nsegs segments) with T
 // threads: one 16-byte record read per entry.
-template <int DIM, bool DEBUG, int T>
+template <int DIM, bool WRAP, bool DEBUG, int T>
 __device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s, const uint2 *segs, int nsegs,
                                              int w0, int wn)
 {
@@ -507,8 +548,9 @@ __device__ __forceinline__ void stage_window(const ForceArgs &a, const Staged &s
         }
         const uint32_t slot = sg + segs[lo].y;
         const uint4 q = a.rec[slot];
-        s.xy[t] = make_uint2(high_halves(q.x, q.y), low_halves(q.x, q.y));
-        if constexpr (DIM == 3) s.z[t] = q.z;
+        const uint32_t x = staged_axis<WRAP>(q.x), y = staged_axis<WRAP>(q.y);
+        s.xy[t] = make_uint2(high_halves(x, y), low_halves(x, y));
+        if constexpr (DIM == 3) s.z[t] = staged_axis<WRAP>(q.z);
         if constexpr (DEBUG) s.id[t] = (uint32_t)a.id[a.perm[slot]];
         s.type[t] = (uint8_t)q.w;
     }
@@ -537,81 +579,88 @@ __device__ __forceinline__ uint32_t low_bits(int n)
     return n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
 }
 
-// Staged candidate k against a home at (px, py, pz) with matrix row mrow: the
-// coefficient (0 when the pair does not interact or !ok) and the difference.
-// No branch, so that the chains of neighbouring candidates can overlap; a
-// coefficient of 0 leaves the sums bit-identical.
+// Staged candidate at place k (the LDS address of its type, from which the
+// others follow in one instruction each) against a home at (px, py, pz)
+// (staged_axis) with matrix row mrow: the coefficient (0, or finite with a
+// difference of 0, where the pair does not interact), the difference and its
+// square.
 template <int DIM, bool WRAP, bool MLDS, bool EXACT>
 __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                              const double *M, int k, bool ok, uint32_t px, uint32_t py,
-                                              uint32_t pz, int mrow, int &dxi, int &dyi, int &dzi, bool &in)
+                                              const double *M, uint32_t k, uint32_t px, uint32_t py, uint32_t pz,
+                                              int mrow, int &dxi, int &dyi, int &dzi, double &d2)
 {
-    const uint2 hl = s.xy[k];
-    const uint32_t qx = join_x(hl), qy = join_y(hl), qz = DIM == 3 ? s.z[k] : 0u;
-    dxi = (int)(qx - px);
-    dyi = (int)(qy - py);
-    dzi = DIM == 3 ? (int)(qz - pz) : 0;
-    if constexpr (!WRAP) {
-        // plain difference of the clamped world: |D| >= 1/2 unless the
-        // int32 difference has the sign of the unsigned order
-        ok &= ((dxi >= 0) == (qx >= px)) & ((dyi >= 0) == (qy >= py));
-        if (DIM == 3) ok &= ((dzi >= 0) == (qz >= pz));
-    }
-    const int idx = mrow + (int)s.type[k];
+    const uint64_t xy = lds_read<uint64_t>(8u * k + s.at.xy);
+    const uint2 hl = make_uint2((uint32_t)xy, (uint32_t)(xy >> 32));
+    dxi = staged_diff<WRAP>(join_x(hl), px);
+    dyi = staged_diff<WRAP>(join_y(hl), py);
+    dzi = DIM == 3 ? staged_diff<WRAP>(lds_read<uint32_t>(4u * k + s.at.z), pz) : 0;
+    const int idx = mrow + (int)lds_read<uint8_t>(k);
     const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-    const double d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
-    in = ok & (d2 != 0.0) & (d2 <= w.r2u);               // Physics.java:432
-    double cf = pair_coef_sum(d2, m, w);
-    asm volatile("" : "+v"(cf));        // computed for every candidate: no branch
-    return in ? cf : 0.0;
+    d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
+    return pair_coef_sum(d2, m, w);
 }
 
+// Mask words: the top kWordCands bits one candidate each, first at the top, the
+// rest the first candidate's place.  Phase B needs a new word for some lane
+// nearly every candidate: one 4-byte read at a running address, where 32-bit
+// masks with a table of their bases took two reads at computed ones and 6 bytes
+// (force kernel, 1M 2D world 173 -> 165 us, 512-world batch 1740 -> 1619; with
+// 16-bit bases, 22% more LDS and a workgroup less on a CU, 1M 175).
+constexpr int kWordCands = 20, kPlaceBits = 32 - kWordCands;
+constexpr int kMaxStaged = (1 << kPlaceBits) - 64;    // places are below it: the types are at LDS address 0
+
 // Phase B of one home at (px, py, pz) with matrix row mrow: its `left` kept
-// candidates, word by word in candidate order, two per iteration (half the
-// loop's bookkeeping; their force laws overlap).  load(m, kb) fetches the
-// next non-zero mask word and its first candidate.
-template <int DIM, bool WRAP, bool DEBUG, bool MLDS, bool EXACT, typename Load>
+// candidates, word by word from `at` in candidate order, two per iteration (half
+// the loop's bookkeeping; their force laws overlap).  ab.cnt counts the lane's
+// interacting pairs in debug mode; else, on the scalar unit, `loop` those of all
+// the wave's lanes while this lane is in the loop (the wave's total is its
+// largest) and ab.cnt the lane's odd last one.
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS, bool EXACT>
 __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                             const double *M, Acc &ab, int left, Load &&load, uint32_t px,
-                                             uint32_t py, uint32_t pz, int mrow)
+                                             const double *M, Acc &ab, int &loop, int left, const uint32_t *at,
+                                             uint32_t px, uint32_t py, uint32_t pz, int mrow)
 {
-    auto visit = [&](int k) {
+    auto visit = [&](uint32_t k, bool last) {
         int dxi, dyi, dzi;
-        bool in;
-        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, true, px, py, pz, mrow, dxi, dyi,
-                                                             dzi, in);
+        double d2;
+        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, d2);
         ab.x = fma(c, (double)dxi, ab.x);
         ab.y = fma(c, (double)dyi, ab.y);
         if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);
-        ab.cnt += in ? 1 : 0;
-        if constexpr (DEBUG)
-            if (in) ab.hash += id_hash(s.id[k]);
+        // Physics.java:432
+        if (DEBUG || last) {
+            const bool in = (d2 != 0.0) & (d2 <= w.r2u);
+            ab.cnt += in ? 1 : 0;
+            if constexpr (DEBUG)
+                if (in) ab.hash += id_hash(s.id[k - s.at.type]);
+        } else {
+            loop += __popcll(__ballot(d2 != 0.0) & __ballot(d2 <= w.r2u));
+        }
     };
     uint32_t m = 0;
-    int kb = 0;
     auto next = [&]() {
-        if (m == 0) load(m, kb);
-        const int k = kb + __builtin_ctz(m);
-        m &= m - 1u;
-        return k;
+        if (m < (1u << kPlaceBits)) m = *at++;
+        const int b = __builtin_clz(m);
+        m ^= 0x80000000u >> b;
+        return (m & ((1u << kPlaceBits) - 1u)) + (uint32_t)b;
     };
 #pragma unroll 1
     for (; left >= 2; left -= 2) {
-        const int k1 = next();
-        const int k2 = next();
-        visit(k1);
-        visit(k2);
+        const uint32_t k1 = next();
+        const uint32_t k2 = next();
+        visit(k1, false);
+        visit(k2, false);
     }
-    if (left > 0) visit(next());
+    if (left > 0) visit(next(), true);
 }
 
-template <int DIM, bool WRAP, bool DEBUG, bool MLDS, typename Load>
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS>
 __device__ __forceinline__ void walk_home(const ForceArgs &a, const WorldDev &w, const Staged &s,
-                                          const double *M, Acc &ab, int left, Load &&load, uint32_t px,
-                                          uint32_t py, uint32_t pz, int mrow)
+                                          const double *M, Acc &ab, int &loop, int left, const uint32_t *at,
+                                          uint32_t px, uint32_t py, uint32_t pz, int mrow)
 {
-    if (w.exact_d2) walk_home_of<DIM, WRAP, DEBUG, MLDS, true>(a, w, s, M, ab, left, load, px, py, pz, mrow);
-    else walk_home_of<DIM, WRAP, DEBUG, MLDS, false>(a, w, s, M, ab, left, load, px, py, pz, mrow);
+    if (w.exact_d2) walk_home_of<DIM, WRAP, DEBUG, MLDS, true>(a, w, s, M, ab, loop, left, at, px, py, pz, mrow);
+    else walk_home_of<DIM, WRAP, DEBUG, MLDS, false>(a, w, s, M, ab, loop, left, at, px, py, pz, mrow);
 }
 
 // Counting sort of the HPT * T homes of a workgroup by their kept-candidate
@@ -657,28 +706,46 @@ __device__ __forceinline__ void deal_homes(const int (&count)[HPT], int shift, u
 // The LDS of a staged workgroup: `cap` staged entries at most; the windowed
 // path streams a denser neighbourhood through it.
 struct ForceLds {
-    size_t m, sxy, words, wbase, ax, ay, az, dhash, hxy, hz, dcnt, words2, wbase2, ht, sz, sid, off, st, total;
+    size_t st, m, sxy, words, ax, ay, az, dhash, hxy, hz, dcnt, words2, ht, sz, sid, off, fixed, total;
 };
 
 // Bytes per home that several windows keep in LDS besides the mask words: the
 // sums, the home's position and type, and (debug) its count and hash.
 constexpr int force_home_bytes(int dim, bool debug) { return dim * 8 + (dim == 3 ? 12 : 8) + 1 + (debug ? 12 : 0); }
 
-// A workgroup whose neighbourhood is one window has a pool of wpool mask words
-// (u32 bits + u16 first staged index); one that streams several windows keeps
-// the per-home data in the same region and a pool of wpool2 words.
+// LDS of a workgroup of BS homes whose size does not depend on the plan.
+template <int BS, int NR>
+struct ForceFixed {
+    uint2 seg[kMaxSegs * NR];
+    unsigned long long pairs[BS / kWave];
+    uint32_t bin[256];
+    uint32_t cnt[BS / kWave + 1];
+    int part[kMaxParts][3];            // row, first column, last column
+    uint16_t deal[BS];
+    uint16_t si[BS], hc[BS], wo[BS];   // per home: its staged index, kept candidates and first mask word
+};
+constexpr size_t force_fixed_bytes(int dim, int bs)
+{
+    return dim == 3 ? (bs == 64 ? sizeof(ForceFixed<64, 9>) : bs == 128 ? sizeof(ForceFixed<128, 9>) : sizeof(ForceFixed<256, 9>))
+                    : (bs == 64 ? sizeof(ForceFixed<64, 3>) : bs == 128 ? sizeof(ForceFixed<128, 3>) : sizeof(ForceFixed<256, 3>));
+}
+
+// A workgroup whose neighbourhood is one window has a pool of wpool mask words;
+// one that streams several windows keeps the per-home data in the same region
+// and a pool of wpool2 words.
 __host__ __device__ inline ForceLds force_lds_layout(int dim, bool debug, int ntypes, bool m_in_lds,
                                                      int cap, int bs, int max_cells, int wpool, int wpool2)
 {
     ForceLds L;
     size_t o = 0;
+    // the types first: a candidate's place is its type's address (kMaxStaged)
+    L.st = o;    o += ((size_t)cap + 7) & ~(size_t)7;
     L.m = o;     o += m_in_lds ? (size_t)ntypes * ntypes * 8 : 0;
     // the screened arrays carry kScreenPad spare entries: a screen step reads
-    // up to 32 candidates from one base, up to 31 past a lane's range
+    // up to that many candidates from one base, all but one past a lane's range
     L.sxy = o;   o += (size_t)(cap + kScreenPad) * 8;
     L.words = o;
-    L.wbase = o + (size_t)wpool * 4;
-    const size_t wend = o + (size_t)wpool * 6;
+    const size_t wend = o + (size_t)wpool * 4;
     L.ax = o;    o += (size_t)bs * 8;
     L.ay = o;    o += (size_t)bs * 8;
     L.az = o;    o += dim == 3 ? (size_t)bs * 8 : 0;
@@ -687,14 +754,14 @@ __host__ __device__ inline ForceLds force_lds_layout(int dim, bool debug, int nt
     L.hz = o;    o += dim == 3 ? (size_t)bs * 4 : 0;
     L.dcnt = o;  o += debug ? (size_t)bs * 4 : 0;
     L.words2 = o; o += (size_t)wpool2 * 4;
-    L.wbase2 = o; o += (size_t)wpool2 * 2;
     L.ht = o;    o += (size_t)bs;
     o = o > wend ? o : wend;
     o = (o + 3) & ~(size_t)3;
     L.sz = o;    o += dim == 3 ? (size_t)(cap + kScreenPad) * 4 : 0;
     L.sid = o;   o += debug ? (size_t)cap * 4 : 0;
     L.off = o;   o += (size_t)(max_cells + 1) * 4;
-    L.st = o;    o += (size_t)cap;
+    o = (o + 7) & ~(size_t)7;
+    L.fixed = o; o += force_fixed_bytes(dim, bs);
     L.total = (o + 15) & ~(size_t)15;
     return L;
 }
@@ -716,15 +783,6 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     constexpr int U = 8;                      // candidates per screen group
     constexpr int NW = BS / kWave;
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int s_part[kMaxParts][3];      // row, first column, last column
-    __shared__ uint32_t s_cnt[NW + 1];
-    __shared__ unsigned long long s_pairs[NW];
-    __shared__ uint16_t s_deal[BS];
-    // per home: its staged index, kept candidates and first mask word
-    __shared__ uint16_t s_si[BS], s_hc[BS], s_wo[BS];
-    __shared__ uint32_t s_bin[256];
-    __shared__ uint2 s_seg[kMaxSegs * NR];
-
     const ForceLds L = force_lds_layout(DIM, DEBUG, a.ntypes_max, MLDS, a.cap, BS, a.max_cells,
                                         a.wpool, a.wpool2);
     double *M = reinterpret_cast<double *>(smem + L.m);
@@ -732,7 +790,13 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     uint32_t *szz = reinterpret_cast<uint32_t *>(smem + L.sz);
     uint32_t *sid = reinterpret_cast<uint32_t *>(smem + L.sid);
     uint32_t *off = reinterpret_cast<uint32_t *>(smem + L.off);
-    uint8_t *st = reinterpret_cast<uint8_t *>(smem + L.st);
+    uint8_t *st = smem;                       // L.st
+    auto &fix = *reinterpret_cast<ForceFixed<BS, NR> *>(smem + L.fixed);
+    auto &s_part = fix.part;
+    uint32_t *const s_cnt = fix.cnt, *const s_bin = fix.bin;
+    unsigned long long *const s_pairs = fix.pairs;
+    uint16_t *const s_deal = fix.deal, *const s_si = fix.si, *const s_hc = fix.hc, *const s_wo = fix.wo;
+    uint2 *const s_seg = fix.seg;
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
     const int blk = xcd_remap(blockIdx.x, gridDim.x);
@@ -809,7 +873,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
     WorldDev wf = w;
     asm volatile("" : "+v"(wf.one_plus_beta));
     asm volatile("" : "+v"(wf.inv_beta));
-    const Staged stg{sxy, szz, sid, st};
+    const Staged stg = staged_at(sxy, szz, sid, st);
 
     Acc acc;
     acc.x = acc.y = acc.z = 0.0;
@@ -833,7 +897,8 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
         if (cy == nx - 1) q2y = stencil_origin(hy, w.cs) == nx;
         if (DIM == 3 && cz == nx - 1) q2z = stencil_origin(hz, w.cs) == nx;
         const int j_lo = jh - 1 + (q2x ? 1 : 0);
-        const uint32_t hq = high_halves(hx, hy);
+        const uint32_t bx = staged_axis<WRAP>(hx), by = staged_axis<WRAP>(hy), bz = staged_axis<WRAP>(hz);
+        const uint32_t hq = high_halves(bx, by);
 
         // The home's run of stencil row r inside the window [w0, w0 + wn),
         // window-relative: returns its length, its first entry in lo.
@@ -846,22 +911,23 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             return skip ? 0 : max(0, hi - lo);
         };
         // First mask word of each home in the pool (s_wo) for a window, a run of
-        // len candidates taking ceil(len / 32) words; returns the words needed.
+        // len candidates taking ceil(len / kWordCands) words; returns the words
+        // needed.
         auto place_words = [&](int w0, int wn) -> uint32_t {
             int need = 0;
 #pragma unroll 1
             for (int r = 0; r < NR; ++r) {
                 int lo;
-                need += (run_of(r, w0, wn, lo) + 31) >> 5;
+                need += (run_of(r, w0, wn, lo) + kWordCands - 1) / kWordCands;
             }
             uint32_t total = 0;
             s_wo[tid] = (uint16_t)block_excl_scan<BS>((uint32_t)need, s_cnt, total);
             return total;
         };
-        // Phase A: thread tid screens home tid; each 32 candidates of a row run
-        // give one mask word, stored (with its first candidate's index) when any
-        // candidate passed.  Returns the kept candidates.
-        auto screen_home = [&](int w0, int wn, uint32_t *wmask, uint16_t *wbase) -> int {
+        // Phase A: thread tid screens home tid; each 20 candidates of a row run
+        // give one mask word, stored when any candidate passed.  Returns the kept
+        // candidates.
+        auto screen_home = [&](int w0, int wn, uint32_t *wmask) -> int {
             int at = s_wo[tid], npass = 0;
 #pragma unroll 1
             for (int r = 0; r < NR; ++r) {
@@ -869,34 +935,46 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 const int len = run_of(r, w0, wn, klo);
                 const int K = wave_max(len);
 #pragma unroll 1
-                for (int i = 0; i < K; i += 4 * U) {
+                for (int i = 0; i < K; i += 2 * kWordCands) {
                     // a lane past its run reads the window's first entries
                     // (and keeps none of them)
                     const int kb = i < len ? klo + i : 0;
+                    auto put = [&](uint32_t word, int c) {
+                        word &= low_bits(len - i - c);
+                        if (word) {
+                            wmask[at] = __builtin_bitreverse32(word) | ((uint32_t)(kb + c) + stg.at.type);
+                            ++at;
+                            npass += __popc(word);
+                        }
+                    };
                     uint32_t word = 0;
-#pragma unroll
-                    for (int gq = 3; gq >= 0; --gq)
-                        if (i + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, hz, w.sbias, word);
-                    word &= low_bits(len - i);
-                    if (word) {
-                        wmask[at] = word;
-                        wbase[at] = (uint16_t)kb;
-                        ++at;
-                        npass += __popc(word);
+                    if (i + 16 < K) word = screen_group<DIM, 4>(stg, kb + 16, hq, bz, w.sbias, word);
+                    if (i + 8 < K) word = screen_group<DIM, U>(stg, kb + 8, hq, bz, w.sbias, word);
+                    put(screen_group<DIM, U>(stg, kb, hq, bz, w.sbias, word), 0);
+                    if (i + 20 < K) {
+                        word = 0;
+                        if (i + 36 < K) word = screen_group<DIM, 4>(stg, kb + 36, hq, bz, w.sbias, word);
+                        if (i + 28 < K) word = screen_group<DIM, U>(stg, kb + 28, hq, bz, w.sbias, word);
+                        put(screen_group<DIM, U>(stg, kb + 20, hq, bz, w.sbias, word), kWordCands);
                     }
                 }
             }
             return npass;
         };
 
+        // this thread's share of the pairs walk_home counted
+        auto wave_pairs = [&](int loop, int cnt) -> unsigned long long {
+            const int most = wave_max(loop);
+            return (unsigned long long)cnt + (lane == 0 ? (unsigned long long)most : 0ull);
+        };
+
         const int S = (int)carry, nsegs = (int)nparts * NR * 3;
         if (a.wpool > 0 && S <= a.cap && place_words(0, S) <= (uint32_t)a.wpool) {
             // ---- one window ----------------------------------------------
             uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words);
-            uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase);
-            stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, 0, S);
+            stage_window<DIM, WRAP, DEBUG, BS>(a, stg, s_seg, nsegs, 0, S);
             __syncthreads();
-            const int count[1] = {screen_home(0, S, wmask, wbase)};
+            const int count[1] = {screen_home(0, S, wmask)};
             int si = 0;
             if (active) {
                 const int f = pb + RMID * pw + jh;
@@ -908,6 +986,7 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             // scan order, so its sums do not depend on the windows.
             deal_homes<BS, 1>(count, 0, s_bin, s_deal, s_cnt);
             const int h = (int)s_deal[tid];
+            int wloop = 0, wcnt = 0;
             if (h < nact) {
                 const int hsi = s_si[h];
                 const uint2 hhl = sxy[hsi];
@@ -918,16 +997,14 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 ab.x = ab.y = ab.z = 0.0;
                 ab.cnt = 0;
                 ab.hash = 0ull;
-                int j = s_wo[h];
-                walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, (int)s_hc[h], [&](uint32_t &m, int &kb) {
-                    m = wmask[j];
-                    kb = wbase[j];
-                    ++j;
-                }, hp.x, hp.y, bhz, btype * w.ntypes);
+                walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, wloop, (int)s_hc[h], wmask + s_wo[h], hp.x, hp.y,
+                                                  bhz, btype * w.ntypes);
                 const int gh = g0 + h;
-                finish_home<DIM, WRAP, DEBUG>(a, w, ab, hp.x, hp.y, bhz, btype, a.perm[gh], gh);
-                mycnt = (unsigned long long)ab.cnt;
+                finish_home<DIM, WRAP, DEBUG>(a, w, ab, staged_axis<WRAP>(hp.x), staged_axis<WRAP>(hp.y),
+                                              staged_axis<WRAP>(bhz), btype, a.perm[gh], gh);
+                wcnt = ab.cnt;
             }
+            mycnt = wave_pairs(wloop, wcnt);
         } else {
             // ---- several windows -----------------------------------------
             // The staged neighbourhood streams through LDS in windows of at most
@@ -947,13 +1024,12 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
             uint32_t *const hzz = reinterpret_cast<uint32_t *>(smem + L.hz);
             uint8_t *const ht = smem + L.ht;
             uint32_t *const wmask = reinterpret_cast<uint32_t *>(smem + L.words2);
-            uint16_t *const wbase = reinterpret_cast<uint16_t *>(smem + L.wbase2);
             ax[tid] = ay[tid] = 0.0;
-            hxy[tid] = make_uint2(hx, hy);
+            hxy[tid] = make_uint2(bx, by);
             ht[tid] = (uint8_t)htype;
             if constexpr (DIM == 3) {
                 az[tid] = 0.0;
-                hzz[tid] = hz;
+                hzz[tid] = bz;
             }
             if constexpr (DEBUG) {
                 dhash[tid] = 0ull;
@@ -963,15 +1039,16 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                 // one entry needs a word per home at most, and wpool2 >= BS
                 int wn = min(a.cap, S - w0);
                 while (place_words(w0, wn) > (uint32_t)a.wpool2) wn = (wn + 1) >> 1;
-                stage_window<DIM, DEBUG, BS>(a, stg, s_seg, nsegs, w0, wn);
+                stage_window<DIM, WRAP, DEBUG, BS>(a, stg, s_seg, nsegs, w0, wn);
                 __syncthreads();
-                const int count[1] = {screen_home(w0, wn, wmask, wbase)};
+                const int count[1] = {screen_home(w0, wn, wmask)};
                 s_hc[tid] = (uint16_t)count[0];
                 int shift = 0;
                 while ((wn >> shift) > 256) ++shift;
                 deal_homes<BS, 1>(count, shift, s_bin, s_deal, s_cnt);
                 const int h = (int)s_deal[tid];
                 const int left = (int)s_hc[h];
+                int wloop = 0, wcnt = 0;
                 if (left > 0) {
                     Acc ab;
                     ab.x = ax[h];
@@ -980,12 +1057,8 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                     ab.cnt = 0;
                     ab.hash = 0ull;
                     const uint2 hp = hxy[h];
-                    int j = s_wo[h];
-                    walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, left, [&](uint32_t &m, int &kb) {
-                        m = wmask[j];
-                        kb = wbase[j];
-                        ++j;
-                    }, hp.x, hp.y, DIM == 3 ? hzz[h] : 0u, (int)ht[h] * w.ntypes);
+                    walk_home<DIM, WRAP, DEBUG, MLDS>(a, wf, stg, M, ab, wloop, left, wmask + s_wo[h], hp.x, hp.y,
+                                                      DIM == 3 ? hzz[h] : 0u, (int)ht[h] * w.ntypes);
                     ax[h] = ab.x;
                     ay[h] = ab.y;
                     if constexpr (DIM == 3) az[h] = ab.z;
@@ -993,8 +1066,9 @@ __global__ __launch_bounds__(BS) void k_force(ForceArgs a)
                         dcnt[h] += ab.cnt;
                         dhash[h] += ab.hash;
                     }
-                    mycnt += (unsigned long long)ab.cnt;
+                    wcnt = ab.cnt;
                 }
+                mycnt += wave_pairs(wloop, wcnt);
                 __syncthreads();
                 w0 += wn;
             }

@@ -104,7 +104,7 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, int n)
 }
 
 // The last step's counters to the host's pinned copy (the step after copies
-// them itself, in k_bin_tile).
+// them itself, in k_bin).
 __global__ void k_copy_u64(const unsigned long long *__restrict__ src, unsigned long long *__restrict__ dst,
                            int n)
 {

@@ -66,8 +66,8 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
 
     const SplitLds L = split_lds_layout(DIM, DEBUG, a.ntypes_max, MLDS, a.cap, a.max_cells);
     double *const M = reinterpret_cast<double *>(smem + L.m);
-    const Staged stg{reinterpret_cast<uint2 *>(smem + L.xy), reinterpret_cast<uint32_t *>(smem + L.z),
-                     reinterpret_cast<uint32_t *>(smem + L.id), smem + L.type};
+    const Staged stg = staged_at(reinterpret_cast<uint2 *>(smem + L.xy), reinterpret_cast<uint32_t *>(smem + L.z),
+                                 reinterpret_cast<uint32_t *>(smem + L.id), smem + L.type);
     uint32_t *const off = reinterpret_cast<uint32_t *>(smem + L.off);
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
@@ -147,7 +147,8 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
         if (cy == nx - 1) q2y = stencil_origin(hy, w.cs) == nx;
         if (DIM == 3 && cz == nx - 1) q2z = stencil_origin(hz, w.cs) == nx;
         const int j_lo = jh - 1 + (q2x ? 1 : 0);
-        const uint32_t hq = high_halves(hx, hy);
+        const uint32_t bx = staged_axis<WRAP>(hx), by = staged_axis<WRAP>(hy), bz = staged_axis<WRAP>(hz);
+        const uint32_t hq = high_halves(bx, by);
         WorldDev wf = w;
         asm volatile("" : "+v"(wf.one_plus_beta));
         asm volatile("" : "+v"(wf.inv_beta));
@@ -155,14 +156,15 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
         auto step_list = [&](auto exact, int n) {
             constexpr bool EXACT = decltype(exact)::value;
             auto coef = [&](int p, int &dx, int &dy, int &dz) -> double {
-                const int k = list[min(p, n - 1)];
-                bool in;
-                const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, p < n, hx, hy, hz, mrow, dx,
-                                                                     dy, dz, in);
+                const uint32_t k = list[min(p, n - 1)];
+                double d2;
+                const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, bx, by, bz, mrow, dx, dy, dz,
+                                                                     d2);
+                const bool in = (p < n) & (d2 != 0.0) & (d2 <= w.r2u);      // Physics.java:432
                 acc.cnt += in ? 1 : 0;
                 if constexpr (DEBUG)
-                    if (in) acc.hash += id_hash(stg.id[k]);
-                return c;
+                    if (in) acc.hash += id_hash(stg.id[k - stg.at.type]);
+                return p < n ? c : 0.0;
             };
 #pragma unroll 1
             for (int s = 0; s < n; s += 2 * G) {
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
 
         for (int w0 = 0; w0 < S; w0 += a.cap) {
             const int wn = min(a.cap, S - w0);
-            stage_window<DIM, DEBUG, T>(a, stg, s_seg, nsegs, w0, wn);
+            stage_window<DIM, WRAP, DEBUG, T>(a, stg, s_seg, nsegs, w0, wn);
             __syncthreads();
             // ---- phase A: the home's kept candidates, in order, into its list
             int n = 0;
@@ -195,14 +197,15 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
                     uint32_t word = 0;
 #pragma unroll
                     for (int gq = 3; gq >= 0; --gq)
-                        if (i0 + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, hz, w.sbias, word);
+                        if (i0 + gq * U < K) word = screen_group<DIM, U>(stg, kb + gq * U, hq, bz, w.sbias, word);
                     word &= low_bits(len - i);
                     const uint32_t c = (uint32_t)__popc(word);
                     const uint32_t c0 = group_bcast<G, 0>(c), c1 = group_bcast<G, 1>(c), c2 = group_bcast<G, 2>(c),
                                    c3 = group_bcast<G, 3>(c);
                     int at = n + (int)((sub > 0 ? c0 : 0u) + (sub > 1 ? c1 : 0u) + (sub > 2 ? c2 : 0u));
+                    const uint32_t ka = (uint32_t)kb + stg.at.type;
                     while (word) {
-                        list[at++] = (uint16_t)(kb + __builtin_ctz(word));
+                        list[at++] = (uint16_t)(ka + (uint32_t)__builtin_ctz(word));
                         word &= word - 1u;
                     }
                     n += (int)(c0 + c1 + c2 + c3);
