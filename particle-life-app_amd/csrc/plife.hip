@@ -81,6 +81,7 @@ constexpr long long kClusteredWide = 1000000;
 constexpr double kStageSlack = 1.25, kPoolSlack = 1.1;   // over the expected staged entries and mask words
 constexpr double kMaxSlack = 1.6;     // over those, where LDS is free
 constexpr int kCus = 256;             // gfx950: CUs, LDS per CU, and what a workgroup uses besides the layout
+constexpr int kSnakeRounds = 4;       // blocks of a launch on a CU at once that balance_blocks counts on
 constexpr size_t kCuLds = 163840, kStaticLds = 2048, kLdsGrain = 1280;
 
 struct ForcePlan {
@@ -991,7 +992,7 @@ double run_words(double mean)
 }
 
 ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustered, bool mixed,
-                         const plife_tuning &t, bool dbg, int ntypes_max)
+                         const plife_tuning &t, bool dbg, int ntypes_max, size_t max_lds = kMaxLds)
 {
     const int NR = dim == 3 ? 9 : 3;
     ForcePlan p;
@@ -1033,7 +1034,7 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
         if (t.stage_slack == 0.0 && n > 0) {
             const long long per_cu = (ceil_div(n, p.bs) + kCus - 1) / kCus;
             const long long fit = std::max<long long>(1, (long long)(kCuLds / std::max<size_t>(total(p, want), 1)));
-            const size_t room = std::min<size_t>(kMaxLds, kCuLds / (size_t)std::min(per_cu, fit) / kLdsGrain * kLdsGrain);
+            const size_t room = std::min<size_t>(max_lds, kCuLds / (size_t)std::min(per_cu, fit) / kLdsGrain * kLdsGrain);
             for (double more = kMaxSlack; more > 1.0; more -= 0.05) {
                 ForcePlan q = p;
                 q.wpool = (int)pool(kPoolSlack * more);
@@ -1050,14 +1051,16 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
     // its pool: LDS per workgroup sets how many share a CU (1M 2D world: 0.218 ms
     // a step within the pool, 0.231 at 7 words).  Worlds of several densities in
     // one launch stream windows in the denser half of them: 9 words (512-world
-    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9).  Clustered worlds: 7 (4M
+    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9), all of them in a single
+    // dense world: 16 (us a step at 9 / 16 words: 3D 300k of 65 a cell 1094 / 848, 2D 1M of
+    // 100 a cell 1037 / 932, clustered 196k 1870 / 1780).  Clustered worlds: 7 (4M
     // 3D world, 256 homes: 30.3 ms at 5, 28.1 at 7, 30.1 at 9; 1M, 128 homes: 1078
     // us at 5, 911 at 7).
     const int fixed = force_home_bytes(dim, dbg);
     const int fit = (int)(((long long)p.wpool * 4 / p.bs - fixed) / 6.4);
     p.lcap = t.list_cap > 0 ? std::max(t.list_cap, 2)
              : clustered    ? 7
-                            : std::max(mixed || p.wpool == 0 ? 9 : 4, std::min(fit, 16));
+                            : std::max(mixed ? 9 : p.wpool == 0 ? 16 : 4, std::min(fit, 16));
     p.lcap = std::min(p.lcap, 32768 / (7 * p.bs));                       // words stay within 32 KB of LDS
     p.wpool2 = ceil_div(32 * p.lcap, kWordCands) * p.bs;
     // where every workgroup streams windows, stage no more than its words cover
@@ -1067,9 +1070,9 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
     }
     // keep room for a useful staging window: shrink the cell table first
     const long long min_cap = std::min<long long>(want, 256);
-    while (p.max_cells > 64 && total(p, min_cap) > kMaxLds) p.max_cells = std::max(64, p.max_cells * 3 / 4);
+    while (p.max_cells > 64 && total(p, min_cap) > max_lds) p.max_cells = std::max(64, p.max_cells * 3 / 4);
     // then shrink the staging capacity until the layout fits the LDS budget
-    while (want > 64 && total(p, want) > kMaxLds) want -= 64;
+    while (want > 64 && total(p, want) > max_lds) want -= 64;
     p.cap = (int)want;
     p.lds = total(p, p.cap);
     return p;
@@ -1120,7 +1123,12 @@ ForcePlan plan_force(const plife_physics *h)
     // particles' own cells set a workgroup's neighbourhood, not the mean cell.
     double avg = (double)sn / (double)std::max(sc, 1LL);
     if (dim == 3 && !h->clustered && h->worlds.size() == 1) avg = std::max(avg, h->occupancy - 1.0);
-    return plan_force_for(dim, avg, sn, nx, h->clustered, h->worlds.size() > 1, plan_tuning(h), h->debug != 0,
+    // (a single 2D world that has clustered and does not fit the CUs at once is
+    // planned as a batch of worlds of several densities: 800k particles of 1,200
+    // neighbours 2.62 ms, 3.00 as one dense world)
+    const bool mixed = h->worlds.size() > 1 ||
+                       (dim == 2 && h->occupancy > 2.0 * (avg + 1.0) && sn > (long long)kSnakeRounds * kCus * 256);
+    return plan_force_for(dim, avg, sn, nx, h->clustered, mixed, plan_tuning(h), h->debug != 0,
                           h->ntypes_max);
 }
 
@@ -1228,8 +1236,15 @@ int balance_blocks(plife_physics *h)
         std::vector<uint2> blk(n);
         std::vector<uint64_t> key(n);
         std::vector<uint32_t> est(n);
+        // a launch whose blocks are all on the CUs at once gives each CU one block
+        // a round: every other round in reverse, so that the CU with the heaviest
+        // of one round has the lightest of the next (dense 196k 2D world: 2.20 -> 1.87
+        // ms a step)
+        const bool snake = n <= kSnakeRounds * kCus;
         for (int i = 0; i < n; ++i) {
-            const int to = remap_pos(i, n), from = b0 + order[i];
+            const int round = i / kCus, width = std::min(kCus, n - round * kCus), k = i % kCus;
+            const int at = snake && (round & 1) ? round * kCus + width - 1 - k : i;
+            const int to = remap_pos(at, n), from = b0 + order[i];
             blk[to] = h->blocks[from];
             key[to] = h->block_key[from];
             est[to] = work[from];
@@ -1265,12 +1280,15 @@ int balance_blocks(plife_physics *h)
 // class.
 constexpr double kSparseOcc2 = 1.5, kSparseOcc3 = 3.0;
 // The split kernel's line: a home's chain of neighbours on the staged kernel
-// (us a neighbour), the device's time for a pair at its full rate (1M 2D world:
-// 78 M pairs in 167 us), and what a launch of its own costs.  64 clustered
+// (us a neighbour) against the device's time for a pair on the split kernel at
+// its full rate (dense 196k 2D world: 459 M pairs in 2.1 ms) and what a launch of
+// its own costs (us a step, staged / split, clustered worlds: 2D 50k particles of
+// 300 neighbours 307 / 180, 100k of 1000 1116 / 773, 300k of 500 735 / 1000, 196k
+// of 2300 1872 / 2200; 3D 60k of 400 630 / 400).  64 clustered
 // worlds of 1k to 8k particles, us a step: 427 -> 198 with worlds of 500
 // neighbours split, 868 -> 415 at 110 neighbours on average; before they
 // cluster 73 -> 92 where the line was 15 us, unchanged at 45.
-constexpr double kChainUs = 0.38, kPairUs = 2.1e-6, kSplitFloorUs = 45.0;
+constexpr double kChainUs = 0.28, kPairUs = 4.5e-6, kSplitFloorUs = 45.0;
 
 void classify_worlds(plife_physics *h)
 {
@@ -1321,7 +1339,7 @@ void classify_worlds(plife_physics *h)
             const double k = w.kind == kSparse ? 0.75 : 1.0;
             if (occ * k < (dim == 3 ? kSparseOcc3 : kSparseOcc2) || NR * (span + 6.0) > 2048.0 * k) kind = kSparse;
         }
-        // the densest homes' chain against the whole launch at the device's rate
+        // the densest homes' chain against the whole launch at the split kernel's rate
         if (kind != kSparse && !shaped && mode == 0 && w.hot > 0.0 && w.nb >= 0.0 &&
             w.hot * kChainUs * (w.kind == kSplit ? 1.25 : 1.0) > pairs * kPairUs + kSplitFloorUs)
             kind = kSplit;
@@ -1849,6 +1867,7 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
     // per workgroup (a single world; a batch's updates do not wait).
     const bool fresh = h->n > 0 && !h->small && h->tune.block_homes == 0;
     if (fresh && h->dim == 3 && h->occupancy <= 0.0 && nsteps - k >= 3) {
+        if (honour_stop && h->stop.load()) return PLIFE_STOPPED;
         if ((rc = measure_cells(h))) return rc;
         if ((rc = prepare_step(h))) return rc;
     }
@@ -2738,7 +2757,8 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
     const WorldDev wd = world_dev(wh, 0u, 0);
     const int nc = (int)gr.ncells;
     const double avg = (double)n / (double)nc;
-    const ForcePlan fp = plan_force_for(s->dim, avg, n, gr.nx, false, false, plife_tuning{}, false, ntypes);
+    // (at most 64 KB of LDS: more needs a call that a capture may not take)
+    const ForcePlan fp = plan_force_for(s->dim, avg, n, gr.nx, false, false, plife_tuning{}, false, ntypes, 65536);
     const int nblocks = ceil_div(n, fp.bs);
 
     // a transient view of the scratch as the step helpers' buffers (no
