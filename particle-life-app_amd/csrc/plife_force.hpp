@@ -13,9 +13,8 @@
 //
 // Each home particle runs two phases over its candidates:
 //   A  integer screen on the high 16 bits of the coordinates (screen_hi).  Kept
-//      candidates become bits of mask words in LDS, or indices appended to a
-//      per-thread list.
-//   B  For listed candidates only: the reference's predicate in FP64
+//      candidates become bits of mask words in LDS.
+//   B  For kept candidates only: the reference's predicate in FP64
 //      (d2 = dx*dx + dy*dy, d2 != 0 && d2 <= rmax*rmax; Physics.java:430-432) and
 //      the force law in FP64 (FP64 FMA issues at the non-packed FP32 rate on
 //      CDNA4), accumulated in FP64.

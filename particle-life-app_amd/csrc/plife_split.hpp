@@ -4,7 +4,7 @@
 // Reference: backend/Physics.java:397-450 (updateVelocity, updatePosition).
 //
 // A home's candidates are added in order, so one lane steps them as a chain:
-// about 0.38 us a neighbour on k_force.  Where a launch holds few particles
+// about 0.28 us a neighbour on k_force.  Where a launch holds few particles
 // with thousands of neighbours (a small world that has clustered), that chain
 // and not the device's rate is the step's time.  Here four lanes share a home:
 // a workgroup of 256 threads owns 64 homes and streams their neighbourhood
@@ -16,7 +16,7 @@
 //      and every lane adds their terms in candidate order (group_terms).
 // The sums stay in registers from window to window.  These are k_force's
 // operations in its order: the bits do not change.  The instructions per pair
-// grow by about two thirds, which a launch that leaves most of the device idle
+// are 2.1 times k_force's, which a launch that leaves most of the device idle
 // does not notice (classify_worlds).
 #pragma once
 
