@@ -383,7 +383,10 @@ void free_state(plife_physics *h)
 }
 
 // Room for `need` particles.  With keep, the particles in the first h->used
-// slots of the current buffers move to the new buffers.
+// slots of the current buffers move to the new buffers.  Where the state's
+// arrays cannot be had, the handle keeps the old ones.  Where the sort's
+// cannot (the old ones are gone by then, so that they need not fit together),
+// its particles stay with keep, and are none without.
 int ensure_capacity(plife_physics *h, int need, bool keep)
 {
     if (need <= h->cap && h->cap > 0) return PLIFE_OK;
@@ -438,11 +441,21 @@ int ensure_capacity(plife_physics *h, int need, bool keep)
     }
     h->pc = 0;
     h->ac = 0;
-    if ((rc = dev_alloc(&h->keys0, cap))) return rc;
-    if ((rc = dev_alloc(&h->kA, (size_t)cap + kRankPad))) return rc;
-    if ((rc = dev_alloc(&h->perm, cap))) return rc;
-    if ((rc = dev_alloc(&h->rec, cap))) return rc;
-    if ((rc = dev_alloc(&h->skeys, cap))) return rc;
+    if (!rc) rc = dev_alloc(&h->keys0, cap);
+    if (!rc) rc = dev_alloc(&h->kA, (size_t)cap + kRankPad);
+    if (!rc) rc = dev_alloc(&h->perm, cap);
+    if (!rc) rc = dev_alloc(&h->rec, cap);
+    if (!rc) rc = dev_alloc(&h->skeys, cap);
+    if (rc) {
+        // h->cap stays 0: no step runs (prepare_step) until a later call has it all
+        h->stepped = false;
+        if (!keep) {
+            for (WorldHost &w : h->worlds) w.n = 0;
+            h->used = 0;
+            h->layout_dirty = true;
+        }
+        return rc;
+    }
     h->cap = cap;
     return PLIFE_OK;
 }
@@ -1471,6 +1484,8 @@ int prepare_step(plife_physics *h)
                         "world %d: particle types reach %d but the matrix has %d types; set particles "
                         "with types below the matrix size before stepping", w.id, w.max_type, w.ntypes);
     if ((rc = sync_layout(h))) return rc;
+    if (h->n > h->cap)
+        return fail(PLIFE_ERR_MEMORY, "the sort's buffers for %d particles could not be allocated", h->n);
     refresh_occupancy(h);
     classify_worlds(h);
     // a layout of a class measured before takes that class's homes per workgroup
