@@ -1831,7 +1831,8 @@ int throttle(plife_physics *h, int k, int limit)
 }
 
 // The clustering measure of the current state, ahead of a step: bins and scans
-// it (as the step will again) and waits for the sum of the squared counts.
+// it (as the step will again) and waits for the sum of the squared counts.  The
+// other counters are of no step, so their tag is none of a layout's.
 int measure_cells(plife_physics *h)
 {
     int rc;
@@ -1842,7 +1843,7 @@ int measure_cells(plife_physics *h)
     }
     h->cells_dirty = true;
     if ((rc = bin_cells(h, h->dim, h->P(h->pc), h->n, h->worlds.size() > 1 ? h->world_of : nullptr,
-                        2 + (int)h->worlds.size(), h->version + 1, nullptr)))
+                        2 + (int)h->worlds.size(), 0ull, nullptr)))
         return rc;
     if ((rc = scan_cells(h, nc, h->d_pairs + 1))) return rc;
     h->cells_dirty = false;
@@ -1877,9 +1878,10 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
     // The first update of a fresh state.  In 3D the launch plan follows the
     // clustering of the cells: binned and scanned ahead of the first step, so
     // that it need not run on the uniform plan (4M clustered world: 78 ms there,
-    // 31 on the clustered plan).  Then a long update steps once, waits for that
-    // step's counters and re-plans the rest from its neighbours per particle and
-    // per workgroup (a single world; a batch's updates do not wait).
+    // 31 on the clustered plan).  Then a single world's long update steps once,
+    // waits for that step's counters and re-plans the rest from its neighbours per
+    // particle and per workgroup.  (Both wait for the stream; a batch's later
+    // updates, and a 2D batch's first, do not.)
     const bool fresh = h->n > 0 && !h->small && h->tune.block_homes == 0;
     if (fresh && h->dim == 3 && h->occupancy <= 0.0 && nsteps - k >= 3) {
         if (honour_stop && h->stop.load()) return PLIFE_STOPPED;

@@ -186,12 +186,36 @@ void failed_growth()
         }
 }
 
+// What measure_cells leaves in the counters is of no step: while the device is
+// at the first step's binning, a 3D batch's neighbours are still unknown.
+void measured_cells_are_no_step()
+{
+    plife_batch *b = nullptr;
+    const plife_settings s = settings(3, 0.1);
+    const plife_tuning t{0, 0, 1, 0.0, 0, 0, 1};        // direct launches, multi-launch path
+    int32_t id;
+    CHECK(plife_batch_create(0, &b) == PLIFE_OK && plife_batch_set_tuning(b, &t) == PLIFE_OK);
+    CHECK(plife_batch_add_generated_world(b, &s, 2, kMatrix, 20000, 1, &id) == PLIFE_OK);
+    int bins = 0;
+    fake::device = [&](const std::string &name, void **a) {
+        if (bins >= 2) return;
+        bins += fake::has(name, "k_bin");
+        fake::counters(name, a);
+    };
+    CHECK(plife_batch_update(b, 3) == PLIFE_OK);
+    CHECK(fake::count("k_bin") == 4);                    // the measurement's and three steps'
+    CHECK(plife_batch_update(b, 1) == PLIFE_OK);
+    CHECK(b->worlds[0].nb < 0.0);
+    plife_batch_destroy(b);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
+        {"measured_cells_are_no_step", measured_cells_are_no_step},
     };
     const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
     if (it == cases.end()) return 2;
