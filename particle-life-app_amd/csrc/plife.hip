@@ -1832,7 +1832,8 @@ int throttle(plife_physics *h, int k, int limit)
 
 // The clustering measure of the current state, ahead of a step: bins and scans
 // it (as the step will again) and waits for the sum of the squared counts.  The
-// other counters are of no step, so their tag is none of a layout's.
+// other counters are of no step, so their tag is none of a layout's.  Only where
+// no step has run on the state: it overwrites a step's exports.
 int measure_cells(plife_physics *h)
 {
     int rc;
@@ -1850,7 +1851,6 @@ int measure_cells(plife_physics *h)
     k_copy_u64<<<1, kBlock, 0, h->stream>>>(h->d_pairs + 1, h->stat_dev + 1, 1);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(h->stream));
-    h->stepped = false;                // the cell by-products are of no step
     return PLIFE_OK;
 }
 
@@ -1878,14 +1878,16 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
     // The first update of a fresh state.  In 3D the launch plan follows the
     // clustering of the cells: binned and scanned ahead of the first step, so
     // that it need not run on the uniform plan (4M clustered world: 78 ms there,
-    // 31 on the clustered plan).  Then a single world's long update steps once,
-    // waits for that step's counters and re-plans the rest from its neighbours per
-    // particle and per workgroup.  (Both wait for the stream; a batch's later
-    // updates, and a 2D batch's first, do not.)
+    // 31 on the clustered plan).  (A step may have run whose counters have not
+    // arrived yet: they are waited for, and its exports stay.)  Then a single
+    // world's long update steps once, waits for that step's counters and re-plans
+    // the rest from its neighbours per particle and per workgroup.  (Both wait
+    // for the stream; a batch's later updates, and a 2D batch's first, do not.)
     const bool fresh = h->n > 0 && !h->small && h->tune.block_homes == 0;
     if (fresh && h->dim == 3 && h->occupancy <= 0.0 && nsteps - k >= 3) {
         if (honour_stop && h->stop.load()) return PLIFE_STOPPED;
-        if ((rc = measure_cells(h))) return rc;
+        if (h->stepped) HIP_TRY(hipStreamSynchronize(h->stream));
+        else if ((rc = measure_cells(h))) return rc;
         if ((rc = prepare_step(h))) return rc;
     }
     if (fresh && !h->batch && h->worlds[0].nb < 0.0 && nsteps - k >= (h->dim == 3 ? 3 : 8)) {

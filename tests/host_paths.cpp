@@ -209,6 +209,25 @@ void measured_cells_are_no_step()
     plife_batch_destroy(b);
 }
 
+// A stop that arrives before an update's first step leaves the last step's
+// exports, also where that step's counters have not reached the host yet.
+void stopped_update_keeps_the_last_step()
+{
+    plife_physics *h = engine(3, 0.1, 20000, plife_tuning{0, 0, 1, 0.0, 0, 0, 1});
+    CHECK(plife_update(h, 1) == PLIFE_OK);               // (the device has copied no counters)
+    fake::device = [&](const std::string &name, void **) {
+        if (fake::has(name, "k_bin")) CHECK(plife_force_update_stop(h) == PLIFE_OK);
+    };
+    int64_t steps = 0;
+    CHECK(plife_update(h, 8) == PLIFE_STOPPED);
+    CHECK(plife_get_steps(h, &steps) == PLIFE_OK && steps >= 1);
+    int32_t ncells = 0;
+    std::vector<int32_t> end(1000);
+    CHECK(plife_get_grid(h, nullptr, &ncells) == PLIFE_OK && ncells == 1000);
+    CHECK(plife_get_cells(h, nullptr, end.data(), nullptr, ncells) == PLIFE_OK);
+    plife_destroy(h);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -216,6 +235,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
+        {"stopped_update_keeps_the_last_step", stopped_update_keeps_the_last_step},
     };
     const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
     if (it == cases.end()) return 2;

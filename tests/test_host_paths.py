@@ -21,7 +21,10 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["failed_growth", "measured_cells_are_no_step"])
+CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step"]
+
+
+@pytest.mark.parametrize("case", CASES)
 def test_host_path(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
