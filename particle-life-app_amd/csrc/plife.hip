@@ -709,6 +709,16 @@ int sync_layout(plife_physics *h)
 // Homes per workgroup of a force kernel; bs: the staged kernel's.
 int kind_homes(int kind, int bs) { return kind == kSparse ? kSparseBlock : kind == kSplit ? kSplitHomes : bs; }
 
+// Pairs expected of `homes` homes of a world: its measured neighbours, or a
+// uniform world's.
+uint32_t expected_pairs(const WorldHost &w, int homes)
+{
+    const double r = w.st.rmax;
+    const double ball = w.st.dim == 3 ? 4.0 / 3.0 * M_PI * r * r * r : M_PI * r * r;
+    const double nb = w.nb >= 0.0 ? w.nb : std::max(w.n - 1, 0) * ball;
+    return (uint32_t)std::min(nb * std::max(homes, 0), 4.0e9);
+}
+
 // Force workgroup table: segments of periodic staged, sparse and split worlds,
 // then clamped ones (one launch each).
 int ensure_blocks(plife_physics *h, int bs)
@@ -734,18 +744,13 @@ int ensure_blocks(plife_physics *h, int bs)
             const WorldHost &wh = h->worlds[w];
             if ((wh.st.wrap != 0) != wrap || wh.kind != kind) continue;
             const int step = kind_homes(kind, bs);
-            // expected pairs per home where no measurement carries over
-            const double r = wh.st.rmax;
-            const double ball = wh.st.dim == 3 ? 4.0 / 3.0 * M_PI * r * r * r : M_PI * r * r;
-            const double nb = wh.nb >= 0.0 ? wh.nb : std::max(wh.n - 1, 0) * ball;
             for (int g = 0; g < wh.n; g += step) {
                 const uint64_t key = ((uint64_t)(uint32_t)wh.id << 33) | ((uint64_t)kind << 31) | (uint32_t)g;
                 const auto it = prev.find(key);
-                const double homes = std::min(step, wh.n - g);
                 h->blocks.push_back(make_uint2((uint32_t)w, (uint32_t)(wh.off + g)));
                 h->block_key.push_back(key);
                 h->block_est.push_back(it != prev.end() ? it->second
-                                                        : (uint32_t)std::min(nb * homes, 4.0e9));
+                                                        : expected_pairs(wh, std::min(step, wh.n - g)));
             }
         }
         h->seg[s] = (int)(h->blocks.size() - before);
@@ -2295,6 +2300,27 @@ int generate_particles(plife_physics *h, int off, int n, uint64_t seed, int ntyp
     return PLIFE_OK;
 }
 
+// World w's particles have new positions: forgets what steps measured of the
+// old ones, its neighbours and its workgroups' pairs.  The stream is idle.
+int forget_world(plife_physics *h, WorldHost &w)
+{
+    w.nb = w.hot = -1.0;
+    for (size_t i = 0; i < h->block_key.size() && h->blocks_bs > 0; ++i) {
+        if ((int32_t)(h->block_key[i] >> 33) != w.id) continue;
+        const int first = (int)(h->block_key[i] & 0x7FFFFFFF), kind = (int)(h->block_key[i] >> 31 & 3);
+        h->block_est[i] = expected_pairs(w, std::min(kind_homes(kind, h->blocks_bs), w.n - first));
+        if (h->work_host && i < h->work_host_cap) h->work_host[i] = h->block_est[i];
+    }
+    // the last step's counters, and the copy the next step makes of them: of no layout
+    const size_t tag = 2 + h->worlds.size();
+    if (tag < h->stat_cap) h->stat_host[tag] = 0;
+    if (h->d_pairs && tag < h->pairs_cap) {
+        k_zero_u64<<<1, kBlock, 0, h->stream>>>(h->d_pairs + tag, 1);
+        LAUNCH_CHECK();
+    }
+    return PLIFE_OK;
+}
+
 // Applies position preset (positions) or type preset (!positions) `preset`
 // to the slots of world w, with draws from `seed`; the layout must be synced.
 int apply_preset(plife_physics *h, WorldHost &w, bool positions, int preset, uint64_t seed)
@@ -2326,10 +2352,9 @@ int apply_preset(plife_physics *h, WorldHost &w, bool positions, int preset, uin
     else k_set_types<<<ceil_div(w.n, kBlock), kBlock, 0, h->stream>>>(g);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(h->stream));
-    w.nb = w.hot = -1.0;     // the world's clustering is no longer known
     if (!positions) w.max_type = w.ntypes - 1;
     h->stepped = false;      // cell by-products describe the old state
-    return PLIFE_OK;
+    return positions ? forget_world(h, w) : PLIFE_OK;
 }
 
 // Overwrites k particles of world w at slots of its current order (the
@@ -2588,10 +2613,12 @@ void destroy_handle(plife_physics *h)
     if (h->stream) (void)hipStreamDestroy(h->stream);
 }
 
-// A new world: forget the clustering measure of the old ones.
+// A new world: forget the clustering measure of the old ones, and their
+// workgroups' pairs (the tag of the record of them).
 void reset_planner(plife_physics *h)
 {
     std::memset(h->stat_host, 0, h->stat_cap * sizeof(uint64_t));
+    if (h->work_host && h->blocks.size() < h->work_host_cap) h->work_host[h->blocks.size()] = 0;
     h->occupancy = 0.0;
     h->clustered = false;
     for (WorldHost &w : h->worlds) w.nb = w.hot = -1.0;

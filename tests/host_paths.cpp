@@ -26,7 +26,7 @@ int count(const char *what)
 template <typename T>
 T arg(void **args, int k) { return *static_cast<T *>(args[k]); }
 
-// k_bin and k_copy_u64 as far as the host sees them: the step's counters.
+// k_bin, k_zero_u64 and k_copy_u64 as far as the host sees them: the step's counters.
 void counters(const std::string &name, void **a)
 {
     if (has(name, "k_bin")) {
@@ -37,9 +37,20 @@ void counters(const std::string &name, void **a)
             if (out) out[t] = counters[t];
             counters[t] = t < nc ? 0ull : arg<unsigned long long>(a, 11);
         }
+    } else if (has(name, "k_zero_u64")) {
+        std::memset(arg<unsigned long long *>(a, 0), 0, 8u * (size_t)arg<int>(a, 1));
     } else if (has(name, "k_copy_u64")) {
         std::memcpy(arg<unsigned long long *>(a, 1), arg<const unsigned long long *>(a, 0), 8u * (size_t)arg<int>(a, 2));
     }
+}
+
+// The force kernels' record of their workgroups' pairs: table entry e had pairs_of(e).
+void work(const std::string &name, void **args, const std::function<uint32_t(int)> &pairs_of)
+{
+    if (!has(name, "k_force")) return;
+    const ForceArgs &a = *static_cast<ForceArgs *>(args[0]);
+    for (int e = 0; e < a.nb_total; ++e) a.block_work[e] = pairs_of(e);
+    a.block_work[a.nb_total] = a.work_tag;
 }
 }  // namespace fake
 
@@ -228,6 +239,50 @@ void stopped_update_keeps_the_last_step()
     plife_destroy(h);
 }
 
+// New positions or particles: the planner keeps neither the workgroups' measured
+// work nor the neighbours of the state before, whatever the way in.
+void new_state_forgets_measured_work()
+{
+    const plife_tuning t{256, 0, 1, 0.0, 1, 0, 1};
+    for (int way = 0; way < 3; ++way) {
+        plife_physics *h = nullptr;
+        plife_batch *b = nullptr;
+        int32_t id = 0;
+        const plife_settings s = settings(2, 0.05);
+        if (way == 2) {
+            CHECK(plife_batch_create(0, &b) == PLIFE_OK && plife_batch_set_tuning(b, &t) == PLIFE_OK);
+            CHECK(plife_batch_add_generated_world(b, &s, 2, kMatrix, 40000, 1, &id) == PLIFE_OK);
+            h = b;
+        } else {
+            h = engine(2, 0.05, 40000, t);
+        }
+        auto update = [&]() { return b ? plife_batch_update(b, 1) : plife_update(h, 1); };
+        bool recording = true;
+        fake::device = [&](const std::string &name, void **a) {
+            fake::counters(name, a);
+            if (recording) fake::work(name, a, [&](int e) { return e == h->nb_total - 1 ? 1000000u : 1000u; });
+            if (fake::has(name, "k_force")) h->d_pairs[2] = 4000000ull;       // 100 neighbours each
+        };
+        CHECK(update() == PLIFE_OK);
+        recording = false;                  // the device's next record is not there yet
+        if (way == 0) CHECK(plife_set_positions(h, 0, 5) == PLIFE_OK);
+        if (way == 1) CHECK(plife_generate_particles(h, 40000, 5) == PLIFE_OK);
+        if (way == 2) CHECK(plife_batch_set_world_positions(b, id, 0, 5) == PLIFE_OK);
+        CHECK(prepare_step(h) == PLIFE_OK);
+        CHECK(h->worlds[0].nb < 0.0 && (int)h->blocks.size() == 157);
+        for (int i = 0; i < 157; ++i) {
+            CHECK((int)h->blocks[i].y == 256 * i);                            // no order made from the old work
+            if (i < 156) CHECK(h->block_est[i] == h->block_est[0]);
+        }
+        CHECK(do_step(h, nullptr) == PLIFE_OK);   // its binning hands on the counters of the state before
+        fake::device = nullptr;
+        refresh_occupancy(h);
+        if (way != 1) CHECK(h->stat_host[2 + 1] != h->version + 1);
+        if (b) plife_batch_destroy(b);
+        else plife_destroy(h);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -235,6 +290,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
+        {"new_state_forgets_measured_work", new_state_forgets_measured_work},
         {"stopped_update_keeps_the_last_step", stopped_update_keeps_the_last_step},
     };
     const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();

@@ -21,7 +21,8 @@ def program(tmp_path_factory):
     return exe
 
 
-CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step"]
+CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step",
+         "new_state_forgets_measured_work"]
 
 
 @pytest.mark.parametrize("case", CASES)
