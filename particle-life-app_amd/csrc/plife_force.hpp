@@ -105,23 +105,6 @@ __device__ __forceinline__ double pair_coef(double d2, double mR, const WorldDev
     return u < a.betaR ? rep : att;
 }
 
-template <int DIM, bool DEBUG>
-__device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, double mR, uint32_t qid,
-                                       const WorldDev &a)
-{
-    const double dx = (double)dxi, dy = (double)dyi, dz = (double)dzi;
-    const double d2 = pair_d2<DIM>(dx, dy, dz);
-    const bool in = (d2 != 0.0) & (d2 <= a.r2u);     // Physics.java:432
-    if (in) {
-        const double c = pair_coef(d2, mR, a);
-        acc.x = fma(c, dx, acc.x);
-        acc.y = fma(c, dy, acc.y);
-        if constexpr (DIM == 3) acc.z = fma(c, dz, acc.z);
-        acc.cnt += 1;
-        if constexpr (DEBUG) acc.hash += id_hash(qid);
-    }
-}
-
 // pair_d2 where every square of a pair in range is below 2^52 (rmax <= 2^-6,
 // WorldDev::exact_d2): squares and sums of integers below 2^53 are exact, so
 // FMAs give the same value in one instruction less per axis; a pair whose sum
@@ -138,12 +121,18 @@ __device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
 // max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
 // zero to the other branch's value -- two instructions where the compare, the
 // two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
-// free on its FMA, is max(g, 0).)  No predicate either: past rmax g is negative
-// and 1/beta - 1/dist is not, so both are zero; where d2 = 0 the square root's
-// argument of 1/2 keeps every term finite, and the difference it multiplies is 0.
-__device__ __forceinline__ double pair_coef_sum(double d2, double mR, const WorldDev &a)
+// free on its FMA, is max(g, 0).  y is low by up to 2^-44 of itself, one Newton
+// step from FP32; within that of beta both terms are zero, where the selected
+// form has one of that size and the wrong sign.)  A pair not `in` range loses the
+// high word of its coefficient, in place of the guard that d2 = 0 would need in
+// FP32: the 2^-1042 that may be left, times any difference and count, stays
+// below 2^-980, which no velocity, position or exported acceleration shows
+// (world_dev keeps force and dt within 2^400).  Clearing both words, 1.3% more
+// instructions: 512-world batch 1655 us a launch, 1638 so; clearing 1/|D| in FP32
+// instead lengthens the chain, dense 196k 2D world 1870 -> 1975.
+__device__ __forceinline__ double pair_coef_sum(double d2, double mR, bool in, const WorldDev &a)
 {
-    const double y0 = (double)__builtin_amdgcn_rsqf(fmaxf((float)d2, 0.5f));
+    const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
     const double e = d2 * y0;
     const double h = fma(-e, y0, 1.0);
     const double y = fma(0.5 * y0, h, y0);
@@ -151,7 +140,34 @@ __device__ __forceinline__ double pair_coef_sum(double d2, double mR, const Worl
     const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
     const double g = fmin(fmax(fma(t, -a.inv_1mb, 1.0), 0.0), 1.0);
     const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);
-    return fma(mR * g, y, rep);
+    const double c = fma(mR * g, y, rep);
+    uint2 b = __builtin_bit_cast(uint2, c);
+    b.y = in ? b.y : 0u;
+    return __builtin_bit_cast(double, b);
+}
+
+// The form for a pair in range, by world: one for all kernels, so that the bits
+// do not depend on the kernel that steps the world.
+__device__ __forceinline__ double pair_law(double d2, double mR, const WorldDev &a)
+{
+    return a.all_global ? pair_coef(d2, mR, a) : pair_coef_sum(d2, mR, true, a);
+}
+
+template <int DIM, bool DEBUG>
+__device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, double mR, uint32_t qid,
+                                       const WorldDev &a)
+{
+    const double dx = (double)dxi, dy = (double)dyi, dz = (double)dzi;
+    const double d2 = pair_d2<DIM>(dx, dy, dz);
+    const bool in = (d2 != 0.0) & (d2 <= a.r2u);     // Physics.java:432
+    if (in) {
+        const double c = pair_law(d2, mR, a);
+        acc.x = fma(c, dx, acc.x);
+        acc.y = fma(c, dy, acc.y);
+        if constexpr (DIM == 3) acc.z = fma(c, dz, acc.z);
+        acc.cnt += 1;
+        if constexpr (DEBUG) acc.hash += id_hash(qid);
+    }
 }
 
 // G lanes share a home (G = 4: a quad of lanes; G = 16: a row of 16): lane k of
@@ -580,13 +596,12 @@ __device__ __forceinline__ uint32_t low_bits(int n)
 
 // Staged candidate at place k (the LDS address of its type, from which the
 // others follow in one instruction each) against a home at (px, py, pz)
-// (staged_axis) with matrix row mrow: the coefficient (0, or finite with a
-// difference of 0, where the pair does not interact), the difference and its
-// square.
+// (staged_axis) with matrix row mrow: the coefficient (0 where the pair does not
+// interact, Physics.java:432), the difference, and the wave's lanes whose pairs do.
 template <int DIM, bool WRAP, bool MLDS, bool EXACT>
 __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev &w, const Staged &s,
                                               const double *M, uint32_t k, uint32_t px, uint32_t py, uint32_t pz,
-                                              int mrow, int &dxi, int &dyi, int &dzi, double &d2)
+                                              int mrow, int &dxi, int &dyi, int &dzi, uint64_t &in)
 {
     const uint64_t xy = lds_read<uint64_t>(8u * k + s.at.xy);
     const uint2 hl = make_uint2((uint32_t)xy, (uint32_t)(xy >> 32));
@@ -595,8 +610,9 @@ __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev
     dzi = DIM == 3 ? staged_diff<WRAP>(lds_read<uint32_t>(4u * k + s.at.z), pz) : 0;
     const int idx = mrow + (int)lds_read<uint8_t>(k);
     const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-    d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
-    return pair_coef_sum(d2, m, w);
+    const double d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
+    in = __ballot(d2 != 0.0) & __ballot(d2 <= w.r2u);
+    return pair_coef_sum(d2, m, __builtin_amdgcn_inverse_ballot_w64(in), w);
 }
 
 // Mask words: the top kWordCands bits one candidate each, first at the top, the
@@ -621,19 +637,18 @@ __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev 
 {
     auto visit = [&](uint32_t k, bool last) {
         int dxi, dyi, dzi;
-        double d2;
-        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, d2);
+        uint64_t in;
+        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, in);
         ab.x = fma(c, (double)dxi, ab.x);
         ab.y = fma(c, (double)dyi, ab.y);
         if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);
-        // Physics.java:432
         if (DEBUG || last) {
-            const bool in = (d2 != 0.0) & (d2 <= w.r2u);
-            ab.cnt += in ? 1 : 0;
+            const bool mine = __builtin_amdgcn_inverse_ballot_w64(in);
+            ab.cnt += mine ? 1 : 0;
             if constexpr (DEBUG)
-                if (in) ab.hash += id_hash(s.id[k - s.at.type]);
+                if (mine) ab.hash += id_hash(s.id[k - s.at.type]);
         } else {
-            loop += __popcll(__ballot(d2 != 0.0) & __ballot(d2 <= w.r2u));
+            loop += __popcll(in);
         }
     };
     uint32_t m = 0;

@@ -157,10 +157,10 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
             constexpr bool EXACT = decltype(exact)::value;
             auto coef = [&](int p, int &dx, int &dy, int &dz) -> double {
                 const uint32_t k = list[min(p, n - 1)];
-                double d2;
+                uint64_t lanes;
                 const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, bx, by, bz, mrow, dx, dy, dz,
-                                                                     d2);
-                const bool in = (p < n) & (d2 != 0.0) & (d2 <= w.r2u);      // Physics.java:432
+                                                                     lanes);
+                const bool in = p < n && __builtin_amdgcn_inverse_ballot_w64(lanes);
                 acc.cnt += in ? 1 : 0;
                 if constexpr (DEBUG)
                     if (in) acc.hash += id_hash(stg.id[k - stg.at.type]);

@@ -283,6 +283,22 @@ void new_state_forgets_measured_work()
     }
 }
 
+// Forces and time steps so large that what pair_coef_sum leaves out of range
+// could show take the literal law, as matrices that are not finite do.
+void extreme_forces_take_the_literal_law()
+{
+    auto literal = [](double force, double dt, double entry) {
+        WorldHost w;
+        w.st = settings(2, 0.05);
+        w.st.force = force;
+        w.st.dt = dt;
+        w.matrix = {entry};
+        return world_dev(w, 0u, 0).all_global;
+    };
+    CHECK(!literal(0x1p400, 0.01, 1.0) && !literal(1.0, -0x1p400, 1.0) && !literal(1.0, 0.01, 1e290));
+    CHECK(literal(0x1p401, 0.01, 1.0) && literal(-1e300, 0.01, 1.0) && literal(1.0, 1e121, 1.0) && literal(1.0, 0.01, 1e301));
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -290,6 +306,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
+        {"extreme_forces_take_the_literal_law", extreme_forces_take_the_literal_law},
         {"new_state_forgets_measured_work", new_state_forgets_measured_work},
         {"stopped_update_keeps_the_last_step", stopped_update_keeps_the_last_step},
     };

@@ -22,7 +22,7 @@ def program(tmp_path_factory):
 
 
 CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step",
-         "new_state_forgets_measured_work"]
+         "new_state_forgets_measured_work", "extreme_forces_take_the_literal_law"]
 
 
 @pytest.mark.parametrize("case", CASES)
