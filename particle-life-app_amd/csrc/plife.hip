@@ -2742,6 +2742,7 @@ int na_scratch_base(int dev, unsigned char **out)
 // previous call may have stopped between binning and the cell scan).
 // Block 0 also looks the matrix over (it is in device memory): entries that
 // are not finite times R send the world down the literal path, as world_dev does.
+// (A call of no particles passes no matrix.)
 __global__ void k_na_setup(WorldDev wd, const double *matrix, WorldDev *world, uint2 *blocks, int nblocks,
                            int bs, unsigned long long *counters, uint32_t *work, uint32_t *cell_count,
                            int ncells)
@@ -2749,7 +2750,7 @@ __global__ void k_na_setup(WorldDev wd, const double *matrix, WorldDev *world, u
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == 0) {
         bool bad = false;
-        for (int t = threadIdx.x; t < wd.ntypes * wd.ntypes; t += blockDim.x) bad |= !isfinite(matrix[t] * wd.R);
+        for (int t = threadIdx.x; matrix && t < wd.ntypes * wd.ntypes; t += blockDim.x) bad |= !isfinite(matrix[t] * wd.R);
         if (__syncthreads_or(bad)) wd.all_global = 1;
         if (i == 0) *world = wd;
     }
@@ -2837,7 +2838,7 @@ int noalloc_step(const plife_settings *s, int32_t ntypes, const double *matrix, 
 
     const int setup_threads = std::max(nblocks + 1, 8);
     k_na_setup<<<std::min(ceil_div(std::max(setup_threads, nc), kBlock), 1024), kBlock, 0, stream>>>(
-        wd, matrix, t.d_worlds, t.d_blocks, nblocks, fp.bs, t.d_pairs, work, t.cell_count, nc);
+        wd, n > 0 ? matrix : nullptr, t.d_worlds, t.d_blocks, nblocks, fp.bs, t.d_pairs, work, t.cell_count, nc);
     LAUNCH_CHECK();
     if (n > 0) {
         // 1. cell keys and histogram; counters [0, 3) cleared, tag in [3]

@@ -299,6 +299,22 @@ void extreme_forces_take_the_literal_law()
     CHECK(literal(0x1p401, 0.01, 1.0) && literal(-1e300, 0.01, 1.0) && literal(1.0, 1e121, 1.0) && literal(1.0, 0.01, 1e301));
 }
 
+// A no-alloc step of no particles hands no kernel the caller's matrix: it was
+// never read for one.
+void empty_noalloc_step_reads_no_matrix()
+{
+    const plife_settings s = settings(2, 0.05);
+    bool seen = false;
+    fake::device = [&](const std::string &name, void **a) {
+        if (!fake::has(name, "k_na_setup")) return;
+        seen = true;
+        CHECK(fake::arg<const double *>(a, 1) == nullptr);
+    };
+    CHECK(plife_step_noalloc(&s, 2, kMatrix, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                             nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr) == PLIFE_OK);
+    CHECK(seen);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -306,6 +322,7 @@ int main(int argc, char **argv)
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
+        {"empty_noalloc_step_reads_no_matrix", empty_noalloc_step_reads_no_matrix},
         {"extreme_forces_take_the_literal_law", extreme_forces_take_the_literal_law},
         {"new_state_forgets_measured_work", new_state_forgets_measured_work},
         {"stopped_update_keeps_the_last_step", stopped_update_keeps_the_last_step},

@@ -22,7 +22,8 @@ def program(tmp_path_factory):
 
 
 CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step",
-         "new_state_forgets_measured_work", "extreme_forces_take_the_literal_law"]
+         "new_state_forgets_measured_work", "extreme_forces_take_the_literal_law",
+         "empty_noalloc_step_reads_no_matrix"]
 
 
 @pytest.mark.parametrize("case", CASES)
