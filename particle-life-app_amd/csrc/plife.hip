@@ -320,6 +320,7 @@ struct plife_physics {
     plife_tuning tune{};
     ForcePlan plan{};
     SplitPlan split{};
+    uint32_t lds_raised[3] = {};       // per homes (64, 128, 256): kernels whose LDS limit is raised (ready_kernels)
     size_t last_lds = 0;
     int last_cap = 0, last_bs = 0, last_lcap = 0;
 
@@ -860,11 +861,6 @@ int sort_cells(plife_physics *h, int dim, const PosBuf &P, const int32_t *type, 
 template <int DIM, bool WRAP, bool DEBUG, bool MLDS, int BS>
 void launch_staged(plife_physics *h, const ForceArgs &a, int nblocks, size_t lds)
 {
-    // (a launch with more dynamic LDS than 64 KB needs the limit raised; an
-    // error shows at the launch)
-    if (lds > 65536)
-        (void)hipFuncSetAttribute((const void *)k_force<DIM, WRAP, DEBUG, MLDS, BS>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     k_force<DIM, WRAP, DEBUG, MLDS, BS><<<nblocks, BS, lds, h->stream>>>(a);
 }
 
@@ -1389,6 +1385,43 @@ const void *small_kernel(int dim, bool dbg, bool mlds)
     return mlds ? small_kernel_of<2, false, true>() : small_kernel_of<2, false, false>();
 }
 
+// k_force of bs homes.
+template <int DIM, bool WRAP, bool DEBUG, bool MLDS>
+const void *staged_kernel_of(int bs)
+{
+    void (*f)(ForceArgs) = bs == 64    ? k_force<DIM, WRAP, DEBUG, MLDS, 64>
+                           : bs == 128 ? k_force<DIM, WRAP, DEBUG, MLDS, 128>
+                                       : k_force<DIM, WRAP, DEBUG, MLDS, 256>;
+    return reinterpret_cast<const void *>(f);
+}
+
+template <int DIM, bool WRAP>
+const void *staged_kernel(bool dbg, bool mlds, int bs)
+{
+    if (dbg) return mlds ? staged_kernel_of<DIM, WRAP, true, true>(bs) : staged_kernel_of<DIM, WRAP, true, false>(bs);
+    return mlds ? staged_kernel_of<DIM, WRAP, false, true>(bs) : staged_kernel_of<DIM, WRAP, false, false>(bs);
+}
+
+// A staged launch of more than 64 KB of dynamic LDS needs its kernel's limit
+// raised, once in a handle's life and never in a capture.
+int ready_kernels(plife_physics *h)
+{
+    if (h->plan.lds <= 65536) return PLIFE_OK;
+    const bool d3 = h->dim == 3, dbg = h->debug != 0, mlds = h->ntypes_max <= kMaxTypesLds;
+    const int bs = h->plan.bs;
+    for (const bool wrap : {true, false}) {
+        if (h->seg[(wrap ? 0 : kForceKinds) + kStaged] == 0) continue;
+        const uint32_t bit = 1u << (d3 + 2 * wrap + 4 * dbg + 8 * mlds);
+        uint32_t &ready = h->lds_raised[bs == 64 ? 0 : bs == 128 ? 1 : 2];
+        if (ready & bit) continue;
+        HIP_TRY(hipFuncSetAttribute(d3 ? (wrap ? staged_kernel<3, true>(dbg, mlds, bs) : staged_kernel<3, false>(dbg, mlds, bs))
+                                       : (wrap ? staged_kernel<2, true>(dbg, mlds, bs) : staged_kernel<2, false>(dbg, mlds, bs)),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
+        ready |= bit;
+    }
+    return PLIFE_OK;
+}
+
 // Whether the handle steps in one launch (k_step_small): every world fits one
 // workgroup's LDS (particles, cells, types), and the tuning allows it.  Homes
 // per workgroup: the fewest of 256, 512, 1024, ... for which the workgroups of
@@ -1518,6 +1551,7 @@ int prepare_step(plife_physics *h)
     if ((rc = ensure_dev(&h->bsq, &h->bsq_cap, nb, &h->retired))) return rc;
     if (h->small) return ensure_small_blocks(h);
     if ((rc = ensure_blocks(h, h->plan.bs))) return rc;
+    if ((rc = ready_kernels(h))) return rc;
     return balance_blocks(h);
 }
 
@@ -1527,6 +1561,7 @@ int select_path(plife_physics *h, bool one)
     h->small = one;
     if (one) return ensure_small_blocks(h);
     int rc = ensure_blocks(h, h->plan.bs);
+    if (!rc) rc = ready_kernels(h);
     return rc ? rc : balance_blocks(h);
 }
 

@@ -13,6 +13,9 @@ std::map<const void *, std::string> kernels;       // host stub -> mangled name
 std::vector<std::string> launched;
 int syncs = 0;                                      // waits for a stream
 long allocs_left = -1;                              // hipMalloc calls that succeed (-1: all)
+bool capturing = false;
+int attributes = 0, attributes_in_capture = 0;      // hipFuncSetAttribute calls
+hipError_t attribute_result = hipSuccess;
 std::function<void(const std::string &, void **)> device;
 
 bool has(const std::string &name, const char *what) { return name.find(what) != std::string::npos; }
@@ -117,13 +120,18 @@ hipError_t hipGetSymbolAddress(void **p, const void *)
     *p = scratch_mem;
     return hipSuccess;
 }
-hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int)
+{
+    ++fake::attributes;
+    fake::attributes_in_capture += fake::capturing;
+    return fake::attribute_result;
+}
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = new ihipStream_t; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { ++fake::syncs; return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { *g = new ihipGraph; return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { fake::capturing = true; return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { fake::capturing = false; *g = new ihipGraph; return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { *e = new ihipEvent_t; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
@@ -315,12 +323,36 @@ void empty_noalloc_step_reads_no_matrix()
     CHECK(seen);
 }
 
+// A launch of more than 64 KB of LDS raises the kernel's limit before any
+// capture, once, and an update whose limit cannot be raised says so.
+void lds_limit_is_raised_ahead()
+{
+    const plife_tuning t{0, 0, 0, 0.0, 1, 0, 1};
+    for (const bool fails : {true, false}) {
+        plife_physics *h = engine(3, 0.04, 130000, t);
+        fake::attribute_result = fails ? hipErrorInvalidValue : hipSuccess;
+        fake::launched.clear();
+        fake::attributes = 0;
+        const int rc = plife_update(h, 70);
+        CHECK(h->plan.lds > 65536);
+        if (fails) {
+            CHECK(rc == PLIFE_ERR_DEVICE && fake::count("k_force") == 0);
+        } else {
+            CHECK(rc == PLIFE_OK && fake::attributes_in_capture == 0);
+            const int before = fake::attributes;
+            CHECK(before > 0 && plife_update(h, 3) == PLIFE_OK && fake::attributes == before);
+        }
+        plife_destroy(h);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
+        {"lds_limit_is_raised_ahead", lds_limit_is_raised_ahead},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
         {"empty_noalloc_step_reads_no_matrix", empty_noalloc_step_reads_no_matrix},
         {"extreme_forces_take_the_literal_law", extreme_forces_take_the_literal_law},
