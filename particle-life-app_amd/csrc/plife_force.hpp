@@ -622,7 +622,9 @@ __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev
 // (force kernel, 1M 2D world 173 -> 165 us, 512-world batch 1740 -> 1619; with
 // 16-bit bases, 22% more LDS and a workgroup less on a CU, 1M 175).
 constexpr int kWordCands = 20, kPlaceBits = 32 - kWordCands;
-constexpr int kMaxStaged = (1 << kPlaceBits) - 64;    // places are below it: the types are at LDS address 0
+// Places are below it: the types are at LDS address 0, as long as k_force has no
+// static LDS (which is checked in the built library).
+constexpr int kMaxStaged = (1 << kPlaceBits) - 64;
 
 // Phase B of one home at (px, py, pz) with matrix row mrow: its `left` kept
 // candidates, word by word from `at` in candidate order, two per iteration (half

@@ -32,7 +32,8 @@ struct SplitLds {
     size_t m, xy, list, z, id, off, type, total;
 };
 
-// List entries per home: a window's worth, plus two so that the homes' lists
+// List entries (16-bit LDS addresses of candidates' types: static and dynamic
+// LDS together stay within 64 KB, plan_split_for) per home: a window's worth, plus two so that the homes' lists
 // start in different banks.
 __host__ __device__ constexpr int split_list_stride(int cap) { return cap + 2; }
 
