@@ -217,9 +217,10 @@ int plife_get_accelerations(plife_physics *h, int32_t n, float *acc);
  * the latest measurement that has reached the host.  Two automatic choices
  * are measured instead, on the first update of at least 24 steps: the step
  * path (small_step 0, where every world fits) and, on the multi-launch path,
- * block_homes (256 or 128 homes per workgroup; kept per class of layout:
- * dimension, clustering, mean particles per cell, particle count).  Both
- * time the candidates on steps of that update, which the update counts. */
+ * block_homes (the planner's own choice against the next one; kept per class
+ * of layout: dimension, clustering, the planner's own choice, particles per
+ * cell, particle count).  Both time the candidates on steps of that update,
+ * which the update counts. */
 typedef struct {
     int32_t block_homes;
     int32_t list_cap;

@@ -1118,51 +1118,61 @@ SplitPlan plan_split_for(int dim, bool dbg, int ntypes_max)
     }
 }
 
-ForcePlan plan_force(const plife_physics *h)
+// What the planner goes by: the density of the worlds the staged kernel steps
+// (all of them if none is), their particles, the cells per row of a single one,
+// and whether several densities share the launch.
+struct PlanInput {
+    double avg;
+    long long n;
+    int nx;
+    bool mixed;
+};
+
+PlanInput plan_input(const plife_physics *h)
 {
-    const int dim = h->dim == 3 ? 3 : 2;
-    // density of the worlds the staged kernel steps (all of them if none is)
-    long long sn = 0, sc = 0;
-    int nx = 0;                        // cells per row of a single world
+    PlanInput p{};
+    long long sc = 0;
     for (const WorldHost &w : h->worlds)
         if (w.kind == kStaged) {
-            sn += w.n;
+            p.n += w.n;
             sc += grid_of(w.st).ncells;
-            if (h->worlds.size() == 1) nx = grid_of(w.st).nx;
+            if (h->worlds.size() == 1) p.nx = grid_of(w.st).nx;
         }
     if (sc == 0) {
-        sn = h->n;
+        p.n = h->n;
         sc = h->ncells;
     }
     // Where a single 3D world has drawn together, but not into clusters, the
     // particles' own cells set a workgroup's neighbourhood, not the mean cell.
-    double avg = (double)sn / (double)std::max(sc, 1LL);
-    if (dim == 3 && !h->clustered && h->worlds.size() == 1) avg = std::max(avg, h->occupancy - 1.0);
+    p.avg = (double)p.n / (double)std::max(sc, 1LL);
+    if (h->dim == 3 && !h->clustered && h->worlds.size() == 1) p.avg = std::max(p.avg, h->occupancy - 1.0);
     // (a single 2D world that has clustered and does not fit the CUs at once is
     // planned as a batch of worlds of several densities: 800k particles of 1,200
     // neighbours 2.62 ms, 3.00 as one dense world)
-    const bool mixed = h->worlds.size() > 1 ||
-                       (dim == 2 && h->occupancy > 2.0 * (avg + 1.0) && sn > (long long)kSnakeRounds * kCus * 256);
-    return plan_force_for(dim, avg, sn, nx, h->clustered, mixed, plan_tuning(h), h->debug != 0,
+    p.mixed = h->worlds.size() > 1 ||
+              (h->dim != 3 && h->occupancy > 2.0 * (p.avg + 1.0) && p.n > (long long)kSnakeRounds * kCus * 256);
+    return p;
+}
+
+ForcePlan plan_force(const plife_physics *h, const plife_tuning &t)
+{
+    const PlanInput p = plan_input(h);
+    return plan_force_for(h->dim == 3 ? 3 : 2, p.avg, p.n, p.nx, h->clustered, p.mixed, t, h->debug != 0,
                           h->ntypes_max);
 }
 
 // The class of a layout for the measured homes per workgroup: dimension,
-// clustering, batch or single, the staged worlds' mean particles per cell in
+// clustering, batch or single, what the planner would choose by itself and
+// whether it plans for several densities, the particles per cell it goes by in
 // half octaves and the particle count in octaves.
 uint64_t shape_class(const plife_physics *h)
 {
-    long long sn = 0, sc = 0;
-    for (const WorldHost &w : h->worlds)
-        if (w.kind == kStaged) {
-            sn += w.n;
-            sc += grid_of(w.st).ncells;
-        }
-    const double avg = sc > 0 ? (double)sn / (double)sc : 0.0;
-    const int da = (int)std::floor(std::log2(std::max(avg, 1.0 / 64.0)) * 2.0) + 64;
+    const PlanInput p = plan_input(h);
+    const int own = plan_force(h, h->tune).bs / 64;
+    const int da = (int)std::floor(std::log2(std::max(p.avg, 1.0 / 64.0)) * 2.0) + 64;
     const int nn = (int)std::floor(std::log2((double)std::max(h->n, 1)));
     return (uint64_t)(h->dim == 3) | (uint64_t)h->clustered << 1 | (uint64_t)(h->batch != 0) << 2 |
-           (uint64_t)(uint32_t)da << 8 | (uint64_t)(uint32_t)nn << 24;
+           (uint64_t)p.mixed << 3 | (uint64_t)own << 4 | (uint64_t)(uint32_t)da << 8 | (uint64_t)(uint32_t)nn << 24;
 }
 
 // Whether the next long update measures the homes per workgroup: the
@@ -1528,7 +1538,7 @@ int prepare_step(plife_physics *h)
     refresh_occupancy(h);
     classify_worlds(h);
     // a layout of a class measured before takes that class's homes per workgroup
-    if (h->tune.block_homes == 0 && h->bs_meas != h->version) {
+    if (h->tune.block_homes == 0 && h->bs_meas != h->version && !h->bs_seen.empty()) {
         const uint64_t c = shape_class(h);
         for (const auto &e : h->bs_seen)
             if (e.first == c) {
@@ -1537,7 +1547,7 @@ int prepare_step(plife_physics *h)
                 classify_worlds(h);
             }
     }
-    h->plan = plan_force(h);
+    h->plan = plan_force(h, plan_tuning(h));
     h->split = plan_split_for(h->dim == 3 ? 3 : 2, h->debug != 0, h->ntypes_max);
     if ((rc = ensure_cells(h, h->ncells))) return rc;
     if ((rc = ensure_debug(h))) return rc;
@@ -2023,6 +2033,7 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
     // other (time_pair) and keeps the faster for every layout of the class.
     if (shape_tune_due(h) && nsteps >= kTuneSteps && nsteps - k >= kTuneMax) {
         const int cand[2] = {h->plan.bs, h->plan.bs == 128 ? 256 : 128};            // the planner's first
+        const uint64_t layout = shape_class(h);
         float t[2];
         rc = time_pair([&](int p) {
             h->auto_bs = cand[p];
@@ -2037,7 +2048,7 @@ int run_steps(plife_physics *h, int nsteps, bool honour_stop)
             return rc;
         }
         h->auto_bs = faster(t) ? cand[1] : cand[0];
-        h->bs_seen.emplace_back(shape_class(h), h->auto_bs);
+        h->bs_seen.emplace_back(layout, h->auto_bs);
         if ((rc = prepare_step(h))) return rc;
     }
     bool use_graph = nsteps - k >= 2 && !h->tune.direct_launch;

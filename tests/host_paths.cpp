@@ -346,12 +346,29 @@ void lds_limit_is_raised_ahead()
     }
 }
 
+// The homes per workgroup measured for a layout go to no layout that the planner
+// itself would give others: here two worlds of one density, either side of the
+// particle count its rule for short rows changes at.
+void kept_homes_follow_the_plan()
+{
+    const double rmax = 1.0 / 700.5;
+    const plife_tuning t{0, 0, 0, 0.0, 1, 0, 1};
+    plife_physics *h = engine(2, rmax, 99999, t);
+    CHECK(plife_update(h, 40) == PLIFE_OK && h->bs_seen.size() == 1 && h->plan.bs == 128);
+    CHECK(plife_generate_particles(h, 99998, 8) == PLIFE_OK && plife_update(h, 3) == PLIFE_OK);
+    CHECK(h->bs_meas == h->version && h->plan.bs == 128);        // the same class: kept
+    CHECK(plife_generate_particles(h, 100001, 8) == PLIFE_OK && plife_update(h, 3) == PLIFE_OK);
+    CHECK(h->plan.bs == 256);
+    plife_destroy(h);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"failed_growth", failed_growth},
+        {"kept_homes_follow_the_plan", kept_homes_follow_the_plan},
         {"lds_limit_is_raised_ahead", lds_limit_is_raised_ahead},
         {"measured_cells_are_no_step", measured_cells_are_no_step},
         {"empty_noalloc_step_reads_no_matrix", empty_noalloc_step_reads_no_matrix},
