@@ -235,6 +235,11 @@ int plife_set_tuning(plife_physics *h, const plife_tuning *t);
 /* Current tuning with automatic fields resolved, and the LDS bytes per
  * workgroup of the last force launch. */
 int plife_get_tuning(plife_physics *h, plife_tuning *t, int32_t *lds_bytes);
+/* Workgroups of the last step's force launches by kernel: workgroups[0] the
+ * staged one, [1] the sparse-world one, [2] the one in which four lanes share a
+ * particle (worlds whose densest particles' neighbours outlast the launch).
+ * All 0 after a one-launch step.  A world takes one kernel as a whole. */
+int plife_get_force_kernels(plife_physics *h, int32_t workgroups[3]);
 
 /* One Physics.update() (Physics.java:112-134) of one world whose state lives
  * in caller-owned device memory, enqueued on `stream` (a hipStream_t; NULL =
@@ -330,6 +335,7 @@ int plife_batch_count(plife_batch *b, int32_t *nworlds, int64_t *nparticles);
 
 int plife_batch_set_tuning(plife_batch *b, const plife_tuning *t);
 int plife_batch_get_tuning(plife_batch *b, plife_tuning *t, int32_t *lds_bytes);
+int plife_batch_get_force_kernels(plife_batch *b, int32_t workgroups[3]);
 int plife_batch_time_steps(plife_batch *b, int32_t nsteps, double *ms);
 int plife_batch_profile(plife_batch *b, int32_t nsteps, plife_timing *out);
 

@@ -323,6 +323,7 @@ struct plife_physics {
     uint32_t lds_raised[3] = {};       // per homes (64, 128, 256): kernels whose LDS limit is raised (ready_kernels)
     size_t last_lds = 0;
     int last_cap = 0, last_bs = 0, last_lcap = 0;
+    int last_blocks[kForceKinds] = {};
 
     // the one-launch step of worlds that fit one workgroup's LDS (k_step_small)
     int lds_limit = 65536;             // the device's LDS per workgroup
@@ -1646,6 +1647,7 @@ int do_small_step(plife_physics *h, PhaseEvents *ev)
     h->small_kbuf ^= 1;
     h->last_lds = lds;
     h->last_bs = h->small_homes;
+    for (int &b : h->last_blocks) b = 0;
     if ((rc = record(h, ev, 4))) return rc;
     h->pc = po;
     h->ac = ao;
@@ -1745,6 +1747,7 @@ int do_step(plife_physics *h, PhaseEvents *ev)
     h->last_cap = fp.cap;
     h->last_bs = fp.bs;
     h->last_lcap = fp.lcap;
+    for (int k = 0; k < kForceKinds; ++k) h->last_blocks[k] = h->seg[k] + h->seg[kForceKinds + k];
     if ((rc = launch_force_any(h, a, fp.bs, fp.lds))) return rc;
     h->small_kbuf = 0;                 // the sort wrote the sorted keys to skeys
     if ((rc = record(h, ev, 4))) return rc;
@@ -3219,6 +3222,14 @@ int plife_get_tuning(plife_physics *h, plife_tuning *t, int32_t *lds_bytes)
     return PLIFE_OK;
 }
 
+int plife_get_force_kernels(plife_physics *h, int32_t workgroups[3])
+{
+    static_assert(kStaged == 0 && kSparse == 1 && kSplit == 2 && kForceKinds == 3, "the order plife.h states");
+    if (!h || !workgroups) return fail(PLIFE_ERR_ARGUMENT, "null argument");
+    for (int k = 0; k < kForceKinds; ++k) workgroups[k] = h->last_blocks[k];
+    return PLIFE_OK;
+}
+
 int plife_set_debug(plife_physics *h, int32_t on)
 {
     if (!h) return fail(PLIFE_ERR_ARGUMENT, "null handle");
@@ -3514,6 +3525,11 @@ int plife_batch_set_tuning(plife_batch *b, const plife_tuning *t) { return plife
 int plife_batch_get_tuning(plife_batch *b, plife_tuning *t, int32_t *lds_bytes)
 {
     return plife_get_tuning(b, t, lds_bytes);
+}
+
+int plife_batch_get_force_kernels(plife_batch *b, int32_t workgroups[3])
+{
+    return plife_get_force_kernels(b, workgroups);
 }
 
 int plife_batch_time_steps(plife_batch *b, int32_t nsteps, double *ms)

@@ -46,6 +46,7 @@ EXPORTS = (
     "plife_step_noalloc",
     "plife_set_tuning",
     "plife_get_tuning",
+    "plife_get_force_kernels",
     "plife_profile",
     "plife_time_steps",
     "plife_batch_create",
@@ -65,6 +66,7 @@ EXPORTS = (
     "plife_batch_count",
     "plife_batch_set_tuning",
     "plife_batch_get_tuning",
+    "plife_batch_get_force_kernels",
     "plife_batch_time_steps",
     "plife_batch_profile",
 )
@@ -157,6 +159,7 @@ def load() -> ctypes.CDLL:
         "plife_step_noalloc": [ctypes.POINTER(PlifeSettings), i32, vp, i32] + [vp] * 16 + [vp, vp],
         "plife_set_tuning": [vp, ctypes.POINTER(PlifeTuning)],
         "plife_get_tuning": [vp, ctypes.POINTER(PlifeTuning), ctypes.POINTER(i32)],
+        "plife_get_force_kernels": [vp, ctypes.POINTER(i32)],
         "plife_profile": [vp, i32, ctypes.POINTER(PlifeTiming)],
         "plife_time_steps": [vp, i32, ctypes.POINTER(ctypes.c_double)],
         "plife_batch_create": [i32, ctypes.POINTER(vp)],
@@ -178,6 +181,7 @@ def load() -> ctypes.CDLL:
         "plife_batch_count": [vp, ctypes.POINTER(i32), i64p],
         "plife_batch_set_tuning": [vp, ctypes.POINTER(PlifeTuning)],
         "plife_batch_get_tuning": [vp, ctypes.POINTER(PlifeTuning), ctypes.POINTER(i32)],
+        "plife_batch_get_force_kernels": [vp, ctypes.POINTER(i32)],
         "plife_batch_time_steps": [vp, i32, ctypes.POINTER(ctypes.c_double)],
         "plife_batch_profile": [vp, i32, ctypes.POINTER(PlifeTiming)],
     }

@@ -175,6 +175,12 @@ class Batch:
                 "windowed_only": bool(t.windowed_only), "small_step": t.small_step,
                 "lds_bytes": lds.value}
 
+    def force_kernels(self) -> dict:
+        """Workgroups of the last step's force launches by kernel."""
+        g = (ctypes.c_int32 * 3)()
+        check(self._lib.plife_batch_get_force_kernels(self._h, g))
+        return {"staged": g[0], "sparse": g[1], "split": g[2]}
+
     def time_steps(self, nsteps: int) -> float:
         ms = ctypes.c_double()
         check(self._lib.plife_batch_time_steps(self._h, int(nsteps), ctypes.byref(ms)))
