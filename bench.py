@@ -409,7 +409,7 @@ def main() -> int:
         },
         "step_path": ("one launch per step (k_step_small: keys, sort, cell table and force in one "
                       "workgroup's LDS)" if one_launch else
-                      "multi-launch (bin, scans, radix sort, force)"),
+                      "multi-launch (bin, scans, counting sort, force)"),
         "launch": {k: launch[k] for k in ("block_homes", "list_cap", "small_step", "lds_bytes")},
         "phases_ms": {k: prof[k] for k in ("bin_ms", "sort_ms", "gather_ms", "force_ms", "step_ms")},
         "app_path": {"ms_per_frame": frame_ms, "get_state_ms": get_state_ms,

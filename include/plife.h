@@ -55,7 +55,7 @@ typedef struct {
     double step_ms;     /* wall time per step, event-to-event over all steps */
     double bin_ms;      /* cell keys + cell histogram + cell scan */
     double sort_ms;     /* the stable counting sort */
-    double gather_ms;   /* 0: the force kernel reads the pre-sort state through the permutation */
+    double gather_ms;   /* 0: the sort writes the records the force kernel reads */
     double force_ms;    /* force + integrate kernel (average launch duration) */
     int64_t pairs;      /* interacting ordered pairs in the last step */
     int32_t steps;
@@ -144,7 +144,11 @@ int plife_generate_matrix(int32_t preset, int32_t size, uint64_t seed, double *o
  * them.  To keep a stop prompt, it keeps only about 20 ms of device work
  * queued (at least 2 steps, at most 62), waiting for the oldest queued
  * launch before it queues more, and checks the stop flag before every launch
- * (one launch is 1 or 2 steps).  Returns PLIFE_STOPPED if
+ * (one launch is 1 or 2 steps).  It also waits, to plan the other steps from
+ * what one measured: a new state's first update of 8 or more steps (3D: 3) for
+ * its first step, in 3D after binning the state once ahead of it, and a
+ * layout's first update of 24 or more steps for the steps it times (see
+ * plife_tuning).  Returns PLIFE_STOPPED if
  * plife_force_update_stop() arrived: nothing more is queued, the steps
  * already queued complete, and the state is then at a step boundary;
  * plife_get_steps counts them. */
@@ -196,15 +200,18 @@ int plife_get_accelerations(plife_physics *h, int32_t n, float *acc);
 
 /* Launch shape (no counterpart in the reference, which has no device).  Zero
  * fields mean automatic.  block_homes in {0, 64, 128, 256}: home particles
- * (threads) per force workgroup; list_cap in [0, 512]: LDS mask
- * words per home (32 candidates each) of a force workgroup that streams its
- * neighbourhood in several windows; stage_slack in [0, 16]: LDS
+ * (threads) per force workgroup; list_cap in [0, 512]: LDS for the screened
+ * candidates of a force workgroup that streams its neighbourhood in several
+ * windows, in units of 32 candidates a home (2 or more take effect, and at most
+ * 73, 36 or 18 for 64, 128 or 256 homes); stage_slack in [0, 16]: LDS
  * staging capacity as a multiple of the expected staged particles;
  * direct_launch 1: launch every kernel directly instead of replaying a HIP
  * graph of two steps; sparse_worlds: which worlds the sparse-world force
  * kernel (one thread per particle, stencil read from global memory) steps
  * instead of the staged one -- 0 those whose cells hold too few particles
- * for staging to pay, 1 none, 2 all; windowed_only 1: the staged force
+ * for staging to pay (and, no other launch-shape field set, worlds whose
+ * densest particles outlast the launch take a kernel of four lanes a
+ * particle), 1 none, 2 all; windowed_only 1: the staged force
  * kernel always streams a neighbourhood in windows, also where it would fit
  * one; small_step: whether worlds that fit one
  * workgroup's LDS (up to about 10,000 particles in 2D, 7,000 in 3D) step in
@@ -319,8 +326,10 @@ int plife_batch_set_world_settings(plife_batch *b, int32_t world_id, const plife
 
 /* nsteps steps of every world, all enqueued at once (unlike plife_update,
  * which bounds its queue: a batch's updates are short quanta, and batches on
- * their own streams overlap only if neither waits).  A stop request is
- * checked before every launch of this call. */
+ * their own streams overlap only if neither waits).  Two first updates do wait:
+ * of 3 or more steps in 3D, for the clustering of the cells, and of 24 or more
+ * steps of a layout, for the steps it times.  A stop request is checked before
+ * every launch of this call. */
 int plife_batch_update(plife_batch *b, int32_t nsteps);
 int plife_batch_force_update_stop(plife_batch *b);
 int plife_batch_synchronize(plife_batch *b);

@@ -831,7 +831,7 @@ int scan_cells(plife_physics *h, int ncells, unsigned long long *sq)
 int bin_cells(plife_physics *h, int dim, const PosBuf &P, int n, const uint16_t *world_of, int ncounters,
               unsigned long long tag, unsigned long long *stat_out)
 {
-    const int nb = ceil_div(n, kBlock * kBinItems);
+    const int nb = ceil_div(n, kBlock);
     if (dim == 3)
         k_bin<3><<<nb, kBlock, 0, h->stream>>>(P.x, P.y, P.z, n, h->d_worlds, world_of, h->keys0, h->perm,
                                                h->cell_count, h->d_pairs, ncounters, tag, stat_out);
@@ -1062,13 +1062,13 @@ ForcePlan plan_force_for(int dim, double avg, long long n, int nx, bool clustere
             }
         }
     }
-    // Several windows: mask words per home (in units of 32 candidates).  Where one
+    // Several windows: mask bits per home, in units of 32 candidates.  Where one
     // window is the rule (a single uniform world), no more than fit the space of
     // its pool: LDS per workgroup sets how many share a CU (1M 2D world: 0.218 ms
-    // a step within the pool, 0.231 at 7 words).  Worlds of several densities in
-    // one launch stream windows in the denser half of them: 9 words (512-world
-    // batch: 2.32 ms at 5 words, 2.33 at 7, 2.19 at 9), all of them in a single
-    // dense world: 16 (us a step at 9 / 16 words: 3D 300k of 65 a cell 1094 / 848, 2D 1M of
+    // a step within the pool, 0.231 at 7).  Worlds of several densities in
+    // one launch stream windows in the denser half of them: 9 (512-world
+    // batch: 2.32 ms at 5, 2.33 at 7, 2.19 at 9), all of them in a single
+    // dense world: 16 (us a step at 9 / 16: 3D 300k of 65 a cell 1094 / 848, 2D 1M of
     // 100 a cell 1037 / 932, clustered 196k 1870 / 1780).  Clustered worlds: 7 (4M
     // 3D world, 256 homes: 30.3 ms at 5, 28.1 at 7, 30.1 at 9; 1M, 128 homes: 1078
     // us at 5, 911 at 7).

@@ -212,8 +212,6 @@ __device__ __forceinline__ uint32_t count_runs(uint32_t key, bool valid, uint32_
 // Binning: cell keys, the cell histogram (run-aggregated atomics) and each
 // particle's place among its cell's arrivals.  Block 0 also clears the step's
 // counters.
-constexpr int kBinItems = 1;
-
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_bin(const uint32_t *__restrict__ px, const uint32_t *__restrict__ py,
                                                 const uint32_t *__restrict__ pz, int n,
@@ -236,27 +234,24 @@ __global__ __launch_bounds__(kBlock) void k_bin(const uint32_t *__restrict__ px,
     double cs = worlds[0].cs, ics = worlds[0].ics;
     int nx = worlds[0].nx;
     uint32_t cb = worlds[0].cell_base;
-#pragma unroll
-    for (int r = 0; r < kBinItems; ++r) {
-        const int i = (blockIdx.x * kBinItems + r) * kBlock + threadIdx.x;
-        const bool valid = i < n;
-        uint32_t key = 0xFFFFFFFFu;
-        if (valid) {
-            if (world_of) {                            // several worlds: this slot's world
-                const WorldDev *w = worlds + world_of[i];
-                cs = w->cs;
-                ics = w->ics;
-                nx = w->nx;
-                cb = w->cell_base;
-            }
-            key = (uint32_t)key_axis_fast(px[i], cs, ics, nx) + (uint32_t)key_axis_fast(py[i], cs, ics, nx) * (uint32_t)nx;
-            if constexpr (DIM == 3) key += (uint32_t)key_axis_fast(pz[i], cs, ics, nx) * (uint32_t)nx * (uint32_t)nx;
-            key += cb;
-            keys[i] = key;
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const bool valid = i < n;
+    uint32_t key = 0xFFFFFFFFu;
+    if (valid) {
+        if (world_of) {                                // several worlds: this slot's world
+            const WorldDev *w = worlds + world_of[i];
+            cs = w->cs;
+            ics = w->ics;
+            nx = w->nx;
+            cb = w->cell_base;
         }
-        const uint32_t at = count_runs(key, valid, cell_count);
-        if (valid) arrival[i] = at;
+        key = (uint32_t)key_axis_fast(px[i], cs, ics, nx) + (uint32_t)key_axis_fast(py[i], cs, ics, nx) * (uint32_t)nx;
+        if constexpr (DIM == 3) key += (uint32_t)key_axis_fast(pz[i], cs, ics, nx) * (uint32_t)nx * (uint32_t)nx;
+        key += cb;
+        keys[i] = key;
     }
+    const uint32_t at = count_runs(key, valid, cell_count);
+    if (valid) arrival[i] = at;
 }
 
 // Particle i to its cell's slots in arrival order.

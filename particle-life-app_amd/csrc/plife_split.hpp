@@ -32,9 +32,9 @@ struct SplitLds {
     size_t m, xy, list, z, id, off, type, total;
 };
 
-// List entries (16-bit LDS addresses of candidates' types: static and dynamic
-// LDS together stay within 64 KB, plan_split_for) per home: a window's worth, plus two so that the homes' lists
-// start in different banks.
+// List entries per home: a window's worth, plus two so that the homes' lists
+// start in different banks.  An entry is the LDS address of a candidate's type
+// in 16 bits: static and dynamic LDS together stay within 64 KB (plan_split_for).
 __host__ __device__ constexpr int split_list_stride(int cap) { return cap + 2; }
 
 __host__ __device__ inline SplitLds split_lds_layout(int dim, bool debug, int ntypes, bool m_in_lds, int cap,
