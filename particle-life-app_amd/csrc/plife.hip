@@ -2351,8 +2351,10 @@ int generate_particles(plife_physics *h, int off, int n, uint64_t seed, int ntyp
 }
 
 // World w's particles have new positions: forgets what steps measured of the
-// old ones, its neighbours and its workgroups' pairs.  The stream is idle.
-int forget_world(plife_physics *h, WorldHost &w)
+// old ones, its neighbours and its workgroups' pairs.  The stream is idle, and
+// the device's counters have lost their tag (k_set_positions), so that the next
+// step hands on no copy of them.
+void forget_world(plife_physics *h, WorldHost &w)
 {
     w.nb = w.hot = -1.0;
     for (size_t i = 0; i < h->block_key.size() && h->blocks_bs > 0; ++i) {
@@ -2361,14 +2363,8 @@ int forget_world(plife_physics *h, WorldHost &w)
         h->block_est[i] = expected_pairs(w, std::min(kind_homes(kind, h->blocks_bs), w.n - first));
         if (h->work_host && i < h->work_host_cap) h->work_host[i] = h->block_est[i];
     }
-    // the last step's counters, and the copy the next step makes of them: of no layout
     const size_t tag = 2 + h->worlds.size();
     if (tag < h->stat_cap) h->stat_host[tag] = 0;
-    if (h->d_pairs && tag < h->pairs_cap) {
-        k_zero_u64<<<1, kBlock, 0, h->stream>>>(h->d_pairs + tag, 1);
-        LAUNCH_CHECK();
-    }
-    return PLIFE_OK;
 }
 
 // Applies position preset (positions) or type preset (!positions) `preset`
@@ -2398,13 +2394,16 @@ int apply_preset(plife_physics *h, WorldHost &w, bool positions, int preset, uin
     g.vy = h->vy[a];
     g.vz = h->vz[a];
     g.type = h->type[a];
+    const size_t tag = 2 + h->worlds.size();
+    if (positions && h->d_pairs && tag < h->pairs_cap) g.tag = h->d_pairs + tag;
     if (positions) k_set_positions<<<ceil_div(w.n, kBlock), kBlock, 0, h->stream>>>(g);
     else k_set_types<<<ceil_div(w.n, kBlock), kBlock, 0, h->stream>>>(g);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(h->stream));
     if (!positions) w.max_type = w.ntypes - 1;
     h->stepped = false;      // cell by-products describe the old state
-    return positions ? forget_world(h, w) : PLIFE_OK;
+    if (positions) forget_world(h, w);
+    return PLIFE_OK;
 }
 
 // Overwrites k particles of world w at slots of its current order (the

@@ -584,6 +584,7 @@ struct PresetArgs {
     uint32_t *px, *py, *pz;
     float *vx, *vy, *vz;
     int32_t *type;
+    unsigned long long *tag;           // positions: the step counters' layout tag, cleared (may be null)
 };
 
 __device__ __forceinline__ double preset_u(uint64_t base, uint64_t step)
@@ -610,6 +611,7 @@ __global__ __launch_bounds__(kBlock) void k_set_positions(PresetArgs g)
 #pragma clang fp contract(off)
     const int k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= g.n) return;
+    if (k == 0 && g.tag) *g.tag = 0ull;
     const int i = g.off + k;
     const uint64_t s = (uint64_t)(k + 1) * kGamma;
     const int t = g.type[i];

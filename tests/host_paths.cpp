@@ -29,7 +29,7 @@ int count(const char *what)
 template <typename T>
 T arg(void **args, int k) { return *static_cast<T *>(args[k]); }
 
-// k_bin, k_zero_u64 and k_copy_u64 as far as the host sees them: the step's counters.
+// k_bin, k_set_positions and k_copy_u64 as far as the host sees them: the step's counters.
 void counters(const std::string &name, void **a)
 {
     if (has(name, "k_bin")) {
@@ -40,8 +40,8 @@ void counters(const std::string &name, void **a)
             if (out) out[t] = counters[t];
             counters[t] = t < nc ? 0ull : arg<unsigned long long>(a, 11);
         }
-    } else if (has(name, "k_zero_u64")) {
-        std::memset(arg<unsigned long long *>(a, 0), 0, 8u * (size_t)arg<int>(a, 1));
+    } else if (has(name, "k_set_positions")) {
+        if (arg<PresetArgs>(a, 0).tag) *arg<PresetArgs>(a, 0).tag = 0;
     } else if (has(name, "k_copy_u64")) {
         std::memcpy(arg<unsigned long long *>(a, 1), arg<const unsigned long long *>(a, 0), 8u * (size_t)arg<int>(a, 2));
     }
