@@ -2115,6 +2115,12 @@ int time_steps(plife_physics *h, int nsteps, double *ms)
         if ((rc = run_steps(h, kTuneSteps, false))) return rc;
         if ((rc = prepare_step(h))) return rc;
     }
+    // and the first step of a new state, whose counters an update waits for
+    if (h->n > 0 && !h->small && !h->batch && h->worlds[0].nb < 0.0 && nsteps >= 3) {
+        if ((rc = run_steps(h, 1, false))) return rc;
+        HIP_TRY(hipStreamSynchronize(h->stream));
+        if ((rc = prepare_step(h))) return rc;
+    }
     for (int i = 0; i < 2 && nsteps >= 2 && !h->tune.direct_launch &&
                     (!h->gexec || graph_key(h) != h->gkey); ++i)
         if ((rc = run_steps(h, 2, false))) return rc;

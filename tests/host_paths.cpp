@@ -12,6 +12,7 @@ namespace fake {
 std::map<const void *, std::string> kernels;       // host stub -> mangled name
 std::vector<std::string> launched;
 int syncs = 0;                                      // waits for a stream
+std::vector<int> syncs_at_record;                   // their count at each event record
 long allocs_left = -1;                              // hipMalloc calls that succeed (-1: all)
 bool capturing = false;
 int attributes = 0, attributes_in_capture = 0;      // hipFuncSetAttribute calls
@@ -135,7 +136,7 @@ hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { fake::capturing = f
 hipError_t hipEventCreate(hipEvent_t *e) { *e = new ihipEvent_t; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { fake::syncs_at_record.push_back(fake::syncs); return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
@@ -362,6 +363,25 @@ void kept_homes_follow_the_plan()
     plife_destroy(h);
 }
 
+// A timing of steps holds steps alone: the wait of a new state's first update
+// for its first step lies before it.
+void timed_steps_do_not_wait()
+{
+    for (const int dim : {2, 3}) {
+        plife_physics *h = engine(dim, dim == 3 ? 0.1 : 0.02, 30000, plife_tuning{0, 0, 1, 0.0, 0, 0, 1});
+        fake::device = [&](const std::string &name, void **a) {
+            fake::counters(name, a);
+            if (fake::has(name, "k_scan")) h->d_pairs[1] = 40000;            // sum of squares: uniform
+        };
+        double ms = 0.0;
+        fake::syncs_at_record.clear();
+        CHECK(plife_time_steps(h, 12, &ms) == PLIFE_OK);
+        const std::vector<int> &s = fake::syncs_at_record;
+        CHECK(s.size() >= 2 && s[s.size() - 2] == s.back());                 // the two events around the steps
+        plife_destroy(h);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -374,6 +394,7 @@ int main(int argc, char **argv)
         {"empty_noalloc_step_reads_no_matrix", empty_noalloc_step_reads_no_matrix},
         {"extreme_forces_take_the_literal_law", extreme_forces_take_the_literal_law},
         {"new_state_forgets_measured_work", new_state_forgets_measured_work},
+        {"timed_steps_do_not_wait", timed_steps_do_not_wait},
         {"stopped_update_keeps_the_last_step", stopped_update_keeps_the_last_step},
     };
     const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();

@@ -24,7 +24,7 @@ def program(tmp_path_factory):
 CASES = ["failed_growth", "measured_cells_are_no_step", "stopped_update_keeps_the_last_step",
          "new_state_forgets_measured_work", "extreme_forces_take_the_literal_law",
          "empty_noalloc_step_reads_no_matrix", "lds_limit_is_raised_ahead",
-         "kept_homes_follow_the_plan"]
+         "kept_homes_follow_the_plan", "timed_steps_do_not_wait"]
 
 
 @pytest.mark.parametrize("case", CASES)
