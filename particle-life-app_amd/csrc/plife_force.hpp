@@ -90,13 +90,18 @@ __device__ __forceinline__ double pair_d2(double dx, double dy, double dz)
     return DIM == 3 ? dx * dx + (dy * dy + dz * dz) : dx * dx + dy * dy;
 }
 
-// f/dist of the force law for a pair in range (0 < d2 <= rmax^2).
-__device__ __forceinline__ double pair_coef(double d2, double mR, const WorldDev &a)
+// 1/|D|: one Newton step from FP32, low by up to 2^-44 of itself.  (NaN where d2 = 0.)
+__device__ __forceinline__ double pair_recip(double d2)
 {
     const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
     const double e = d2 * y0;
     const double h = fma(-e, y0, 1.0);
-    const double y = fma(0.5 * y0, h, y0);        // 1/|D|, one Newton step from FP32
+    return fma(0.5 * y0, h, y0);
+}
+
+// f/dist of the force law for a pair in range (0 < d2 <= rmax^2), y = pair_recip(d2).
+__device__ __forceinline__ double pair_coef(double d2, double y, double mR, const WorldDev &a)
+{
     const double u = d2 * y;                       // |D| = dist R
     const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
     const double g = fma(t, -a.inv_1mb, 1.0);
@@ -121,36 +126,37 @@ __device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
 // max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
 // zero to the other branch's value -- two instructions where the compare, the
 // two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
-// free on its FMA, is max(g, 0).  y is low by up to 2^-44 of itself, one Newton
-// step from FP32; within that of beta both terms are zero, where the selected
-// form has one of that size and the wrong sign.)  A pair not `in` range loses the
-// high word of its coefficient, in place of the guard that d2 = 0 would need in
-// FP32: the 2^-1042 that may be left, times any difference and count, stays
-// below 2^-980, which no velocity, position or exported acceleration shows
-// (world_dev keeps force and dt within 2^400).  Clearing both words, 1.3% more
-// instructions: 512-world batch 1655 us a launch, 1638 so; clearing 1/|D| in FP32
-// instead lengthens the chain, dense 196k 2D world 1870 -> 1975.
-__device__ __forceinline__ double pair_coef_sum(double d2, double mR, bool in, const WorldDev &a)
+// free on its FMA, is max(g, 0).  Within 2^-44 of beta both terms are zero,
+// where the selected form has one of that size and the wrong sign.)  For a pair
+// in range only: the caller clears what it gives for others.
+__device__ __forceinline__ double pair_coef_sum(double d2, double y, double mR, const WorldDev &a)
 {
-    const double y0 = (double)__builtin_amdgcn_rsqf((float)d2);
-    const double e = d2 * y0;
-    const double h = fma(-e, y0, 1.0);
-    const double y = fma(0.5 * y0, h, y0);
     const double u = d2 * y;
     const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
     const double g = fmin(fmax(fma(t, -a.inv_1mb, 1.0), 0.0), 1.0);
     const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);
-    const double c = fma(mR * g, y, rep);
+    return fma(mR * g, y, rep);
+}
+
+// The form of a world: one for all kernels, so that the bits do not depend on
+// the kernel that steps it.
+__device__ __forceinline__ double pair_law(double d2, double mR, const WorldDev &a)
+{
+    const double y = pair_recip(d2);
+    return a.all_global ? pair_coef(d2, y, mR, a) : pair_coef_sum(d2, y, mR, a);
+}
+
+// A coefficient, or (almost) zero for a pair out of range: its high word goes,
+// and the 2^-1042 that may be left, times any difference and count, stays below
+// 2^-980, which no velocity, position or exported acceleration shows (world_dev
+// keeps force and dt within 2^400).  Clearing both words, 1.3% more
+// instructions: 512-world batch 1655 us a launch, 1640 so; clearing 1/|D| in FP32
+// instead lengthens the chain, dense 196k 2D world 1870 -> 1975.
+__device__ __forceinline__ double clear_high(double c, bool in)
+{
     uint2 b = __builtin_bit_cast(uint2, c);
     b.y = in ? b.y : 0u;
     return __builtin_bit_cast(double, b);
-}
-
-// The form for a pair in range, by world: one for all kernels, so that the bits
-// do not depend on the kernel that steps the world.
-__device__ __forceinline__ double pair_law(double d2, double mR, const WorldDev &a)
-{
-    return a.all_global ? pair_coef(d2, mR, a) : pair_coef_sum(d2, mR, true, a);
 }
 
 template <int DIM, bool DEBUG>
@@ -596,12 +602,12 @@ __device__ __forceinline__ uint32_t low_bits(int n)
 
 // Staged candidate at place k (the LDS address of its type, from which the
 // others follow in one instruction each) against a home at (px, py, pz)
-// (staged_axis) with matrix row mrow: the coefficient (0 where the pair does not
-// interact, Physics.java:432), the difference, and the wave's lanes whose pairs do.
+// (staged_axis) with matrix row mrow: its matrix entry times R, the difference
+// and its square.
 template <int DIM, bool WRAP, bool MLDS, bool EXACT>
-__device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev &w, const Staged &s,
+__device__ __forceinline__ double staged_pair(const ForceArgs &a, const WorldDev &w, const Staged &s,
                                               const double *M, uint32_t k, uint32_t px, uint32_t py, uint32_t pz,
-                                              int mrow, int &dxi, int &dyi, int &dzi, uint64_t &in)
+                                              int mrow, int &dxi, int &dyi, int &dzi, double &d2)
 {
     const uint64_t xy = lds_read<uint64_t>(8u * k + s.at.xy);
     const uint2 hl = make_uint2((uint32_t)xy, (uint32_t)(xy >> 32));
@@ -609,10 +615,8 @@ __device__ __forceinline__ double staged_coef(const ForceArgs &a, const WorldDev
     dyi = staged_diff<WRAP>(join_y(hl), py);
     dzi = DIM == 3 ? staged_diff<WRAP>(lds_read<uint32_t>(4u * k + s.at.z), pz) : 0;
     const int idx = mrow + (int)lds_read<uint8_t>(k);
-    const double m = MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
-    const double d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
-    in = __ballot(d2 != 0.0) & __ballot(d2 <= w.r2u);
-    return pair_coef_sum(d2, m, __builtin_amdgcn_inverse_ballot_w64(in), w);
+    d2 = pair_d2_of<DIM, EXACT>((double)dxi, (double)dyi, (double)dzi);
+    return MLDS ? M[idx] : a.matrix[w.moff + idx] * w.R;
 }
 
 // Mask words: the top kWordCands bits one candidate each, first at the top, the
@@ -639,13 +643,18 @@ __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev 
 {
     auto visit = [&](uint32_t k, bool last) {
         int dxi, dyi, dzi;
-        uint64_t in;
-        const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, in);
+        double d2;
+        const double m = staged_pair<DIM, WRAP, MLDS, EXACT>(a, w, s, M, k, px, py, pz, mrow, dxi, dyi, dzi, d2);
+        const uint64_t in = __ballot(d2 != 0.0) & __ballot(d2 <= w.r2u);       // Physics.java:432
+        double y = pair_recip(d2);
+        // (the mask is complete by here, off the chain that ends in its use)
+        asm("" : "+v"(y) : "s"(in));
+        const bool mine = __builtin_amdgcn_inverse_ballot_w64(in);
+        const double c = clear_high(pair_coef_sum(d2, y, m, w), mine);
         ab.x = fma(c, (double)dxi, ab.x);
         ab.y = fma(c, (double)dyi, ab.y);
         if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);
         if (DEBUG || last) {
-            const bool mine = __builtin_amdgcn_inverse_ballot_w64(in);
             ab.cnt += mine ? 1 : 0;
             if constexpr (DEBUG)
                 if (mine) ab.hash += id_hash(s.id[k - s.at.type]);

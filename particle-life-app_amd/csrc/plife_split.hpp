@@ -158,14 +158,14 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
             constexpr bool EXACT = decltype(exact)::value;
             auto coef = [&](int p, int &dx, int &dy, int &dz) -> double {
                 const uint32_t k = list[min(p, n - 1)];
-                uint64_t lanes;
-                const double c = staged_coef<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, bx, by, bz, mrow, dx, dy, dz,
-                                                                     lanes);
-                const bool in = p < n && __builtin_amdgcn_inverse_ballot_w64(lanes);
+                double d2;
+                const double m = staged_pair<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, bx, by, bz, mrow, dx, dy, dz, d2);
+                const double c = pair_coef_sum(d2, pair_recip(d2), m, wf);
+                const bool in = (p < n) & (d2 != 0.0) & (d2 <= w.r2u);      // Physics.java:432
                 acc.cnt += in ? 1 : 0;
                 if constexpr (DEBUG)
                     if (in) acc.hash += id_hash(stg.id[k - stg.at.type]);
-                return p < n ? c : 0.0;
+                return in ? c : 0.0;
             };
 #pragma unroll 1
             for (int s = 0; s < n; s += 2 * G) {
