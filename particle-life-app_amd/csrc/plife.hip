@@ -2668,12 +2668,16 @@ void destroy_handle(plife_physics *h)
     if (h->stream) (void)hipStreamDestroy(h->stream);
 }
 
-// A new world: forget the clustering measure of the old ones, and their
-// workgroups' pairs (the tag of the record of them).
-void reset_planner(plife_physics *h)
+// A new world: forget the clustering measure of the old ones and, for a state
+// made anew, their workgroups' pairs (the tag of the record of them).  An
+// uploaded state is often the last one, edited or submitted again: it keeps them
+// as the estimates its first step is ordered by, which costs another state
+// nothing (clustered 2D jobs submitted again, us: 778k particles, 7 steps 15400,
+// 22000 without; 376k, 5 steps 5570 and 7120).
+void reset_planner(plife_physics *h, bool uploaded)
 {
     std::memset(h->stat_host, 0, h->stat_cap * sizeof(uint64_t));
-    if (h->work_host && h->blocks.size() < h->work_host_cap) h->work_host[h->blocks.size()] = 0;
+    if (!uploaded && h->work_host && h->blocks.size() < h->work_host_cap) h->work_host[h->blocks.size()] = 0;
     h->occupancy = 0.0;
     h->clustered = false;
     for (WorldHost &w : h->worlds) w.nb = w.hot = -1.0;
@@ -3020,7 +3024,7 @@ int plife_set_particles(plife_physics *h, int32_t n, const double *pos, const do
     h->used = n;
     h->layout_dirty = true;
     h->stepped = false;
-    reset_planner(h);
+    reset_planner(h, true);
     return PLIFE_OK;
 }
 
@@ -3040,7 +3044,7 @@ int plife_generate_particles(plife_physics *h, int32_t n, uint64_t seed)
     h->used = n;
     h->layout_dirty = true;
     h->stepped = false;
-    reset_planner(h);
+    reset_planner(h, false);
     return PLIFE_OK;
 }
 
@@ -3051,7 +3055,7 @@ int plife_set_positions(plife_physics *h, int32_t preset, uint64_t seed)
     if ((rc = set_device(h))) return rc;
     if ((rc = sync_layout(h))) return rc;
     if ((rc = apply_preset(h, h->worlds[0], true, preset, seed))) return rc;
-    reset_planner(h);
+    reset_planner(h, false);
     return PLIFE_OK;
 }
 

@@ -248,12 +248,13 @@ void stopped_update_keeps_the_last_step()
     plife_destroy(h);
 }
 
-// New positions or particles: the planner keeps neither the workgroups' measured
-// work nor the neighbours of the state before, whatever the way in.
+// Positions or particles made anew: the planner keeps neither the workgroups'
+// measured work nor the neighbours of the state before, whatever the way in.  An
+// uploaded state keeps the work, as estimates.
 void new_state_forgets_measured_work()
 {
     const plife_tuning t{256, 0, 1, 0.0, 1, 0, 1};
-    for (int way = 0; way < 3; ++way) {
+    for (int way = 0; way < 4; ++way) {
         plife_physics *h = nullptr;
         plife_batch *b = nullptr;
         int32_t id = 0;
@@ -277,8 +278,18 @@ void new_state_forgets_measured_work()
         if (way == 0) CHECK(plife_set_positions(h, 0, 5) == PLIFE_OK);
         if (way == 1) CHECK(plife_generate_particles(h, 40000, 5) == PLIFE_OK);
         if (way == 2) CHECK(plife_batch_set_world_positions(b, id, 0, 5) == PLIFE_OK);
+        if (way == 3) {
+            std::vector<double> x(3 * 40000, 0.5);
+            std::vector<int32_t> types(40000, 1);
+            CHECK(plife_set_particles(h, 40000, x.data(), x.data(), types.data()) == PLIFE_OK);
+        }
         CHECK(prepare_step(h) == PLIFE_OK);
         CHECK(h->worlds[0].nb < 0.0 && (int)h->blocks.size() == 157);
+        if (way == 3) {
+            CHECK((int)h->blocks[0].y == 256 * 156 && h->block_est[0] == 1000000u);   // the heaviest, first
+            plife_destroy(h);
+            continue;
+        }
         for (int i = 0; i < 157; ++i) {
             CHECK((int)h->blocks[i].y == 256 * i);                            // no order made from the old work
             if (i < 156) CHECK(h->block_est[i] == h->block_est[0]);
