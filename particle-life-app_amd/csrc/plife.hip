@@ -509,8 +509,8 @@ WorldDev world_dev(const WorldHost &w, uint32_t cell_base, int moff)
     d.n = w.n;
     d.nx = gr.nx;
     // repeated stencil cells (Physics.java:377-395), or matrix entries whose
-    // product with R is not finite, or a force or dt past 2^400: the summed force
-    // law needs finite ones (pair_coef_sum)
+    // product with R is not finite, or a force or dt past 2^400: the staged and
+    // split kernels' form of the law needs finite ones (pair_coef, clear_high)
     d.all_global = gr.nx < 3 || !(std::fabs(s.force) <= 0x1p400 && std::fabs(s.dt) <= 0x1p400) ? 1 : 0;
     for (const double m : w.matrix)
         if (!std::isfinite(m * R)) d.all_global = 1;

@@ -99,17 +99,6 @@ __device__ __forceinline__ double pair_recip(double d2)
     return fma(0.5 * y0, h, y0);
 }
 
-// f/dist of the force law for a pair in range (0 < d2 <= rmax^2), y = pair_recip(d2).
-__device__ __forceinline__ double pair_coef(double d2, double y, double mR, const WorldDev &a)
-{
-    const double u = d2 * y;                       // |D| = dist R
-    const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
-    const double g = fma(t, -a.inv_1mb, 1.0);
-    const double att = (mR * g) * y;
-    const double rep = fma(-a.R, y, a.inv_beta);   // 1/beta - 1/dist
-    return u < a.betaR ? rep : att;
-}
-
 // pair_d2 where every square of a pair in range is below 2^52 (rmax <= 2^-6,
 // WorldDev::exact_d2): squares and sums of integers below 2^53 are exact, so
 // FMAs give the same value in one instruction less per axis; a pair whose sum
@@ -121,29 +110,24 @@ __device__ __forceinline__ double pair_d2_of(double dx, double dy, double dz)
     else return DIM == 3 ? fma(dx, dx, fma(dy, dy, dz * dz)) : fma(dx, dx, dy * dy);
 }
 
-// pair_coef with its branches summed in place of selected, for a finite mR:
-// below beta g is negative, at and above it 1/beta - 1/dist is not, so that of
-// max(g, 0) and min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact
-// zero to the other branch's value -- two instructions where the compare, the
-// two selects and the multiply take four.  (g <= 1, so the clamp to [0, 1],
-// free on its FMA, is max(g, 0).  Within 2^-44 of beta both terms are zero,
-// where the selected form has one of that size and the wrong sign.)  For a pair
-// in range only: the caller clears what it gives for others.
-__device__ __forceinline__ double pair_coef_sum(double d2, double y, double mR, const WorldDev &a)
+// f/dist of the force law for a pair in range (0 < d2 <= rmax^2), y =
+// pair_recip(d2), its branches summed in place of selected: below beta g is
+// negative, at and above it 1/beta - 1/dist is not, so that of max(g, 0) and
+// min(1/beta - 1/dist, 0) one is zero and the FMA adds an exact zero to the other
+// branch's value -- two instructions where a compare, two selects and a multiply
+// take four.  (g <= 1, so the clamp to [0, 1], free on its FMA, is max(g, 0).
+// Within 2^-44 of beta both terms are zero.)  ANY: mR need not be finite -- its
+// term is taken where g is not zero or dist not below beta; for a finite mR the
+// bits are the same, so they do not depend on the kernel that steps a world.
+template <bool ANY>
+__device__ __forceinline__ double pair_coef(double d2, double y, double mR, const WorldDev &a)
 {
-    const double u = d2 * y;
+    const double u = d2 * y;                       // |D| = dist R
     const double t = fabs(fma(u, a.m2S, a.one_plus_beta));
     const double g = fmin(fmax(fma(t, -a.inv_1mb, 1.0), 0.0), 1.0);
-    const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);
-    return fma(mR * g, y, rep);
-}
-
-// The form of a world: one for all kernels, so that the bits do not depend on
-// the kernel that steps it.
-__device__ __forceinline__ double pair_law(double d2, double mR, const WorldDev &a)
-{
-    const double y = pair_recip(d2);
-    return a.all_global ? pair_coef(d2, y, mR, a) : pair_coef_sum(d2, y, mR, a);
+    const double rep = fmin(fma(-a.R, y, a.inv_beta), 0.0);   // 1/beta - 1/dist
+    const double att = !ANY || g > 0.0 || !(u < a.betaR) ? mR * g : 0.0;
+    return fma(att, y, rep);
 }
 
 // A coefficient, or (almost) zero for a pair out of range: its high word goes,
@@ -167,7 +151,7 @@ __device__ __forceinline__ void pair64(Acc &acc, int dxi, int dyi, int dzi, doub
     const double d2 = pair_d2<DIM>(dx, dy, dz);
     const bool in = (d2 != 0.0) & (d2 <= a.r2u);     // Physics.java:432
     if (in) {
-        const double c = pair_law(d2, mR, a);
+        const double c = pair_coef<true>(d2, pair_recip(d2), mR, a);
         acc.x = fma(c, dx, acc.x);
         acc.y = fma(c, dy, acc.y);
         if constexpr (DIM == 3) acc.z = fma(c, dz, acc.z);
@@ -650,7 +634,7 @@ __device__ __forceinline__ void walk_home_of(const ForceArgs &a, const WorldDev 
         // (the mask is complete by here, off the chain that ends in its use)
         asm("" : "+v"(y) : "s"(in));
         const bool mine = __builtin_amdgcn_inverse_ballot_w64(in);
-        const double c = clear_high(pair_coef_sum(d2, y, m, w), mine);
+        const double c = clear_high(pair_coef<false>(d2, y, m, w), mine);
         ab.x = fma(c, (double)dxi, ab.x);
         ab.y = fma(c, (double)dyi, ab.y);
         if constexpr (DIM == 3) ab.z = fma(c, (double)dzi, ab.z);

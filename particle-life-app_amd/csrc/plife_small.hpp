@@ -177,7 +177,7 @@ __device__ __forceinline__ void small_run_split(const ForceArgs &a, const WorldD
         }
         const double d2 = pair_d2<DIM>((double)dxi, (double)dyi, (double)dzi);
         in &= (d2 != 0.0) & (d2 <= w.r2u);           // Physics.java:432
-        const double c = in ? pair_law(d2, m, w) : 0.0;
+        const double c = in ? pair_coef<true>(d2, pair_recip(d2), m, w) : 0.0;
         acc.cnt += in ? 1 : 0;
         if constexpr (DEBUG)
             if (in) acc.hash += id_hash(a.id[w.off + min((int)(P[jc] & 0xFFFFu), w.n - 1)]);

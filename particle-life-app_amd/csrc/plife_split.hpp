@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kSplitThreads) void k_force_split(ForceArgs a)
                 const uint32_t k = list[min(p, n - 1)];
                 double d2;
                 const double m = staged_pair<DIM, WRAP, MLDS, EXACT>(a, wf, stg, M, k, bx, by, bz, mrow, dx, dy, dz, d2);
-                const double c = pair_coef_sum(d2, pair_recip(d2), m, wf);
+                const double c = pair_coef<false>(d2, pair_recip(d2), m, wf);
                 const bool in = (p < n) & (d2 != 0.0) & (d2 <= w.r2u);      // Physics.java:432
                 acc.cnt += in ? 1 : 0;
                 if constexpr (DEBUG)

@@ -303,8 +303,8 @@ void new_state_forgets_measured_work()
     }
 }
 
-// Forces and time steps so large that what pair_coef_sum leaves out of range
-// could show take the literal law, as matrices that are not finite do.
+// Forces and time steps so large that what clear_high leaves of a pair out of
+// range could show take the literal path, as matrices that are not finite do.
 void extreme_forces_take_the_literal_law()
 {
     auto literal = [](double force, double dt, double entry) {
